@@ -166,6 +166,12 @@ struct oi_hit_digits {
     uint8_t shift[OI_HIT_DIGITS];
 };
 
+// bits that the mesh ids and the face ids of a hit list can have (a sort key
+// holds two of each)
+struct oi_pair_bits {
+    uint32_t mesh, tri;
+};
+
 // a scene's concatenated implicit index space must stay below this bound
 #define OI_IMPLICIT_LIMIT 0xfffffffeu
 

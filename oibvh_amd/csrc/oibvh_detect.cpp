@@ -105,6 +105,7 @@ void oi_det_free(oi_detector* d)
     dfree(d->sort_words);
     dfree(d->sort_vals);
     dfree(d->sort_scratch);
+    dfree(d->sort_mem);
     dfree(d->d_stage);
     dfree(d->ctl_base);
     d->ctl = nullptr;
@@ -423,11 +424,20 @@ static uint32_t bits_for(uint32_t max_value)
     return max_value ? 32u - (uint32_t)__builtin_clz(max_value) : 0u;
 }
 
+// Lists up to this length are ranked in one launch (k_pairs_rank, n^2
+// compares: 11 us at 5,100 pairs), longer ones sample sorted in five (27 us at
+// 15,800); the two meet at about 9,000 pairs.
+#define OI_PAIRS_RANK_MAX 9216u
+// The sample sort's buckets hold about n / 1024 keys at this length, a quarter
+// of what a workgroup sorts in LDS.
+#define OI_PAIRS_SORT_MAX (1u << 20)
+
 // The checked hits sorted on the device into d_sorted, in get_pairs order
-// (meshA, meshB, triA, triB): LSD radix passes over the bytes that can be
-// non-zero (mesh ids below the table's mesh count, face ids below its
-// largest face count), sorting hit indices with keys looked up by index,
-// then one gather. Once per query.
+// (meshA, meshB, triA, triB), once per query. Mesh ids are below the table's
+// mesh count and face ids below its largest face count; where two of each fit
+// into a 64-bit key, or the list is short, oibvh_pairs.hip sorts it, else LSD
+// radix passes over the bytes that can be non-zero sort hit indices with keys
+// looked up by index, then one gather.
 static oibvh_status sort_hits(oi_detector* d)
 {
     oibvh_ctx* c = d->ctx;
@@ -437,6 +447,28 @@ static oibvh_status sort_hits(oi_detector* d)
     uint32_t max_f = 1;
     for (uint32_t m = 0; m < d->tab.n_meshes; m++) max_f = std::max(max_f, d->tab.h_meshes[m].F);
     const uint32_t mbits = bits_for(d->tab.n_meshes ? d->tab.n_meshes - 1 : 0), tbits = bits_for(max_f - 1);
+    uint64_t gen = 0;
+    oibvh_status r;
+    const bool wide = 2u * (mbits + tbits) > 64u;
+    if (n <= OI_PAIRS_RANK_MAX || (n <= OI_PAIRS_SORT_MAX && !wide)) {
+        const oi_pair_bits bits{mbits, tbits};
+        if ((r = grow(c, d->d_sorted, d->d_sorted_cap, n, gen)) != OIBVH_OK) return r;
+        if (n <= OI_PAIRS_RANK_MAX) {
+            HIPCHK(c, oi_launch_pairs_rank(c->stream, d->hits, n, bits, wide, d->d_sorted));
+        } else {
+            if (d->sort_mem_cap < oi_pairs_sort_bytes(n)) {
+                // sized with headroom, so that the next queries rarely grow it
+                const uint64_t cap = oi_pairs_sort_bytes(std::min(OI_PAIRS_SORT_MAX, n + (n >> 2)));
+                dfree(d->sort_mem);
+                d->sort_mem_cap = 0;
+                HIPCHK(c, dalloc(&d->sort_mem, cap));
+                d->sort_mem_cap = cap;
+            }
+            HIPCHK(c, oi_launch_pairs_sort(c->stream, d->hits, n, bits, d->sort_mem, d->d_sorted));
+        }
+        d->sorted_ok = true;
+        return OIBVH_OK;
+    }
     oi_hit_digits dg{};
     for (uint32_t w : {3u, 2u, 1u, 0u}) {
         const uint32_t nb = ((w >= 2 ? tbits : mbits) + 7u) / 8u;
@@ -447,15 +479,6 @@ static oibvh_status sort_hits(oi_detector* d)
         }
     }
     const uint32_t tiles = (n + oi_sort_tile() - 1) / oi_sort_tile();
-    uint64_t gen = 0;
-    oibvh_status r;
-    if (n <= oi_hits_sort_small_max()) {
-        // one workgroup, every pass in LDS, one launch
-        if ((r = grow(c, d->d_sorted, d->d_sorted_cap, n, gen)) != OIBVH_OK) return r;
-        HIPCHK(c, oi_launch_hits_sort_small(c->stream, d->hits, n, &dg, d->d_sorted));
-        d->sorted_ok = true;
-        return OIBVH_OK;
-    }
     if (d->sort_cap < n) {
         // sized with headroom, so that the next queries rarely grow them
         const uint64_t cap = std::min<uint64_t>((1ull << 30) - 1, (uint64_t)n + (n >> 2));

@@ -72,8 +72,9 @@ hipError_t oi_launch_pair_vertices(hipStream_t, const oi_build_desc*, const uint
 hipError_t oi_launch_zero_u32(hipStream_t, uint32_t*, uint32_t);
 hipError_t oi_launch_hits_digits(hipStream_t, const uint4*, uint32_t, uint32_t*, uint32_t*, const oi_hit_digits*);
 hipError_t oi_launch_hits_gather(hipStream_t, const uint4*, const uint32_t*, uint32_t, uint4*);
-hipError_t oi_launch_hits_sort_small(hipStream_t, const uint4*, uint32_t, const oi_hit_digits*, uint4*);
-uint32_t oi_hits_sort_small_max();
+hipError_t oi_launch_pairs_rank(hipStream_t, const uint4*, uint32_t, oi_pair_bits, int, uint4*);
+uint64_t oi_pairs_sort_bytes(uint32_t);
+hipError_t oi_launch_pairs_sort(hipStream_t, const uint4*, uint32_t, oi_pair_bits, void*, uint4*);
 }
 
 // side streams of overlapped frames' detects, and the ring of their events
@@ -292,6 +293,8 @@ struct oi_detector {
     uint32_t* sort_vals = nullptr;   // two buffers of hit indices
     uint32_t* sort_scratch = nullptr;  // histograms | tile counters | two look-back buffers
     uint32_t sort_cap = 0;           // hits the sort buffers hold
+    uint8_t* sort_mem = nullptr;     // scratch of the sample sort
+    uint64_t sort_mem_cap = 0;
     float* d_stage = nullptr;     // vertex export staging for host output
     uint64_t stage_cap = 0;
     oibvh_detect_stats stats{};

@@ -1169,6 +1169,42 @@ def test_pairs_sorted_on_device(api, ctx, orc):
     assert far.pairs_device()[1] == 0 and len(far.getIntTriPairs()) == 0
 
 
+@pytest.mark.parametrize("subdiv", [0, 1, 2, 3, 4, 5, 6])
+def test_pairs_sorted_lengths(api, ctx, orc, subdiv):
+    """Pair lists of 200 to 1.06M pairs (a sphere against itself: every face
+    meets itself and its neighbours): ranked in one launch, sample sorted
+    (from 9,217) and, above 2^20, sorted by LSD passes, in oracle order."""
+    say(f"pair list length, subdiv {subdiv}")
+    a = M.icosphere(subdiv, 1.0, 0.0, 0)
+    t = [gpu_tree(api, ctx, *a), gpu_tree(api, ctx, *a)]
+    sc = api.Scene(ctx)
+    for x in t:
+        sc.addOibvhTree(x)
+    sc.detectCollision(4, 3)
+    want = orc.detect([orc.Tree(*a), orc.Tree(*a)])
+    assert len(want) >= 10 * a[1].shape[0] and (subdiv < 6 or len(want) > 1 << 20)
+    assert np.array_equal(sc.getIntTriPairs(), want)
+
+
+def test_pairs_sorted_wide_keys(api, ctx, orc):
+    """Ids that do not fit into a 64-bit key (301 trees: 9 bits, one of them
+    of more than 2^23 faces: 24 bits) are compared as 128 bits."""
+    say("pair keys above 64 bits")
+    shapes = [M.icosphere(1, 0.6, 0.02, 900 + i, center=(0.9 * i, 0.0, 0.0)) for i in range(300)]
+    trees = [gpu_tree(api, ctx, *m) for m in shapes]
+    F = (1 << 23) + 1  # far away from all others
+    faces = (np.arange(3 * F, dtype=np.uint32) % np.uint32(3000)).reshape(F, 3)
+    xyz = (M.uniform(5, 9000, 0.0, 1.0).reshape(-1, 3) + 5000.0).astype(np.float32)
+    trees.append(gpu_tree(api, ctx, xyz, faces))
+    sc = api.Scene(ctx)
+    for t in trees:
+        sc.addOibvhTree(t)
+    sc.detectCollision(0, 2)
+    want = orc.detect([orc.Tree(x, f, order=t.perm()) for (x, f), t in zip(shapes, trees)])
+    assert len(want) > 0
+    assert np.array_equal(sc.getIntTriPairs(), want)
+
+
 def test_scene_build_equals_tree_builds(api, ctx, orc):
     """oibvh_scene_build (the trees sharing each launch of the build chain)
     gives every tree what oibvh_tree_build gives it: leaf order, sorted faces
