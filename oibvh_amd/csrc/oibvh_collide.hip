@@ -1138,6 +1138,34 @@ __global__ void k_seed(uint32_t n0, uint32_t* counts, uint32_t n_counts, oi_dete
     }
 }
 
+// A query's counters and front lengths to pinned host memory, by one wave: its
+// stores are complete at the system-scope release that precedes the sequence
+// number, so a host that sees the number sees the rest. Errors read here are
+// reported once: the error and sticky words are cleared, so that later
+// asynchronous seeds do not fold them in again.
+// It takes the place of two copies, a fill and a stream wait per counter set
+// read (each of them a launch of 2-5 us and a gap of 5-13 us before the next).
+__global__ void __launch_bounds__(64) k_publish(oi_publish_args A)
+{
+    constexpr uint32_t W = sizeof(oi_detect_ctl) / 4u;
+    const uint32_t lane = threadIdx.x;
+    // (constant indices keep the argument block out of scratch memory)
+#pragma unroll
+    for (uint32_t s = 0; s < OI_PUB_SETS; s++) {
+        if (s >= A.n_sets) continue;
+        uint32_t* src = reinterpret_cast<uint32_t*>(A.ctl[s]);
+        if (lane < W) reinterpret_cast<uint32_t*>(&A.out->ctl[s])[lane] = src[lane];
+    }
+    for (uint32_t i = lane; i < A.n_counts; i += 64u) A.out->counts[i] = A.counts[i];
+#pragma unroll
+    for (uint32_t s = 0; s < OI_PUB_SETS; s++)
+        if (s < A.n_sets && lane == 0) {
+            A.ctl[s]->error = 0;
+            A.ctl[s]->sticky = 0;
+        }
+    if (lane == 0) __hip_atomic_store(&A.out->seq, A.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
@@ -1303,6 +1331,13 @@ hipError_t oi_launch_seed(hipStream_t st, uint32_t n0, uint32_t* counts, uint32_
 {
     if (n_counts > 256) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_seed, dim3(1), dim3(256), 0, st, n0, counts, n_counts, ctl, reset_sticky);
+    return hipGetLastError();
+}
+
+hipError_t oi_launch_publish(hipStream_t st, const oi_publish_args* a)
+{
+    if (a->n_sets > OI_PUB_SETS || a->n_counts > OI_PUB_COUNTS) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, st, *a);
     return hipGetLastError();
 }
 

@@ -122,6 +122,26 @@ struct oi_detect_ctl {
     uint32_t pad;
 };
 
+// What a check reads of a query, in pinned host memory that k_publish writes:
+// the counters of up to OI_PUB_SETS counter sets (the current one first), the
+// current set's front lengths, and last the sequence number that the host waits
+// for
+#define OI_PUB_SETS 4
+#define OI_PUB_COUNTS 256
+struct oi_published {
+    oi_detect_ctl ctl[OI_PUB_SETS];
+    uint32_t counts[OI_PUB_COUNTS];
+    uint32_t seq;
+};
+struct oi_publish_args {
+    oi_detect_ctl* ctl[OI_PUB_SETS];  // the first n_sets are read, and their error and sticky words cleared
+    uint32_t n_sets;
+    const uint32_t* counts;           // n_counts <= OI_PUB_COUNTS
+    uint32_t n_counts;
+    oi_published* out;
+    uint32_t seq;
+};
+
 // a detect's counter reset (zeroed level counts and result counters), done
 // by the last workgroup of a refit's apex launch when a detect follows it in
 // the same frame call, instead of a launch of its own

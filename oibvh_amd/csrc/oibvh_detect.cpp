@@ -2,7 +2,7 @@
 // management, the launch sequence of one query and the overflow re-run loop
 // (Scene::detectCollisionOnGPU, scene.cu:225-446, which instead copies the
 // front size to the host after every level and uses fixed 10M-entry buffers).
-#include <cstddef>
+#include <chrono>
 
 #include "oibvh_internal.h"
 
@@ -35,12 +35,12 @@ oibvh_status oi_det_init(oi_detector* d, oibvh_ctx* c)
     hipError_t e = dalloc(&d->ctl_base, OI_FRAME_DEPTH);
     if (e == hipSuccess) e = hipMemsetAsync(d->ctl_base, 0, OI_FRAME_DEPTH * sizeof(oi_detect_ctl), c->stream);
     if (e == hipSuccess)
-        e = hipHostMalloc((void**)&d->h_ctl, OI_FRAME_DEPTH * sizeof(oi_detect_ctl), hipHostMallocDefault);
+        e = hipHostMalloc((void**)&d->h_pub, sizeof(oi_published), hipHostMallocCoherent | hipHostMallocMapped);
     if (e != hipSuccess) {
         oi_det_free(d);
         return oi_set_err(c, OIBVH_ERR_HIP, "detector alloc: %s", hipGetErrorString(e));
     }
-    std::memset(d->h_ctl, 0, OI_FRAME_DEPTH * sizeof(oi_detect_ctl));
+    std::memset(d->h_pub, 0, sizeof(oi_published));
     d->ctl = d->ctl_base;
     return OIBVH_OK;
 }
@@ -109,8 +109,8 @@ void oi_det_free(oi_detector* d)
     dfree(d->d_stage);
     dfree(d->ctl_base);
     d->ctl = nullptr;
-    if (d->h_ctl) (void)hipHostFree(d->h_ctl);
-    d->h_ctl = nullptr;
+    if (d->h_pub) (void)hipHostFree(d->h_pub);
+    d->h_pub = nullptr;
 }
 
 oibvh_status oi_det_set_front(oi_detector* d, const std::vector<uint2>& front)
@@ -310,6 +310,19 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
     return OIBVH_OK;
 }
 
+// Wait for the sequence number that the last launch on the context's stream
+// writes: a short wait on the memory itself (a stream wait costs about 10 us
+// more than the launch it waits for), then the stream's, which also reports a
+// failed launch.
+static hipError_t wait_published(oi_detector* d)
+{
+    const auto t0 = std::chrono::steady_clock::now();
+    while (__atomic_load_n(&d->h_pub->seq, __ATOMIC_ACQUIRE) != d->pub_seq)
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20))
+            return hipStreamSynchronize(d->ctx->stream);
+    return hipSuccess;
+}
+
 oibvh_status oi_det_check(oi_detector* d)
 {
     oibvh_ctx* c = d->ctx;
@@ -317,30 +330,28 @@ oibvh_status oi_det_check(oi_detector* d)
     HIPCHK(c, oi_ctx_join(c));  // an overlapped frame's detect ran on a side stream
     uint32_t retries = 0, earlier = 0;
     for (;;) {
-        d->h_counts.resize(d->n_levels + 1);
-        HIPCHK(c, hipMemcpyAsync(d->h_ctl, d->ctl, sizeof(oi_detect_ctl), hipMemcpyDeviceToHost, c->stream));
-        // the other sets still holding unchecked overlapped frames' results
+        // this query's counters and front lengths, and those of the other sets
+        // still holding unchecked overlapped frames' results
         uint32_t others[OI_FRAME_DEPTH], n_others = 0;
+        oi_publish_args pa{};
+        pa.ctl[pa.n_sets++] = d->ctl;
         for (uint32_t s = 0; s < OI_FRAME_DEPTH; s++)
-            if (s != d->set && d->set_unchecked[s]) others[n_others++] = s;
-        for (uint32_t j = 0; j < n_others; j++)
-            HIPCHK(c, hipMemcpyAsync(d->h_ctl + 1 + j, d->ctl_base + others[j], sizeof(oi_detect_ctl),
-                                     hipMemcpyDeviceToHost, c->stream));
-        // what is read here is reported once: clear the error and sticky
-        // bits of every set read, so later asynchronous seeds do not fold
-        // them in again (error and sticky are adjacent words)
-        static_assert(offsetof(oi_detect_ctl, sticky) == offsetof(oi_detect_ctl, error) + 4, "ctl layout");
-        HIPCHK(c, hipMemsetAsync(&d->ctl->error, 0, 8, c->stream));
-        for (uint32_t j = 0; j < n_others; j++)
-            HIPCHK(c, hipMemsetAsync(&d->ctl_base[others[j]].error, 0, 8, c->stream));
-        HIPCHK(c, hipMemcpyAsync(d->h_counts.data(), d->counts, (d->n_levels + 1) * sizeof(uint32_t),
-                                 hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        const oi_detect_ctl& k = d->h_ctl[0];
+            if (s != d->set && d->set_unchecked[s]) {
+                others[n_others++] = s;
+                pa.ctl[pa.n_sets++] = d->ctl_base + s;
+            }
+        pa.counts = d->counts;
+        pa.n_counts = d->n_levels + 1;
+        pa.out = d->h_pub;
+        pa.seq = ++d->pub_seq;
+        HIPCHK(c, oi_launch_publish(c->stream, &pa));
+        HIPCHK(c, wait_published(d));
+        d->h_counts.assign(d->h_pub->counts, d->h_pub->counts + d->n_levels + 1);
+        const oi_detect_ctl k = d->h_pub->ctl[0];
         earlier |= k.sticky;  // errors of unchecked asynchronous detects before this one
         for (uint32_t j = 0; j < n_others; j++) {
             // earlier overlapped frames' detects and the unchecked ones before them
-            earlier |= d->h_ctl[1 + j].sticky | d->h_ctl[1 + j].error;
+            earlier |= d->h_pub->ctl[1 + j].sticky | d->h_pub->ctl[1 + j].error;
             d->set_unchecked[others[j]] = false;
         }
         if (d->h_counts[d->n_levels] != 0) {

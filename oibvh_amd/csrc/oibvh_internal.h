@@ -61,6 +61,7 @@ hipError_t oi_launch_reduce_apex_inline(hipStream_t, int, const oi_build_desc*, 
                                         hipEvent_t);
 hipError_t oi_launch_set_mesh_pos(hipStream_t, oi_build_desc*, oi_mesh_desc*, uint32_t, const float*);
 hipError_t oi_launch_seed(hipStream_t, uint32_t, uint32_t*, uint32_t, oi_detect_ctl*, uint32_t);
+hipError_t oi_launch_publish(hipStream_t, const oi_publish_args*);
 hipError_t oi_launch_bvtt_step(hipStream_t, uint32_t, const oi_tab_args*, int, const uint2*, const uint32_t*,
                                uint32_t, uint32_t, uint2*, uint32_t*, uint32_t, uint2*, uint32_t*, uint32_t, uint4*,
                                uint32_t, oi_detect_ctl*, uint32_t, uint32_t, int, hipEvent_t);
@@ -231,6 +232,8 @@ static inline uint32_t oi_grid_for(const oibvh_ctx* c)
 // prepare sizes the buffers beforehand, check waits, grows what overflowed
 // and runs the query again.
 // ---------------------------------------------------------------------------
+static_assert(OI_FRAME_DEPTH <= OI_PUB_SETS, "one launch publishes every counter set");
+
 struct oi_detector {
     oibvh_ctx* ctx = nullptr;
     uint2* d_init = nullptr;  // initial BVTT front
@@ -268,7 +271,8 @@ struct oi_detector {
     // overflows, so that a set does not overflow where another already did)
     uint32_t want_front = 0, want_cands = 0, want_hits = 0;
     oi_detect_ctl* ctl = nullptr;    // counters of the current set
-    oi_detect_ctl* h_ctl = nullptr;  // pinned, OI_FRAME_DEPTH (the current set's, then the others read)
+    oi_published* h_pub = nullptr;   // pinned: what the last check read (h_pub->seq == pub_seq once it has landed)
+    uint32_t pub_seq = 0;
     std::vector<uint32_t> h_counts;
     // the query (kept for re-runs)
     oi_tab_args tab{};
