@@ -323,6 +323,18 @@ static hipError_t wait_published(oi_detector* d)
     return hipSuccess;
 }
 
+// wait until everything queued on the context's stream so far has completed,
+// through the published sequence number
+static oibvh_status finish(oi_detector* d)
+{
+    oi_publish_args pa{};
+    pa.out = d->h_pub;
+    pa.seq = ++d->pub_seq;
+    HIPCHK(d->ctx, oi_launch_publish(d->ctx->stream, &pa));
+    HIPCHK(d->ctx, wait_published(d));
+    return OIBVH_OK;
+}
+
 oibvh_status oi_det_check(oi_detector* d)
 {
     oibvh_ctx* c = d->ctx;
@@ -550,7 +562,7 @@ oibvh_status oi_det_sorted_device(oi_detector* d, const uint4** dptr, uint32_t* 
     if ((r = sort_hits(d)) != OIBVH_OK) return r;
     // the sort runs on the context's stream: complete it before the pointer
     // is handed to a consumer on any stream or the host
-    HIPCHK(d->ctx, hipStreamSynchronize(d->ctx->stream));
+    if ((r = finish(d)) != OIBVH_OK) return r;
     *dptr = d->d_sorted;
     *n = d->n_pairs;
     return OIBVH_OK;
@@ -582,10 +594,10 @@ oibvh_status oi_det_pair_vertices(oi_detector* d, const oi_build_desc* geom, flo
     HIPCHK(c, oi_launch_pair_vertices(c->stream, geom, d->d_sorted, d->n_pairs, dst));
     if (ptr_kind == OIBVH_PTR_HOST) {
         HIPCHK(c, hipMemcpyAsync(out, d->d_stage, need * sizeof(float), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        return OIBVH_OK;
     }
-    // host output must land; device output is complete when this returns
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return OIBVH_OK;
+    return finish(d);  // device output is complete when this returns
 }
 
 oibvh_status oi_det_level_counts(oi_detector* d, uint32_t* out, uint64_t cap, uint32_t* n)
