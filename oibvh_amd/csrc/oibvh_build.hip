@@ -1163,16 +1163,7 @@ __device__ __forceinline__ void seed_counters(const oi_seed_args& s)
 {
     const uint32_t i = threadIdx.x;
     if (i < s.n_counts) s.counts[i] = (i == 0) ? s.n0 : 0u;
-    if (i == 0) {
-        s.ctl->sticky = s.reset_sticky ? 0u : (s.ctl->sticky | s.ctl->error);
-        s.ctl->error = 0;
-        s.ctl->n_hits = 0;
-        s.ctl->cands = 0;
-        s.ctl->fp64 = 0;
-        s.ctl->adj = 0;
-        s.ctl->tests = 0;
-        s.ctl->deferred = 0;
-    }
+    oi_reset_ctl(s.ctl, i, s.reset_sticky);
 }
 
 // with seed.counts set, the launch has one more workgroup, which resets the

@@ -62,6 +62,16 @@ __device__ __forceinline__ uint32_t add_u32(uint32_t* p, uint32_t v)
 {
     return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// a workgroup's statistics to its shard
+__device__ __forceinline__ void add_stat(oi_detect_stat* shards, uint32_t tests, uint32_t adj, uint32_t fp64,
+                                         uint32_t cands)
+{
+    oi_detect_stat* s = shards + (blockIdx.x % OI_STAT_SHARDS);
+    if (tests) __hip_atomic_fetch_add(&s->tests, (u64)tests, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (adj) __hip_atomic_fetch_add(&s->adj, (u64)adj, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (fp64) __hip_atomic_fetch_add(&s->fp64, (u64)fp64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (cands) add_u32(&s->cands, cands);
+}
 __device__ __forceinline__ void or_u32(uint32_t* p, uint32_t v)
 {
     __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -416,8 +426,7 @@ struct StepArgs {
     uint32_t* cand_count;
     uint32_t cand_cap;
     uint32_t* error;
-    unsigned long long* tests;  // box pair tests (statistics)
-    unsigned long long* adj;    // self-mode leaf pairs dropped as adjacent
+    oi_detect_stat* stat;       // shards
     uint4* hits;                // fused narrow phase: hits and their count
     uint32_t* n_hits;
     uint32_t hits_cap;
@@ -727,9 +736,7 @@ k_bvtt_step(StepArgs<Tab> A)
     uint32_t nt, na;
     block_scan(n_tests, s_wsum, nt);
     block_scan(n_adj, s_wsum, na);
-    if (tid == 0 && nt) __hip_atomic_fetch_add(A.tests, (u64)nt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (tid == 0 && na) __hip_atomic_fetch_add(A.adj, (u64)na, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (FUSED && tid == 0 && n_cands) add_u32(A.cand_count, n_cands);
+    if (tid == 0) add_stat(A.stat, nt, na, 0u, FUSED ? n_cands : 0u);
 }
 
 // ---------------------------------------------------------------------------
@@ -769,8 +776,7 @@ struct LocalArgs {
     uint32_t* cand_count;
     uint32_t cand_cap;
     uint32_t* error;
-    unsigned long long* tests;
-    unsigned long long* adj;
+    oi_detect_stat* stat;
     uint4* hits;
     uint32_t* n_hits;
     uint32_t hits_cap;
@@ -896,9 +902,7 @@ __global__ void __launch_bounds__(TB) k_bvtt_local(LocalArgs<Tab> A)
     uint32_t nt, na;
     block_scan(n_tests, s_wsum, nt);
     block_scan(n_adj, s_wsum, na);
-    if (tid == 0 && nt) __hip_atomic_fetch_add(A.tests, (u64)nt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (tid == 0 && na) __hip_atomic_fetch_add(A.adj, (u64)na, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (FUSED && tid == 0 && n_cands) add_u32(A.cand_count, n_cands);
+    if (tid == 0) add_stat(A.stat, nt, na, 0u, FUSED ? n_cands : 0u);
 }
 
 // ---------------------------------------------------------------------------
@@ -914,8 +918,7 @@ struct NarrowArgs {
     uint32_t* n_hits;
     uint32_t hits_cap;
     uint32_t* error;
-    unsigned long long* fp64;   // SAT axis comparisons evaluated in double
-    unsigned long long* adj;    // self-mode leaf pairs dropped as adjacent
+    oi_detect_stat* stat;       // shards
     uint2* defer;               // NARROW_FILTER: undecided candidates for NARROW_FP64
     uint32_t* defer_count;
     uint32_t defer_cap;
@@ -1113,10 +1116,7 @@ __global__ void __launch_bounds__(TB) k_narrow(NarrowArgs<Tab> A)
     uint32_t f, a;
     block_scan(n_fp64, s_wsum, f);
     block_scan(n_adj, s_wsum, a);
-    if (tid == 0) {
-        if (f) __hip_atomic_fetch_add(A.fp64, (u64)f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (a) __hip_atomic_fetch_add(A.adj, (u64)a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (tid == 0) add_stat(A.stat, 0u, a, f, 0u);
 }
 
 // seed: zeroed level counts and result counters (counts[0] = initial front)
@@ -1124,18 +1124,7 @@ __global__ void k_seed(uint32_t n0, uint32_t* counts, uint32_t n_counts, oi_dete
 {
     const uint32_t i = threadIdx.x;
     if (i < n_counts) counts[i] = (i == 0) ? n0 : 0u;
-    if (i == 0) {
-        // errors of the previous detect move to `sticky` unless the caller
-        // checked it synchronously
-        ctl->sticky = reset_sticky ? 0u : (ctl->sticky | ctl->error);
-        ctl->error = 0;
-        ctl->n_hits = 0;
-        ctl->cands = 0;
-        ctl->fp64 = 0;
-        ctl->adj = 0;
-        ctl->tests = 0;
-        ctl->deferred = 0;
-    }
+    oi_reset_ctl(ctl, i, reset_sticky);
 }
 
 // A query's counters and front lengths to pinned host memory, by one wave: its
@@ -1147,22 +1136,40 @@ __global__ void k_seed(uint32_t n0, uint32_t* counts, uint32_t n_counts, oi_dete
 // read (each of them a launch of 2-5 us and a gap of 5-13 us before the next).
 __global__ void __launch_bounds__(64) k_publish(oi_publish_args A)
 {
-    constexpr uint32_t W = sizeof(oi_detect_ctl) / 4u;
     const uint32_t lane = threadIdx.x;
-    // (constant indices keep the argument block out of scratch memory)
-#pragma unroll
-    for (uint32_t s = 0; s < OI_PUB_SETS; s++) {
-        if (s >= A.n_sets) continue;
-        uint32_t* src = reinterpret_cast<uint32_t*>(A.ctl[s]);
-        if (lane < W) reinterpret_cast<uint32_t*>(&A.out->ctl[s])[lane] = src[lane];
-    }
-    for (uint32_t i = lane; i < A.n_counts; i += 64u) A.out->counts[i] = A.counts[i];
-#pragma unroll
-    for (uint32_t s = 0; s < OI_PUB_SETS; s++)
-        if (s < A.n_sets && lane == 0) {
-            A.ctl[s]->error = 0;
-            A.ctl[s]->sticky = 0;
+    static_assert(OI_STAT_SHARDS == 64, "a shard per lane");
+    if (A.n_sets) {
+        const oi_detect_ctl* c = A.ctl[0];
+        u64 tests = c->stat[lane].tests, adj = c->stat[lane].adj, fp64 = c->stat[lane].fp64;
+        uint32_t cands = c->stat[lane].cands;
+        for (int d = 32; d; d >>= 1) {
+            tests += (u64)__shfl_xor((unsigned long long)tests, d, 64);
+            adj += (u64)__shfl_xor((unsigned long long)adj, d, 64);
+            fp64 += (u64)__shfl_xor((unsigned long long)fp64, d, 64);
+            cands += (uint32_t)__shfl_xor((int)cands, d, 64);
         }
+        for (uint32_t i = lane; i < A.n_counts; i += 64u) A.out->counts[i] = A.counts[i];
+        if (lane == 0) {
+            A.out->tests = tests;
+            A.out->adj = adj;
+            A.out->fp64 = fp64;
+            A.out->n_hits = c->n_hits;
+            A.out->cands = c->cands + cands;
+            A.out->deferred = c->deferred;
+            A.out->error = c->error;
+            A.out->sticky = c->sticky;
+            uint32_t earlier = 0;
+            // (constant indices keep the argument block out of scratch memory)
+#pragma unroll
+            for (uint32_t s = 0; s < OI_PUB_SETS; s++) {
+                if (s >= A.n_sets) continue;
+                if (s) earlier |= A.ctl[s]->error | A.ctl[s]->sticky;
+                A.ctl[s]->error = 0;
+                A.ctl[s]->sticky = 0;
+            }
+            A.out->earlier = earlier;
+        }
+    }
     if (lane == 0) __hip_atomic_store(&A.out->seq, A.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -1210,8 +1217,7 @@ static hipError_t launch_step(hipStream_t st, uint32_t grid, const Tab& tab, int
     a.cand_count = cand_count;
     a.cand_cap = cand_cap;
     a.error = &ctl->error;
-    a.tests = &ctl->tests;
-    a.adj = &ctl->adj;
+    a.stat = ctl->stat;
     a.hits = hits;
     a.n_hits = &ctl->n_hits;
     a.hits_cap = hits_cap;
@@ -1273,8 +1279,7 @@ static hipError_t launch_local(hipStream_t st, const Tab& tab, const oi_local_ar
     a.cand_count = cand_count;
     a.cand_cap = cand_cap;
     a.error = &ctl->error;
-    a.tests = &ctl->tests;
-    a.adj = &ctl->adj;
+    a.stat = ctl->stat;
     a.hits = hits;
     a.n_hits = &ctl->n_hits;
     a.hits_cap = hits_cap;
@@ -1310,8 +1315,7 @@ static hipError_t launch_narrow(hipStream_t st, uint32_t grid, const Tab& tab, c
     a.n_hits = n_hits;
     a.hits_cap = hits_cap;
     a.error = &ctl->error;
-    a.fp64 = &ctl->fp64;
-    a.adj = &ctl->adj;
+    a.stat = ctl->stat;
     a.defer = defer;
     a.defer_count = &ctl->deferred;
     a.defer_cap = defer_cap;

@@ -109,32 +109,66 @@ struct oi_tab_args {
     uint32_t shift;
 };
 
-// Detect counters, reset by the seed kernel before each detect.
-struct oi_detect_ctl {
-    uint32_t n_hits;           // hits found (may exceed capacity)
-    uint32_t cands;            // candidate leaf pairs (may exceed capacity)
-    uint32_t error;            // OI_ERR_* bits of this detect
-    uint32_t sticky;           // OI_ERR_* bits of earlier asynchronous detects not checked since
-    unsigned long long fp64;   // SAT axis comparisons re-evaluated in double
-    unsigned long long adj;    // leaf pairs dropped as adjacent (self mode)
+// Statistics of a detect, in shards: workgroup b adds to shard b % OI_STAT_SHARDS
+// and the shards are summed when the counters are read. A thousand workgroups
+// that end together and add to one cache line take 10 us about it (a walk launch
+// of 16 us took 35).
+#define OI_STAT_SHARDS 64
+struct alignas(128) oi_detect_stat {
     unsigned long long tests;  // BVTT box pair tests
-    uint32_t deferred;         // FP64 fallback: candidates the FP32 filter left undecided
-    uint32_t pad;
+    unsigned long long adj;    // leaf pairs dropped as adjacent (self mode)
+    unsigned long long fp64;   // SAT axis comparisons re-evaluated in double
+    uint32_t cands;            // leaf pairs tested where they were found
 };
 
+// Detect counters, reset by the seed kernel before each detect; those that hand
+// out places in a list lie on lines of their own.
+struct oi_detect_ctl {
+    alignas(128) uint32_t n_hits;    // hits found (may exceed capacity)
+    alignas(128) uint32_t cands;     // leaf pairs put into the candidate list (may exceed capacity)
+    alignas(128) uint32_t deferred;  // FP64 fallback: candidates the FP32 filter left undecided
+    alignas(128) uint32_t error;     // OI_ERR_* bits of this detect
+    uint32_t sticky;                 // OI_ERR_* bits of earlier asynchronous detects not checked since
+    oi_detect_stat stat[OI_STAT_SHARDS];
+};
+
+#if defined(__HIPCC__) || defined(__HIP__)
+// thread tid of a workgroup of at least OI_STAT_SHARDS threads resets ctl; errors
+// of the previous detect move to `sticky` unless the caller checked it
+// synchronously
+__device__ __forceinline__ void oi_reset_ctl(oi_detect_ctl* ctl, uint32_t tid, uint32_t reset_sticky)
+{
+    if (tid == 0) {
+        ctl->sticky = reset_sticky ? 0u : (ctl->sticky | ctl->error);
+        ctl->error = 0;
+        ctl->n_hits = 0;
+        ctl->cands = 0;
+        ctl->deferred = 0;
+    }
+    if (tid < OI_STAT_SHARDS) {
+        oi_detect_stat* s = ctl->stat + tid;
+        s->tests = 0;
+        s->adj = 0;
+        s->fp64 = 0;
+        s->cands = 0;
+    }
+}
+#endif
+
 // What a check reads of a query, in pinned host memory that k_publish writes:
-// the counters of up to OI_PUB_SETS counter sets (the current one first), the
-// current set's front lengths, and last the sequence number that the host waits
-// for
+// the current counter set's counters and front lengths, the error words of the
+// other unchecked sets, and last the sequence number that the host waits for
 #define OI_PUB_SETS 4
 #define OI_PUB_COUNTS 256
 struct oi_published {
-    oi_detect_ctl ctl[OI_PUB_SETS];
+    uint32_t n_hits, cands, deferred, error, sticky;
+    uint32_t earlier;  // error and sticky bits of the other sets
+    unsigned long long tests, adj, fp64;
     uint32_t counts[OI_PUB_COUNTS];
     uint32_t seq;
 };
 struct oi_publish_args {
-    oi_detect_ctl* ctl[OI_PUB_SETS];  // the first n_sets are read, and their error and sticky words cleared
+    oi_detect_ctl* ctl[OI_PUB_SETS];  // n_sets sets, the current one first; their error and sticky words are cleared
     uint32_t n_sets;
     const uint32_t* counts;           // n_counts <= OI_PUB_COUNTS
     uint32_t n_counts;

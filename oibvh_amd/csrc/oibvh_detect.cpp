@@ -359,11 +359,10 @@ oibvh_status oi_det_check(oi_detector* d)
         HIPCHK(c, oi_launch_publish(c->stream, &pa));
         HIPCHK(c, wait_published(d));
         d->h_counts.assign(d->h_pub->counts, d->h_pub->counts + d->n_levels + 1);
-        const oi_detect_ctl k = d->h_pub->ctl[0];
-        earlier |= k.sticky;  // errors of unchecked asynchronous detects before this one
+        const oi_published& k = *d->h_pub;
+        earlier |= k.sticky | k.earlier;  // errors of unchecked asynchronous detects before this one
         for (uint32_t j = 0; j < n_others; j++) {
             // earlier overlapped frames' detects and the unchecked ones before them
-            earlier |= d->h_pub->ctl[1 + j].sticky | d->h_pub->ctl[1 + j].error;
             d->set_unchecked[others[j]] = false;
         }
         if (d->h_counts[d->n_levels] != 0) {
