@@ -243,6 +243,36 @@ __device__ int sat_filter(const v3f* P, const v3f* Q)
     return undecided ? SAT_UNDECIDED : SAT_HIT;
 }
 
+// sat_filter's bounds and one axis of it, for lanes that share a pair (sat_lanes):
+// separated or not (SAT_HIT) where the gap exceeds T, else undecided. (sat_filter
+// written with these took 15 % longer in the steps.)
+__device__ __forceinline__ void sat_bounds(const SatFrame<float, v3f>& s, float& t_n1, float& t_ef, float& t_g,
+                                           float& t_h)
+{
+    const v3f M = vmaxc(vmaxc(vmaxc(vabs(s.p2), vabs(s.p3)), vmaxc(vabs(s.q1), vabs(s.q2))), vabs(s.q3));
+    const float xyz = M.x * M.y * M.z;
+    const float xx = M.x * M.x, yy = M.y * M.y, zz = M.z * M.z;
+    const float W = (xx * yy + yy * zz) + zz * xx;
+    constexpr float U = 32.0f * 5.9604645e-8f, TINY = 7.888609e-31f;
+    t_n1 = U * 24.0f * xyz + TINY;
+    t_ef = U * 48.0f * xyz + TINY;
+    t_g = U * 32.0f * W + TINY;
+    t_h = U * 64.0f * W + TINY;
+}
+
+__device__ __forceinline__ int filter_axis(const SatFrame<float, v3f>& s, v3f ax, float T)
+{
+    const v3f p1 = v3f{0, 0, 0};
+    const float P1 = vdot<float>(ax, p1), P2 = vdot<float>(ax, s.p2), P3 = vdot<float>(ax, s.p3);
+    const float Q1 = vdot<float>(ax, s.q1), Q2 = vdot<float>(ax, s.q2), Q3 = vdot<float>(ax, s.q3);
+    const float mx1 = fmaxf(fmaxf(P1, P2), P3), mn1 = fminf(fminf(P1, P2), P3);
+    const float mx2 = fmaxf(fmaxf(Q1, Q2), Q3), mn2 = fminf(fminf(Q1, Q2), Q3);
+    const bool finite = (T < __builtin_inff());
+    // separation on this axis: mn1 > mx2 or mn2 > mx1
+    if (finite && (mn1 - mx2 > T || mn2 - mx1 > T)) return SAT_SEPARATED;
+    return finite && mx2 - mn1 > T && mx1 - mn2 > T ? SAT_HIT : SAT_UNDECIDED;
+}
+
 // the FP64 oracle's SAT over the widened FP32 inputs (every axis until one
 // separates); counts the axes evaluated
 __device__ bool sat_f64_counted(const v3f* P, const v3f* Q, uint32_t& n_fp64)
@@ -466,6 +496,9 @@ __device__ __forceinline__ bool share_vertex(const uint32_t* a, const uint32_t* 
     return s;
 }
 
+template <class Tab>
+__device__ __forceinline__ bool narrow_gather(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
+                                              uint2 c, bool count_adj, uint32_t& n_adj, v3f* P, v3f* Q, uint4& id);
 template <bool FP64, class Tab>
 __device__ __forceinline__ void narrow_one(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
                                            uint2 c, bool& hit, uint4& out, uint32_t& n_fp64, uint32_t& n_adj);
@@ -737,6 +770,457 @@ k_bvtt_step(StepArgs<Tab> A)
     block_scan(n_tests, s_wsum, nt);
     block_scan(n_adj, s_wsum, na);
     if (tid == 0) add_stat(A.stat, nt, na, 0u, FUSED ? n_cands : 0u);
+}
+
+// ---------------------------------------------------------------------------
+// k_bvtt_walk: one or two steps of the walk over a short front, 2^e lanes per
+// front pair (lane x tests child x of the first side against the second side's
+// run) instead of a thread per front pair.
+//
+// A short front is bound by latency, not by work: a k_bvtt_step of E = 3 took
+// 13-16 us on fronts of 100 to 10,000 pairs, most of it a few waves running 30 KB
+// of unrolled code (64 box tests, the output loop) once, cold. Here a wave's code
+// is a few hundred instructions, and the children of the first step stay in LDS,
+// where the workgroup's waves share them for the second: a launch, the front's
+// length, its entries and an output slot are fetched once for two steps.
+//
+// A workgroup takes `per` front pairs at a time: phase 0 loads them (and tests
+// them, on the initial front); then, WALK_MID >> 2 e1 pairs per round, so that
+// their children always fit into LDS, phase 1 expands them by e1 levels and phase
+// 2 their children by e2. Kept pairs of the last phase, and leaf pairs, gather in
+// rings in LDS: the first go to the global front in blocks, one fetch_add each,
+// the others are tested in blocks (FUSE as in k_bvtt_step). Fronts, candidates,
+// counts per level and statistics are those of the same steps one by one.
+// The rings are small (25 KB a workgroup in all) so that workgroups find room
+// beside a refit; with 64 KB lists the same walks took 16 overlapped frames of two
+// 1M-triangle bodies from 1,111 to 1,310 us.
+// Frame and pairs: two bodies of 1,280 triangles 102 -> 68 us, of 81,920 128 -> 91,
+// of 1M 183 -> 159. Of a walk's 11 us on 100 pairs, 1.8 are the launch and the
+// front's length, 3.4 the entries and their boxes, 2.6 each step.
+// ---------------------------------------------------------------------------
+#define WALK_T 256
+#define WALK_MID 1024   // first-step children per round
+#define WALK_RING 512   // a ring is emptied from WALK_T pairs on
+#define WALK_COOP 64    // up to this many leaf pairs at a time are tested by 16 lanes each
+
+template <class Tab>
+struct WalkArgs {
+    Tab tab;
+    const uint2* front_in;
+    const uint32_t* count_in;  // length of front_in; null: n_in
+    uint32_t n_in;
+    uint32_t cap_in;           // entries front_in can hold
+    uint32_t e1, e2;           // levels of the first and the second step (e2 = 0: one step)
+    uint32_t test_entries;     // test the input pairs themselves (the initial front)
+    uint2* front_out;
+    uint32_t* count_mid;       // two steps: pairs the first step keeps (a count only)
+    uint32_t* count_out;
+    uint32_t cap_out;
+    uint2* cands;
+    uint32_t* cand_count;
+    uint32_t cand_cap;
+    uint32_t* error;
+    oi_detect_stat* stat;
+    uint4* hits;
+    uint32_t* n_hits;
+    uint32_t hits_cap;
+    uint2* defer;
+    uint32_t* defer_count;
+    uint32_t defer_cap;
+    uint32_t implicit_end;
+};
+
+struct WalkLds {
+    uint2 q0[WALK_T];
+    uint2 mid[WALK_MID];
+    uint2 out[WALK_RING];
+    uint2 cand[WALK_RING];
+    float box[WALK_T / 64][64 * 6];  // a wave's second-side boxes
+    uint32_t n0, n_mid;              // entries of q0 and mid
+    uint32_t n_out, n_cand;          // pairs ever put into the rings
+    uint32_t base, hbase, dbase, nh, nd;
+};
+
+// orders a wave's LDS accesses (its lanes exchange boxes)
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// n kept pairs of the ring, from the done-th on, to the global front (every
+// thread calls; a barrier precedes)
+template <class Tab>
+__device__ __forceinline__ void walk_flush(const WalkArgs<Tab>& A, WalkLds& S, uint32_t done, uint32_t n)
+{
+    if (threadIdx.x == 0) S.base = add_u32(A.count_out, n);
+    __syncthreads();
+    const uint32_t base = S.base;
+    if (threadIdx.x == 0 && base + n > A.cap_out) or_u32(A.error, OI_ERR_QUEUE_OVERFLOW);
+    for (uint32_t i = threadIdx.x; i < n; i += WALK_T)
+        if (base + i < A.cap_out) A.front_out[base + i] = S.out[(done + i) & (WALK_RING - 1u)];
+    __syncthreads();
+}
+
+// The SAT (or the filter, FILTER) on one candidate by 16 neighbouring lanes, each
+// taking axis `lane mod 16` and the first also the 17th. Every axis is a cross
+// product of two of e1, e2, e3, n1, f1, f2, f3, m1 (n1 = e1 x e2 and m1 = f1 x f2
+// themselves), so a lane picks its two factors; the operations on them are
+// sat_f32's and sat_filter's. All 16 lanes hold the same triangles. Returns
+// SAT_*. For few candidates only: the chain is 2 axes long, not 17, for 16 times
+// the frames.
+template <bool FILTER>
+__device__ __forceinline__ int sat_lanes(const v3f* P, const v3f* Q)
+{
+    SatFrame<float, v3f> s;
+    s.init(P, Q);
+    float t_n1 = 0, t_ef = 0, t_g = 0, t_h = 0;
+    if (FILTER) sat_bounds(s, t_n1, t_ef, t_g, t_h);
+    const uint32_t lane = threadIdx.x & 63u, shift = lane & 48u;
+    bool separated = false, undecided = false;
+    for (uint32_t k = lane & 15u; k < 17u; k += 16u) {
+        // factors 0-2: e, 3: n1, 4-6: f, 7: m1
+        uint32_t iu, iw;
+        if (k < 2u) {
+            iu = 4u * k;
+            iw = iu + 1u;
+        } else if (k < 11u) {
+            iu = (k - 2u) / 3u;
+            iw = 4u + (k - 2u) % 3u;
+        } else if (k < 14u) {
+            iu = k - 11u;
+            iw = 3u;
+        } else {
+            iu = k - 10u;
+            iw = 7u;
+        }
+        v3f u = s.e1, w = s.e2;  // (w: factor 0 never is the second)
+#define OI_PICK(i, f)    \
+    if (iu == i) u = f;  \
+    if (iw == i) w = f;
+        OI_PICK(1u, s.e2)
+        OI_PICK(2u, s.e3)
+        OI_PICK(3u, s.n1)
+        OI_PICK(4u, s.f1)
+        OI_PICK(5u, s.f2)
+        OI_PICK(6u, s.f3)
+        OI_PICK(7u, s.m1)
+#undef OI_PICK
+        const v3f ax = vcross(u, w);
+        if (FILTER) {
+            const float T = k == AX_N1 ? t_n1 : k <= AX_E33 ? t_ef : k <= AX_G3 ? t_g : t_h;
+            const int r = filter_axis(s, ax, T);
+            separated |= r == SAT_SEPARATED;
+            undecided |= r == SAT_UNDECIDED;
+        } else {
+            separated |= !project6<float, v3f>(s, ax);
+        }
+    }
+    const uint32_t sep = (uint32_t)(__ballot(separated) >> shift) & 0xffffu;
+    const uint32_t und = (uint32_t)(__ballot(undecided) >> shift) & 0xffffu;
+    return sep ? SAT_SEPARATED : und ? SAT_UNDECIDED : SAT_HIT;
+}
+
+// n leaf pairs of the ring, from the done-th on: to the candidate list (FUSE 0),
+// or through the SAT (1) or the FP32 filter (2), one per thread, or 16 lanes per
+// pair where there are few (every thread calls; a barrier precedes)
+template <int FUSE, class Tab>
+__device__ __forceinline__ void walk_leaves(const WalkArgs<Tab>& A, WalkLds& S, const oi_mesh_desc* s_desc,
+                                            const uint32_t* s_ibase, uint32_t done, uint32_t n, uint32_t& n_adj)
+{
+    const uint32_t tid = threadIdx.x;
+    if constexpr (FUSE == 0) {
+        if (tid == 0) S.base = add_u32(A.cand_count, n);
+        __syncthreads();
+        const uint32_t base = S.base;
+        if (tid == 0 && base + n > A.cand_cap) or_u32(A.error, OI_ERR_CAND_OVERFLOW);
+        for (uint32_t i = tid; i < n; i += WALK_T)
+            if (base + i < A.cand_cap) A.cands[base + i] = S.cand[(done + i) & (WALK_RING - 1u)];
+        __syncthreads();
+    } else {
+        const bool coop = n <= WALK_COOP;
+        const uint32_t lg = coop ? 4u : 0u, per = WALK_T >> lg;
+        for (uint32_t c0 = 0; c0 < n; c0 += per) {
+            if (tid == 0) S.nh = S.nd = 0;
+            __syncthreads();
+            const uint32_t c = c0 + (tid >> lg);
+            int r = SAT_SEPARATED;
+            uint2 pr = make_uint2(0, 0);
+            uint4 h = make_uint4(0, 0, 0, 0);
+            if (c < n) {
+                pr = S.cand[(done + c) & (WALK_RING - 1u)];
+                v3f P[3], Q[3];
+                if (narrow_gather(A.tab, s_ibase, s_desc, pr, (tid & ((1u << lg) - 1u)) == 0u, n_adj, P, Q, h)) {
+                    if (coop)
+                        r = sat_lanes<FUSE == 2>(P, Q);
+                    else if (FUSE == 2)
+                        r = sat_filter(P, Q);
+                    else
+                        r = sat_f32(P, Q) ? SAT_HIT : SAT_SEPARATED;
+                }
+                if (tid & ((1u << lg) - 1u)) r = SAT_SEPARATED;  // the pair's first lane answers
+            }
+            const bool hit = r == SAT_HIT, dfr = FUSE == 2 && r == SAT_UNDECIDED;
+            const uint32_t at = hit ? atomicAdd(&S.nh, 1u) : 0u, atd = dfr ? atomicAdd(&S.nd, 1u) : 0u;
+            __syncthreads();
+            if (tid == 0) {
+                S.hbase = S.nh ? add_u32(A.n_hits, S.nh) : 0u;
+                if (FUSE == 2) S.dbase = S.nd ? add_u32(A.defer_count, S.nd) : 0u;
+            }
+            __syncthreads();
+            if (hit) {
+                if (S.hbase + at < A.hits_cap)
+                    A.hits[S.hbase + at] = h;
+                else
+                    or_u32(A.error, OI_ERR_HITS_OVERFLOW);
+            }
+            if (dfr) {
+                if (S.dbase + atd < A.defer_cap)
+                    A.defer[S.dbase + atd] = pr;
+                else
+                    or_u32(A.error, OI_ERR_CAND_OVERFLOW);
+            }
+        }
+    }
+}
+
+// One pass of the workgroup over the n pairs of src from the i0-th on, e levels
+// down: lane x of a pair's 2^e lanes tests child x of the first side against every
+// child of the second (whose boxes its lanes share through LDS W). Returns the
+// lane's kept child pairs (bit y: (x, y)) and pr = pair (x, 0); `leaf` says that
+// they are leaf pairs.
+template <class Tab>
+__device__ __forceinline__ uint32_t walk_pass(const WalkArgs<Tab>& A, float* W, const oi_mesh_desc* s_desc,
+                                              const uint32_t* s_ibase, const uint2* src, uint32_t i, uint32_t n,
+                                              uint32_t e, uint2& pr, bool& leaf, uint32_t& n_tests, uint32_t& n_adj)
+{
+    const uint32_t K = 1u << e, lane = threadIdx.x & 63u, x = lane & (K - 1u);
+    bool mine = false, same = false, selfnode = false;
+    uint32_t cntb = 0;
+    const uint32_t *fa = nullptr, *fb = nullptr;
+    float ba[6];
+    if (i < n) {
+        const uint2 en = src[i];
+        uint32_t ma, mb;
+        const MeshRef ra = tab_ref(A.tab, s_desc, s_ibase, en.x, ma);
+        const MeshRef rb = tab_ref(A.tab, s_desc, s_ibase, en.y, mb);
+        const uint32_t ia = en.x - ra.ibase, ib = en.y - rb.ibase;
+        const uint32_t la = oi_ilog2(ia + 1u), lb = oi_ilog2(ib + 1u);
+        selfnode = en.x == en.y;
+        same = ma == mb;
+        const Side sa = expand_side(ia, la, ra.L, ra.vl, e), sb = expand_side(ib, lb, rb.L, rb.vl, e);
+        const uint32_t ca = min(la + e, ra.L), cb = min(lb + e, rb.L);
+        leaf = ca == ra.L && cb == rb.L;
+        mine = x < sa.count;
+        cntb = sb.count;
+        // (slots past a run's end repeat its last node)
+        float bb[6];
+        load_box(ra.nodes, sa.start + min(x, sa.count - 1u) - oi_virt_above(ca, ra.L, ra.vl), ba);
+        load_box(rb.nodes, sb.start + min(x, sb.count - 1u) - oi_virt_above(cb, rb.L, rb.vl), bb);
+        pr = make_uint2(ra.ibase + sa.start + x, rb.ibase + sb.start);
+        const uint32_t leaf0 = (1u << ra.L) - 1u;
+        fa = ra.sfaces + 3ull * (sa.start + x - leaf0);  // (used for leaf pairs of one mesh)
+        fb = ra.sfaces + 3ull * (sb.start - leaf0);
+        float2* w = reinterpret_cast<float2*>(W + 6u * lane);
+        w[0] = make_float2(bb[0], bb[1]);
+        w[1] = make_float2(bb[2], bb[3]);
+        w[2] = make_float2(bb[4], bb[5]);
+    }
+    wave_fence();
+    if (!mine) return 0u;
+    uint32_t hit = 0;
+    const float2* w = reinterpret_cast<const float2*>(W + 6u * (lane & ~(K - 1u)));
+#pragma unroll 1
+    for (uint32_t y = 0; y < K; y += 2u, w += 6) {  // two of the K = 2, 4 or 8 at a time
+        const float2 p0 = w[0], q0 = w[1], r0 = w[2], p1 = w[3], q1 = w[4], r1 = w[5];
+        const float b0[6] = {p0.x, p0.y, q0.x, q0.y, r0.x, r0.y}, b1[6] = {p1.x, p1.y, q1.x, q1.y, r1.x, r1.y};
+        hit |= (overlap6(ba, b0) ? 1u : 0u) << y;
+        hit |= (overlap6(ba, b1) ? 2u : 0u) << y;
+    }
+    // the pairs that exist; of a node with itself the unordered ones, and its
+    // children with themselves unless they are leaves
+    uint32_t tested = (1u << cntb) - 1u;
+    if (selfnode) tested &= ~((2u << x) - 1u);
+    n_tests += (uint32_t)__popc(tested);
+    uint32_t mask = hit & tested;
+    if (selfnode && !leaf) mask |= 1u << x;
+    if (leaf && same && mask) {
+        // inside one mesh (self mode) leaf pairs sharing a vertex are not
+        // collisions
+        uint32_t f[3];
+        oi_ld3(fa, 0, f);
+        for (uint32_t m = mask; m; m &= m - 1u) {
+            const uint32_t y = (uint32_t)__ffs((int)m) - 1u;
+            uint32_t g[3];
+            oi_ld3(fb, y, g);
+            if (share_vertex(f, g)) {
+                mask &= ~(1u << y);
+                n_adj++;
+            }
+        }
+    }
+    return mask;
+}
+
+// One loop over the passes, so that the code of a pass, and of emptying a ring,
+// is there once: a few KB that stay in the instruction cache.
+template <int FUSE, class Tab>
+__global__ void __launch_bounds__(WALK_T) k_bvtt_walk(WalkArgs<Tab> A)
+{
+    __shared__ oi_mesh_desc s_desc[MESH_LDS];
+    __shared__ uint32_t s_ibase[MESH_LDS];
+    __shared__ WalkLds S;
+    // after an overflow the count keeps growing past the buffer (writes were
+    // dropped and the detect will be re-run): read only what exists
+    uint32_t n_in = A.count_in ? *A.count_in : A.n_in;
+    if (n_in > A.cap_in) n_in = A.cap_in;
+    // an even share per workgroup, at most one pair per thread at a time, in
+    // groups of 2^lgg neighbours dealt out in turn: neighbours in a front descend
+    // from one pair and read the same nodes, but a long run of them would leave
+    // one workgroup with all the work of a dense spot. (Shallow steps leave little
+    // work per pair, mostly leaf tests, which run in fewer, fuller workgroups.)
+    const uint32_t lgg = n_in >= 32u * gridDim.x ? 5u : n_in >= 8u * gridDim.x || A.e1 + A.e2 <= 2u ? 3u : 0u;
+    if ((blockIdx.x << lgg) >= n_in) return;
+    const uint32_t share = gridDim.x << lgg;
+    const uint32_t per = min((n_in + share - 1u) / share << lgg, (uint32_t)WALK_T);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    if (tid == 0) S.n0 = S.n_mid = S.n_out = S.n_cand = 0;
+    tab_init(A.tab, s_desc, s_ibase);
+    __syncthreads();
+    uint32_t n_tests = 0, n_adj = 0, n_mids = 0;
+    uint32_t out_done = 0, cand_done = 0;  // pairs that have left the rings
+    const uint32_t round = WALK_MID >> (2u * A.e1);
+    // the list being expanded: n pairs at src, e levels; second: it is S.mid
+    uint32_t b0 = blockIdx.x << lgg, r0 = 0, n0 = 0, i0 = 0, n = 0, e = A.e1;
+    const uint2* src = S.q0;
+    bool second = false, fin = false;
+    while (!fin) {
+        if (i0 >= n) {
+            // the next list (every branch is uniform; the code before ends with
+            // a barrier)
+            i0 = 0;
+            if (n && A.e2 && !second) {
+                second = true;
+                src = S.mid;
+                n = S.n_mid;
+                e = A.e2;
+                n_mids += n;
+                if (n == 0) continue;
+            } else {
+                if (second) {
+                    second = false;
+                    __syncthreads();
+                    if (tid == 0) S.n_mid = 0;
+                    __syncthreads();
+                }
+                r0 += round;
+                if (r0 >= n0) {
+                    if (b0 >= n_in) {
+                        fin = true;  // only the rings are left
+                    } else {
+                        const uint32_t i = b0 + (tid >> lgg) * share + (tid & ((1u << lgg) - 1u));
+                        bool have = tid < per && i < n_in;
+                        uint2 en = make_uint2(0, 0);
+                        if (have) en = A.front_in[i];
+                        if (have && (en.x >= A.implicit_end || en.y >= A.implicit_end)) {
+                            or_u32(A.error, OI_ERR_CORRUPT);  // never dereference a bad entry
+                            have = false;
+                        }
+                        if (have && A.test_entries && en.x != en.y) {
+                            uint32_t ma, mb;
+                            const MeshRef ra = tab_ref(A.tab, s_desc, s_ibase, en.x, ma);
+                            const MeshRef rb = tab_ref(A.tab, s_desc, s_ibase, en.y, mb);
+                            const uint32_t ia = en.x - ra.ibase, ib = en.y - rb.ibase;
+                            const uint32_t la = oi_ilog2(ia + 1u), lb = oi_ilog2(ib + 1u);
+                            if (la != ra.L || lb != rb.L) {  // (a leaf pair is tested when expanded)
+                                float ba[6], bb[6];
+                                load_box(ra.nodes, ia - oi_virt_above(la, ra.L, ra.vl), ba);
+                                load_box(rb.nodes, ib - oi_virt_above(lb, rb.L, rb.vl), bb);
+                                have = overlap6(ba, bb);
+                                n_tests++;
+                            }
+                        }
+                        const u64 m = __ballot(have);
+                        uint32_t at = 0;
+                        if (lane == 0 && m) at = atomicAdd(&S.n0, (uint32_t)__popcll(m));
+                        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+                        if (have)
+                            S.q0[at + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = en;
+                        __syncthreads();
+                        n0 = S.n0;
+                        __syncthreads();
+                        if (tid == 0) S.n0 = 0;
+                        __syncthreads();
+                        b0 += gridDim.x * per;
+                        r0 = 0;
+                    }
+                }
+                src = S.q0 + r0;
+                n = fin ? 0u : min(round, n0 - r0);
+                e = A.e1;
+                if (n == 0 && !fin) continue;
+            }
+        }
+        uint32_t m = 0, at = 0;
+        uint2 pr = make_uint2(0, 0);
+        bool leaf = false;
+        const bool to_mid = A.e2 && !second;
+        if (!fin) {
+            m = walk_pass(A, S.box[tid >> 6], s_desc, s_ibase, src, i0 + (tid >> e), n, e, pr, leaf, n_tests, n_adj);
+            i0 += WALK_T >> e;
+            // places: kept pairs in the low half, leaf pairs in the high half of
+            // one scan (512 a wave at most), one LDS atomic per wave and list
+            const uint32_t cnt = (uint32_t)__popc(m), v = leaf ? cnt << 16 : cnt;
+            const uint32_t incl = oi_wave_scan_incl(v);
+            const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+            uint32_t a0 = 0, a1 = 0;
+            if (lane == 0 && (tot & 0xffffu)) a0 = atomicAdd(to_mid ? &S.n_mid : &S.n_out, tot & 0xffffu);
+            if (lane == 0 && (tot >> 16)) a1 = atomicAdd(&S.n_cand, tot >> 16);
+            a0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)a0);
+            a1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)a1);
+            at = leaf ? a1 + ((incl - v) >> 16) : a0 + ((incl - v) & 0xffffu);
+        }
+        for (;;) {
+            // what fits into the rings (mid holds everything a round can give);
+            // while one is full enough it is emptied and the rest follows
+            uint2* dst = leaf ? S.cand : to_mid ? S.mid : S.out;
+            const uint32_t wrap = !leaf && to_mid ? WALK_MID - 1u : WALK_RING - 1u;
+            const uint32_t lim = leaf ? cand_done + WALK_RING : to_mid ? WALK_MID : out_done + WALK_RING;
+            for (; m && (int32_t)(lim - at) > 0; m &= m - 1u, at++)
+                dst[at & wrap] = make_uint2(pr.x, pr.y + (uint32_t)__ffs((int)m) - 1u);
+            __syncthreads();
+            const uint32_t no = S.n_out - out_done, nc = S.n_cand - cand_done;
+            __syncthreads();  // every thread has read them before the next pass adds
+            const uint32_t full = fin ? 1u : WALK_T;
+            if (no < full && nc < full) break;
+            if (no >= full) {
+                const uint32_t take = min(no, (uint32_t)WALK_RING);
+                walk_flush(A, S, out_done, take);
+                out_done += take;
+            }
+            if (nc >= full) {
+                const uint32_t take = min(nc, (uint32_t)WALK_T);
+                walk_leaves<FUSE>(A, S, s_desc, s_ibase, cand_done, take, n_adj);
+                cand_done += take;
+                __syncthreads();
+            }
+        }
+    }
+    // statistics: the waves' sums, added by one thread
+    for (int d = 32; d; d >>= 1) {
+        n_tests += (uint32_t)__shfl_xor((int)n_tests, d, 64);
+        n_adj += (uint32_t)__shfl_xor((int)n_adj, d, 64);
+    }
+    if (lane == 0) S.mid[tid >> 6] = make_uint2(n_tests, n_adj);
+    __syncthreads();
+    if (tid == 0) {
+        uint2 sum = S.mid[0];
+        for (uint32_t w = 1; w < WALK_T / 64u; w++) sum = make_uint2(sum.x + S.mid[w].x, sum.y + S.mid[w].y);
+        add_stat(A.stat, sum.x, sum.y, 0u, FUSE ? cand_done : 0u);
+    }
+    if (tid == 0 && n_mids) add_u32(A.count_mid, n_mids);
 }
 
 // ---------------------------------------------------------------------------
@@ -1252,6 +1736,46 @@ static hipError_t launch_step(hipStream_t st, uint32_t grid, const Tab& tab, int
 }
 
 template <class Tab>
+static hipError_t launch_walk(hipStream_t st, uint32_t grid, const Tab& tab, const oi_walk_args& w, uint2* cands,
+                              uint32_t* cand_count, uint32_t cand_cap, uint4* hits, uint32_t hits_cap,
+                              oi_detect_ctl* ctl, uint32_t implicit_end, int fused)
+{
+    WalkArgs<Tab> a{};
+    a.tab = tab;
+    a.front_in = w.front_in;
+    a.count_in = w.count_in;
+    a.n_in = w.n_in;
+    a.cap_in = w.count_in ? w.cap_in : w.n_in;
+    a.e1 = w.e1;
+    a.e2 = w.e2;
+    a.test_entries = w.test_entries;
+    a.front_out = w.front_out;
+    a.count_mid = w.count_mid;
+    a.count_out = w.count_out;
+    a.cap_out = w.cap_out;
+    a.cands = cands;
+    a.cand_count = cand_count;
+    a.cand_cap = cand_cap;
+    a.error = &ctl->error;
+    a.stat = ctl->stat;
+    a.hits = hits;
+    a.n_hits = &ctl->n_hits;
+    a.hits_cap = hits_cap;
+    a.defer = cands;  // as in launch_step
+    a.defer_count = &ctl->deferred;
+    a.defer_cap = cand_cap;
+    a.implicit_end = implicit_end;
+    const dim3 g(grid), b(WALK_T);
+    switch (fused) {
+    case 0: launch_done((k_bvtt_walk<0, Tab>), g, b, st, w.done, a); break;
+    case 1: launch_done((k_bvtt_walk<1, Tab>), g, b, st, w.done, a); break;
+    case 2: launch_done((k_bvtt_walk<2, Tab>), g, b, st, w.done, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+template <class Tab>
 static hipError_t launch_local(hipStream_t st, const Tab& tab, const oi_local_args& w, uint2* cands,
                                uint32_t* cand_count, uint32_t cand_cap, uint4* hits, uint32_t hits_cap,
                                oi_detect_ctl* ctl, uint32_t expand, uint32_t implicit_end, int fused)
@@ -1363,6 +1887,19 @@ hipError_t oi_launch_bvtt_step(hipStream_t st, uint32_t grid, const oi_tab_args*
     return launch_step(st, grid, make_tab(t->d_meshes, t->h_meshes, t->n_meshes), first, front_in, count_in, n_in,
                        cap_in, front_out, count_out, cap_out, cands, cand_count, cand_cap, hits, hits_cap, ctl,
                        expand, implicit_end, fused, done);
+}
+
+// one or two steps over a short front (k_bvtt_walk), `grid` workgroups
+hipError_t oi_launch_bvtt_walk(hipStream_t st, uint32_t grid, const oi_tab_args* t, const oi_walk_args* w,
+                               uint2* cands, uint32_t* cand_count, uint32_t cand_cap, uint4* hits, uint32_t hits_cap,
+                               oi_detect_ctl* ctl, uint32_t implicit_end, int fused)
+{
+    if (grid == 0 || w->e1 < 1 || w->e1 > 3 || w->e2 > 3 || (w->e2 && !w->count_mid)) return hipErrorInvalidValue;
+    if (t->chunk_mesh)
+        return launch_walk(st, grid, ChunkTab{t->d_meshes, t->chunk_mesh, t->shift}, *w, cands, cand_count, cand_cap,
+                           hits, hits_cap, ctl, implicit_end, fused);
+    return launch_walk(st, grid, make_tab(t->d_meshes, t->h_meshes, t->n_meshes), *w, cands, cand_count, cand_cap,
+                       hits, hits_cap, ctl, implicit_end, fused);
 }
 
 // the first `levels` steps in one launch, one workgroup per `chunk` initial

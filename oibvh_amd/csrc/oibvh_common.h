@@ -210,6 +210,21 @@ struct oi_local_args {
     hipEvent_t done;           // recorded when the launch completes (null: none)
 };
 
+// one launch of k_bvtt_walk
+struct oi_walk_args {
+    const uint2* front_in;
+    const uint32_t* count_in;  // device length of front_in (null: n_in)
+    uint32_t n_in;
+    uint32_t cap_in;           // entries front_in holds (with count_in)
+    uint32_t e1, e2;           // levels of the first and the second step (e2 = 0: one step)
+    uint32_t test_entries;     // test the input pairs themselves (the initial front)
+    uint2* front_out;
+    uint32_t* count_mid;       // with e2: counts the first step's kept pairs
+    uint32_t* count_out;
+    uint32_t cap_out;
+    hipEvent_t done;           // recorded when the launch completes (null: none)
+};
+
 // the bytes a device sort of the hit list visits, least significant first:
 // digit p is byte shift[p] / 8 of word word[p] (0 meshA, 1 meshB, 2 triA,
 // 3 triB)

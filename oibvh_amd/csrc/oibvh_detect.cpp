@@ -127,6 +127,35 @@ oibvh_status oi_det_set_front(oi_detector* d, const std::vector<uint2>& front)
     return OIBVH_OK;
 }
 
+// Steps over short fronts as k_bvtt_walk launches, two steps each where the
+// second's tests are few as well. The host does not know the fronts' lengths: it
+// takes them to grow by e + 1 per step of e levels (measured: 2.0-2.9 for two
+// levels and 2.8-4.2 for three, two bodies), in self mode by 2^e + 3 (4-8 and
+// 9-15, folded cloth). A wrong guess costs speed only.
+// Where the lines lie: one k_bvtt_step of three levels takes 15 us on any front up
+// to 10,000 pairs and 18-25 us at 50,000, a walk of two such steps 11 us at 100
+// pairs, 19 us at 2,800 and of one step 14 us at 10,000; a step of two levels
+// takes 8 us up to 10,000 pairs, a walk of two 11 us at 36 and 19 us at 2,400.
+#define OI_WALK_MAX3 65536u
+#define OI_WALK_MAX 2048u
+#define OI_WALK_TESTS (1u << 21)
+static void plan_walk(oi_detector* d)
+{
+    std::memset(d->step_walk, 0, sizeof d->step_walk);
+    if (d->local_chunk || d->tail_chunk || d->n_front == 0) return;
+    const bool self = (d->flags & OIBVH_DETECT_SELF) != 0;
+    uint64_t est = d->n_front;
+    auto grown = [&](uint32_t k) { return est * (self ? (1u << d->step_e[k]) + 3u : d->step_e[k] + 1u); };
+    for (uint32_t k = 0; k < d->n_levels && est <= (d->step_e[k] == 3 ? OI_WALK_MAX3 : OI_WALK_MAX); k++) {
+        d->step_walk[k] = 1;
+        est = grown(k);
+        if (k + 1 < d->n_levels && est << (2u * d->step_e[k + 1]) <= OI_WALK_TESTS) {
+            d->step_walk[k++] = 2;
+            est = grown(k);
+        }
+    }
+}
+
 oibvh_status oi_det_prepare(oi_detector* d)
 {
     oibvh_ctx* c = d->ctx;
@@ -149,6 +178,7 @@ oibvh_status oi_det_prepare(oi_detector* d)
         done += e;
     }
     d->n_levels = k;
+    const uint32_t past = d->depth && done > d->depth ? done - d->depth : 0u;
     // the first steps as one local walk when asked for, unless it overflowed
     // recently; its steps all descend `expand` levels
     const uint32_t mode = c->trav_local;
@@ -184,6 +214,10 @@ oibvh_status oi_det_prepare(oi_detector* d)
             d->tail_from = T;
         }
     }
+    // no side has more levels left than the deepest tree: levels of the last step
+    // past its leaves would only repeat tests
+    if (!d->local_chunk && !d->tail_chunk) d->step_e[d->n_levels - 1] -= (uint8_t)past;
+    plan_walk(d);
     const uint32_t fcap = std::max(std::max(c->queue_cap, d->want_front), oi_np2(std::max(1u, d->n_front)));
     if (d->front_cap < fcap) {
         oibvh_status ri = idle(c);
@@ -255,11 +289,37 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
                                        d->ctl, d->expand, d->implicit_end, d->fused ? 1 : 0));
         done_head = nullptr;
     }
+    // the buffer that holds the current front (step 0 reads the initial front
+    // in place); every launch writes the other one
+    uint32_t rd = J ? (J - 1) & 1u : 1u;
     for (uint32_t k = J; k < T; k++) {
-        // step 0 reads the initial front in place; then the fronts alternate
-        const uint2* in = k ? d->front[(k - 1) & 1] : d->d_init;
+        const uint2* in = k ? d->front[rd] : d->d_init;
+        rd ^= 1u;
+        if (d->step_walk[k]) {
+            // this step, or this and the next one, over a short front
+            const bool two = d->step_walk[k] == 2;
+            const uint32_t o = two ? k + 1 : k;
+            oi_walk_args w{};
+            w.front_in = in;
+            w.count_in = k ? d->counts + k : nullptr;
+            w.n_in = d->n_front;
+            w.cap_in = k ? d->front_cap : d->n_front;
+            w.e1 = d->step_e[k];
+            w.e2 = two ? d->step_e[k + 1] : 0u;
+            w.test_entries = k == 0 ? 1u : 0u;
+            w.front_out = d->front[rd];
+            w.count_mid = two ? d->counts + k + 1 : nullptr;
+            w.count_out = d->counts + o + 1;
+            w.cap_out = d->front_cap;
+            w.done = (!narrow && !tail && o + 1 == T) ? done : nullptr;
+            HIPCHK(c, oi_launch_bvtt_walk(st, (uint32_t)std::max(1, c->cus) * 2u, &d->tab, &w, d->cands,
+                                          &d->ctl->cands, d->cand_cap, d->hits, d->hits_cap, d->ctl, d->implicit_end,
+                                          fuse));
+            k = o;
+            continue;
+        }
         HIPCHK(c, oi_launch_bvtt_step(st, grid, &d->tab, k == 0, in, k ? d->counts + k : nullptr, d->n_front,
-                                      k ? d->front_cap : d->n_front, d->front[k & 1], d->counts + k + 1,
+                                      k ? d->front_cap : d->n_front, d->front[rd], d->counts + k + 1,
                                       d->front_cap, d->cands, &d->ctl->cands, d->cand_cap, d->hits, d->hits_cap,
                                       d->ctl, d->step_e[k], d->implicit_end, fuse,
                                       (!narrow && !tail && k + 1 == T) ? done : nullptr));
@@ -270,7 +330,7 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
         // front (its count, checked below, stays 0); front_out is the buffer
         // not being read
         oi_local_args w{};
-        w.front_in = T ? d->front[(T - 1) & 1] : d->d_init;
+        w.front_in = T ? d->front[rd] : d->d_init;
         w.count_in = T ? d->counts + T : nullptr;
         w.n_in = d->n_front;
         w.cap_in = T ? d->front_cap : d->n_front;
@@ -279,7 +339,7 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
         w.grid = 4u * (uint32_t)std::max(1, c->cus);
         w.test_entries = T == 0 ? 1u : 0u;
         w.overflow_bit = OI_ERR_TAIL_OVERFLOW;
-        w.front_out = d->front[T & 1];
+        w.front_out = d->front[rd ^ 1u];
         w.count_out = d->counts + d->n_levels;
         w.cap_out = d->front_cap;
         w.done = done_tail;

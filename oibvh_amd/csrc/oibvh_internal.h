@@ -69,6 +69,8 @@ hipError_t oi_launch_narrow(hipStream_t, uint32_t, const oi_tab_args*, const uin
                             uint4*, uint32_t*, uint32_t, oi_detect_ctl*, int, uint2*, uint32_t, hipEvent_t);
 hipError_t oi_launch_bvtt_local(hipStream_t, const oi_tab_args*, const oi_local_args*, uint2*, uint32_t*, uint32_t,
                                 uint4*, uint32_t, oi_detect_ctl*, uint32_t, uint32_t, int);
+hipError_t oi_launch_bvtt_walk(hipStream_t, uint32_t, const oi_tab_args*, const oi_walk_args*, uint2*, uint32_t*,
+                               uint32_t, uint4*, uint32_t, oi_detect_ctl*, uint32_t, int);
 hipError_t oi_launch_pair_vertices(hipStream_t, const oi_build_desc*, const uint4*, uint32_t, float*);
 hipError_t oi_launch_zero_u32(hipStream_t, uint32_t*, uint32_t);
 hipError_t oi_launch_hits_digits(hipStream_t, const uint4*, uint32_t, uint32_t*, uint32_t*, const oi_hit_digits*);
@@ -279,6 +281,7 @@ struct oi_detector {
     uint32_t depth = 0, expand = 1, flags = 0, implicit_end = 0;
     uint32_t schedule = 0;      // levels per step of the first steps (2 bits each), then `expand`
     uint8_t step_e[256] = {};   // levels descended by each step of the current query
+    uint8_t step_walk[256] = {};  // 1 or 2: step k (and k + 1) as one k_bvtt_walk launch
     uint32_t local_chunk = 0;   // this query: initial pairs per workgroup of the local walk (0: steps)
     uint32_t local_levels = 0;  // this query: steps done by the local walk
     uint64_t local_off = 0;     // 1 + the tuning generation in which the head walk overflowed (0: none)

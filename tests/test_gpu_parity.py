@@ -734,6 +734,33 @@ def test_detect_cfg1_full_size(api, ctx, orc):
         assert st["pairs"] == len(want)
 
 
+@pytest.mark.parametrize("mode", ["fp32", "separate", "fp64"])
+@pytest.mark.parametrize("expand", [1, 2, 3])
+def test_detect_walk_dense_and_sparse(api, ctx, orc, expand, mode):
+    """Short fronts (k_bvtt_walk): a sphere against itself from the root, where
+    every list in LDS fills and wraps (up to 4^e children a pair, 13 leaf pairs a
+    face), a coarse cloth in self mode, trees of unequal depth down to one face,
+    and an entry level at the leaves; with leaf pairs tested in the walk, in one
+    k_narrow launch, and through the filter: the oracle's pairs."""
+    say(f"detect walk expand={expand} {mode}")
+    fp64 = mode == "fp64"
+    a, one = M.icosphere(4, 1.0, 0.0, 0), M.plane(1, 0.5)
+    one = (one[0] + np.float32(0.1), one[1][:1])
+    cl = M.cloth(40, amplitude=0.2, wavelength=0.2, seed=5)
+    small = M.box(3, 0.9, 0.0, 1)
+    ctx.set_tuning(narrow_separate=1 if mode == "separate" else 0)
+    try:
+        for meshes, entry, self_collide in (([a, a], 0, False), ([a, a], 3, False), ([cl], 0, True),
+                                            ([a, small, one, cl], 1, True), ([small, one], 30, False)):
+            p, st, trees = gpu_pairs(api, ctx, meshes, entry, expand, self_collide=self_collide, fp64=fp64)
+            want = orc.detect([orc.Tree(x, f, order=t.perm()) for (x, f), t in zip(meshes, trees)],
+                              self_collide=self_collide, fp64=fp64)
+            assert np.array_equal(p, want), (len(meshes), entry)
+            assert st["retries"] == 0
+    finally:
+        ctx.set_tuning(narrow_separate=0)
+
+
 @pytest.mark.parametrize("entry", [0, 1, 3, 6, 30])
 @pytest.mark.parametrize("expand", [1, 2, 3, 5])
 @pytest.mark.parametrize("mode", [(0, 0), (64, 0), (7, 0), (64, 2), (16, 1),
