@@ -380,6 +380,15 @@ __device__ __forceinline__ MeshRef tab_ref(const ChunkTab& T, const oi_mesh_desc
     return MeshRef{d.nodes, d.sfaces, d.pos, d.perm, d.xf, d.L, d.vl, d.ibase};
 }
 
+__device__ __forceinline__ const uint32_t* mesh_perm(const MeshTab& T, const oi_mesh_desc* s_desc, uint32_t m)
+{
+    return (m < MESH_LDS ? s_desc[m] : T.meshes[m]).perm;
+}
+__device__ __forceinline__ const uint32_t* mesh_perm(const ChunkTab& T, const oi_mesh_desc*, uint32_t m)
+{
+    return T.meshes[m].perm;
+}
+
 // 16 zeros, read in place of a model matrix by meshes that have none
 __device__ const float k_no_xf[16] = {};
 
@@ -499,6 +508,8 @@ __device__ __forceinline__ bool share_vertex(const uint32_t* a, const uint32_t* 
 template <class Tab>
 __device__ __forceinline__ bool narrow_gather(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
                                               uint2 c, bool count_adj, uint32_t& n_adj, v3f* P, v3f* Q, uint4& id);
+template <class Tab>
+__device__ __forceinline__ uint4 hit_ids(const Tab& T, const oi_mesh_desc* s_desc, uint4 id);
 template <bool FP64, class Tab>
 __device__ __forceinline__ void narrow_one(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
                                            uint2 c, bool& hit, uint4& out, uint32_t& n_fp64, uint32_t& n_adj);
@@ -538,6 +549,14 @@ struct PairMasks {
     static constexpr u64 diag = make(true);
 };
 
+// K x K child pairs as bits
+template <int E>
+using PairMask = std::conditional_t<(E <= 2), uint32_t, u64>;
+__device__ __forceinline__ uint32_t mask_count(uint32_t m) { return (uint32_t)__popc(m); }
+__device__ __forceinline__ uint32_t mask_count(u64 m) { return (uint32_t)__popcll(m); }
+__device__ __forceinline__ uint32_t mask_first(uint32_t m) { return (uint32_t)__ffs((int)m) - 1u; }
+__device__ __forceinline__ uint32_t mask_first(u64 m) { return (uint32_t)__ffsll((long long)m) - 1u; }
+
 // One BVTT entry (a pair of implicit indices): with FIRST the pair itself is
 // tested first (an initial-front entry); then both sides descend up to E
 // levels and every pair of the two descendant runs is tested. Bit x * K + y
@@ -546,10 +565,11 @@ struct PairMasks {
 // vertex are dropped here.
 template <int E, bool FIRST, class Tab>
 __device__ __forceinline__ void entry_expand(const Tab& T, const oi_mesh_desc* s_desc, const uint32_t* s_ibase,
-                                             uint2 e, u64& mask, bool& leafout, Side& sa, Side& sb,
+                                             uint2 e, PairMask<E>& mask, bool& leafout, Side& sa, Side& sb,
                                              uint32_t& baseA, uint32_t& baseB, uint32_t& n_tests, uint32_t& n_adj)
 {
     constexpr int K = 1 << E;
+    using M = PairMask<E>;
     uint32_t ma, mb;
     const MeshRef ra = tab_ref(T, s_desc, s_ibase, e.x, ma);
     const MeshRef rb = tab_ref(T, s_desc, s_ibase, e.y, mb);
@@ -580,21 +600,21 @@ __device__ __forceinline__ void entry_expand(const Tab& T, const oi_mesh_desc* s
     // its last node), then masked to the pairs that exist: x < sa.count,
     // y < sb.count, and for a node paired with itself the unordered child
     // pairs, y > x tested and y == x kept unless they are leaves
-    u64 hit = 0;
+    M hit = 0;
 #pragma unroll
     for (int x = 0; x < K; x++)
 #pragma unroll
         for (int y = 0; y < K; y++)
-            if (overlap6(bxa[x], bxb[y])) hit |= 1ull << (x * K + y);
-    u64 rows = 0;
+            if (overlap6(bxa[x], bxb[y])) hit |= (M)1 << (x * K + y);
+    M rows = 0;
 #pragma unroll
     for (int x = 0; x < K; x++)
-        if ((uint32_t)x < sa.count) rows |= 1ull << (x * K);
-    const u64 exist = rows * ((1ull << sb.count) - 1ull);  // sb.count <= K: no carry between rows
-    const u64 tested = selfnode ? (exist & PairMasks<E>::upper) : exist;
-    n_tests += (uint32_t)__popcll(tested);
+        if ((uint32_t)x < sa.count) rows |= (M)1 << (x * K);
+    const M exist = rows * (((M)1 << sb.count) - 1);  // sb.count <= K: no carry between rows
+    const M tested = selfnode ? (exist & (M)PairMasks<E>::upper) : exist;
+    n_tests += mask_count(tested);
     mask = hit & tested;
-    if (selfnode && !leafout) mask |= exist & PairMasks<E>::diag;
+    if (selfnode && !leafout) mask |= exist & (M)PairMasks<E>::diag;
     // inside one mesh (self mode) leaf pairs sharing a vertex are not
     // collisions: drop them before they become candidates
     if (leafout && ma == mb && mask) {
@@ -602,16 +622,16 @@ __device__ __forceinline__ void entry_expand(const Tab& T, const oi_mesh_desc* s
         const uint32_t leaf0 = (1u << ra.L) - 1u;
         load_faces<E>(ra.sfaces, sa.start - leaf0, sa.count, fa);
         load_faces<E>(ra.sfaces, sb.start - leaf0, sb.count, fb);
+        // every slot pair with no branch, then masked (taken pair by pair of the
+        // mask it cost the folded cloth's last step 385 of 1,364 us)
+        M adj = 0;
 #pragma unroll
         for (int x = 0; x < K; x++)
 #pragma unroll
-            for (int y = 0; y < K; y++) {
-                const u64 bit = 1ull << (x * K + y);
-                if ((mask & bit) && share_vertex(fa[x], fb[y])) {
-                    mask &= ~bit;
-                    n_adj++;
-                }
-            }
+            for (int y = 0; y < K; y++)
+                if (share_vertex(fa[x], fb[y])) adj |= (M)1 << (x * K + y);
+        n_adj += mask_count(mask & adj);
+        mask &= ~adj;
     }
 }
 
@@ -684,182 +704,33 @@ __device__ __forceinline__ void fused_narrow(const Tab& T, const uint32_t* s_iba
     }
 }
 
-// FUSE 1: overlapping leaf pairs are tested with the FP32 SAT by the
-// workgroup that found them (fused_narrow) instead of going to the candidate
-// list; FUSE 2: with the FP32 filter, the pairs it leaves undecided going to
-// A.defer for the FP64 pass.
-// Occupancy: the step waits on its child-run loads, so resident waves matter
-// more than loads in flight per wave. E = 3 holds two runs of 8 boxes and
-// would take 153-161 VGPRs (3 waves per SIMD); capped at 128 (4 waves) it
-// keeps the runs in registers (the fused forms spill 2-5 dwords). E = 2 fits
-// 80 VGPRs (6 waves) unspilled.
-template <int E, bool FIRST, int FUSE, class Tab>
-__global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(E == 3 ? 4 : E == 2 ? 6 : 1, 8)))
-k_bvtt_step(StepArgs<Tab> A)
-{
-    constexpr bool FUSED = FUSE != 0;
-    constexpr int K = 1 << E;
-    __shared__ oi_mesh_desc s_desc[MESH_LDS];
-    __shared__ uint32_t s_ibase[MESH_LDS];
-    __shared__ uint32_t s_wsum[4];
-    __shared__ uint32_t s_obase, s_cbase;
-    __shared__ std::conditional_t<FUSED, FusedLds, char> s_f[1];
-    // after an overflow the count keeps growing past the buffer (writes were
-    // dropped and the detect will be re-run): read only what exists
-    uint32_t n_in = A.count_in ? *A.count_in : A.n_in;
-    if (n_in > A.cap_in) n_in = A.cap_in;
-    if (blockIdx.x * TB >= n_in) return;
-    tab_init(A.tab, s_desc, s_ibase);
-    const uint32_t tid = threadIdx.x;
-    uint32_t n_tests = 0, n_adj = 0, n_cands = 0, n_fp64 = 0;
-    for (uint32_t base = blockIdx.x * TB; base < n_in; base += gridDim.x * TB) {
-        const uint32_t i = base + tid;
-        bool have = i < n_in;
-        const uint2 e = have ? A.front_in[i] : make_uint2(0, 0);
-        if (have && (e.x >= A.implicit_end || e.y >= A.implicit_end)) {
-            or_u32(A.error, OI_ERR_CORRUPT);  // never dereference a bad entry
-            have = false;
-        }
-        u64 mask = 0;          // bit (x << E) + y: pair (start_a + x, start_b + y) kept
-        bool leafout = false;  // kept pairs are leaf pairs (candidates)
-        Side sa = {0, 0}, sb = {0, 0};
-        uint32_t baseA = 0, baseB = 0;
-        if (have) entry_expand<E, FIRST, Tab>(A.tab, s_desc, s_ibase, e, mask, leafout, sa, sb, baseA, baseB,
-                                              n_tests, n_adj);
-        const uint32_t nout = (uint32_t)__popcll(mask);
-        // one scan for both counts: front pairs in the high half, leaf pairs
-        // in the low half (at most 256 x 64 each, so no carry crosses)
-        uint32_t TC;
-        const uint32_t oc = block_scan(leafout ? nout : (nout << 16), s_wsum, TC);
-        const uint32_t T = TC >> 16, C = TC & 0xffffu, off = oc >> 16, coff = oc & 0xffffu;
-        if (tid == 0) {
-            s_obase = T ? add_u32(A.count_out, T) : 0u;
-            if (!FUSED) s_cbase = C ? add_u32(A.cand_count, C) : 0u;
-        }
-        if constexpr (FUSED) {
-            s_f[0].cmask[tid] = leafout ? mask : 0ull;
-            s_f[0].coff[tid] = coff;
-            s_f[0].ga[tid] = baseA + sa.start;
-            s_f[0].gb[tid] = baseB + sb.start;
-        }
-        __syncthreads();
-        if (nout && !(FUSED && leafout)) {
-            uint2* dst = leafout ? A.cands : A.front_out;
-            const uint32_t cap = leafout ? A.cand_cap : A.cap_out;
-            uint32_t o = leafout ? s_cbase + coff : s_obase + off;
-            if (o + nout > cap) or_u32(A.error, leafout ? OI_ERR_CAND_OVERFLOW : OI_ERR_QUEUE_OVERFLOW);
-            u64 m = mask;
-            while (m) {
-                const uint32_t k = (uint32_t)__ffsll((long long)m) - 1u;
-                m &= m - 1ull;
-                if (o < cap) dst[o] = make_uint2(baseA + sa.start + (k >> E), baseB + sb.start + (k & (K - 1)));
-                o++;
-            }
-        }
-        if constexpr (FUSED) {
-            if (C) {
-                if (tid == 0) n_cands += C;
-                fused_narrow<E, FUSE == 2, Tab>(A.tab, s_ibase, s_desc, s_f[0], C, s_wsum, A.hits, A.n_hits,
-                                                A.hits_cap, A.defer, A.defer_count, A.defer_cap, A.error, n_fp64,
-                                                n_adj);
-            }
-        }
-        __syncthreads();
-    }
-    uint32_t nt, na;
-    block_scan(n_tests, s_wsum, nt);
-    block_scan(n_adj, s_wsum, na);
-    if (tid == 0) add_stat(A.stat, nt, na, 0u, FUSED ? n_cands : 0u);
-}
-
 // ---------------------------------------------------------------------------
-// k_bvtt_walk: one or two steps of the walk over a short front, 2^e lanes per
-// front pair (lane x tests child x of the first side against the second side's
-// run) instead of a thread per front pair.
-//
-// A short front is bound by latency, not by work: a k_bvtt_step of E = 3 took
-// 13-16 us on fronts of 100 to 10,000 pairs, most of it a few waves running 30 KB
-// of unrolled code (64 box tests, the output loop) once, cold. Here a wave's code
-// is a few hundred instructions, and the children of the first step stay in LDS,
-// where the workgroup's waves share them for the second: a launch, the front's
-// length, its entries and an output slot are fetched once for two steps.
-//
-// A workgroup takes `per` front pairs at a time: phase 0 loads them (and tests
-// them, on the initial front); then, WALK_MID >> 2 e1 pairs per round, so that
-// their children always fit into LDS, phase 1 expands them by e1 levels and phase
-// 2 their children by e2. Kept pairs of the last phase, and leaf pairs, gather in
-// rings in LDS: the first go to the global front in blocks, one fetch_add each,
-// the others are tested in blocks (FUSE as in k_bvtt_step). Fronts, candidates,
-// counts per level and statistics are those of the same steps one by one.
-// The rings are small (25 KB a workgroup in all) so that workgroups find room
-// beside a refit; with 64 KB lists the same walks took 16 overlapped frames of two
-// 1M-triangle bodies from 1,111 to 1,310 us.
-// Frame and pairs: two bodies of 1,280 triangles 102 -> 68 us, of 81,920 128 -> 91,
-// of 1M 183 -> 159. Of a walk's 11 us on 100 pairs, 1.8 are the launch and the
-// front's length, 3.4 the entries and their boxes, 2.6 each step.
+// Rings in LDS in which a workgroup gathers the pairs it keeps: kept front pairs,
+// which leave for the global front in blocks (one fetch_add and whole cache lines
+// per block), and leaf pairs, which are tested once there is one per thread. A
+// place counts the pairs ever put in; `done` counts those that have left.
 // ---------------------------------------------------------------------------
-#define WALK_T 256
-#define WALK_MID 1024   // first-step children per round
-#define WALK_RING 512   // a ring is emptied from WALK_T pairs on
-#define WALK_COOP 64    // up to this many leaf pairs at a time are tested by 16 lanes each
+#define RING_COOP 64  // up to this many leaf pairs at a time are tested by 16 lanes each
 
-template <class Tab>
-struct WalkArgs {
-    Tab tab;
-    const uint2* front_in;
-    const uint32_t* count_in;  // length of front_in; null: n_in
-    uint32_t n_in;
-    uint32_t cap_in;           // entries front_in can hold
-    uint32_t e1, e2;           // levels of the first and the second step (e2 = 0: one step)
-    uint32_t test_entries;     // test the input pairs themselves (the initial front)
-    uint2* front_out;
-    uint32_t* count_mid;       // two steps: pairs the first step keeps (a count only)
-    uint32_t* count_out;
-    uint32_t cap_out;
-    uint2* cands;
-    uint32_t* cand_count;
-    uint32_t cand_cap;
-    uint32_t* error;
-    oi_detect_stat* stat;
-    uint4* hits;
-    uint32_t* n_hits;
-    uint32_t hits_cap;
-    uint2* defer;
-    uint32_t* defer_count;
-    uint32_t defer_cap;
-    uint32_t implicit_end;
-};
-
-struct WalkLds {
-    uint2 q0[WALK_T];
-    uint2 mid[WALK_MID];
-    uint2 out[WALK_RING];
-    uint2 cand[WALK_RING];
-    float box[WALK_T / 64][64 * 6];  // a wave's second-side boxes
-    uint32_t n0, n_mid;              // entries of q0 and mid
-    uint32_t n_out, n_cand;          // pairs ever put into the rings
+template <uint32_t NOUT, uint32_t NCAND>
+struct RingLds {
+    static constexpr uint32_t OUT = NOUT, CAND = NCAND;  // powers of two
+    uint2 out[NOUT];
+    uint2 cand[NCAND];
     uint32_t base, hbase, dbase, nh, nd;
 };
 
-// orders a wave's LDS accesses (its lanes exchange boxes)
-__device__ __forceinline__ void wave_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // n kept pairs of the ring, from the done-th on, to the global front (every
 // thread calls; a barrier precedes)
-template <class Tab>
-__device__ __forceinline__ void walk_flush(const WalkArgs<Tab>& A, WalkLds& S, uint32_t done, uint32_t n)
+template <class Args, class Ring>
+__device__ __forceinline__ void ring_flush(const Args& A, Ring& S, uint32_t done, uint32_t n)
 {
     if (threadIdx.x == 0) S.base = add_u32(A.count_out, n);
     __syncthreads();
     const uint32_t base = S.base;
     if (threadIdx.x == 0 && base + n > A.cap_out) or_u32(A.error, OI_ERR_QUEUE_OVERFLOW);
-    for (uint32_t i = threadIdx.x; i < n; i += WALK_T)
-        if (base + i < A.cap_out) A.front_out[base + i] = S.out[(done + i) & (WALK_RING - 1u)];
+    for (uint32_t i = threadIdx.x; i < n; i += TB)
+        if (base + i < A.cap_out) A.front_out[base + i] = S.out[(done + i) & (Ring::OUT - 1u)];
     __syncthreads();
 }
 
@@ -925,8 +796,8 @@ __device__ __forceinline__ int sat_lanes(const v3f* P, const v3f* Q)
 // n leaf pairs of the ring, from the done-th on: to the candidate list (FUSE 0),
 // or through the SAT (1) or the FP32 filter (2), one per thread, or 16 lanes per
 // pair where there are few (every thread calls; a barrier precedes)
-template <int FUSE, class Tab>
-__device__ __forceinline__ void walk_leaves(const WalkArgs<Tab>& A, WalkLds& S, const oi_mesh_desc* s_desc,
+template <int FUSE, class Args, class Ring>
+__device__ __forceinline__ void ring_leaves(const Args& A, Ring& S, const oi_mesh_desc* s_desc,
                                             const uint32_t* s_ibase, uint32_t done, uint32_t n, uint32_t& n_adj)
 {
     const uint32_t tid = threadIdx.x;
@@ -935,12 +806,12 @@ __device__ __forceinline__ void walk_leaves(const WalkArgs<Tab>& A, WalkLds& S, 
         __syncthreads();
         const uint32_t base = S.base;
         if (tid == 0 && base + n > A.cand_cap) or_u32(A.error, OI_ERR_CAND_OVERFLOW);
-        for (uint32_t i = tid; i < n; i += WALK_T)
-            if (base + i < A.cand_cap) A.cands[base + i] = S.cand[(done + i) & (WALK_RING - 1u)];
+        for (uint32_t i = tid; i < n; i += TB)
+            if (base + i < A.cand_cap) A.cands[base + i] = S.cand[(done + i) & (Ring::CAND - 1u)];
         __syncthreads();
     } else {
-        const bool coop = n <= WALK_COOP;
-        const uint32_t lg = coop ? 4u : 0u, per = WALK_T >> lg;
+        const bool coop = n <= RING_COOP;
+        const uint32_t lg = coop ? 4u : 0u, per = TB >> lg;
         for (uint32_t c0 = 0; c0 < n; c0 += per) {
             if (tid == 0) S.nh = S.nd = 0;
             __syncthreads();
@@ -949,7 +820,7 @@ __device__ __forceinline__ void walk_leaves(const WalkArgs<Tab>& A, WalkLds& S, 
             uint2 pr = make_uint2(0, 0);
             uint4 h = make_uint4(0, 0, 0, 0);
             if (c < n) {
-                pr = S.cand[(done + c) & (WALK_RING - 1u)];
+                pr = S.cand[(done + c) & (Ring::CAND - 1u)];
                 v3f P[3], Q[3];
                 if (narrow_gather(A.tab, s_ibase, s_desc, pr, (tid & ((1u << lg) - 1u)) == 0u, n_adj, P, Q, h)) {
                     if (coop)
@@ -962,6 +833,7 @@ __device__ __forceinline__ void walk_leaves(const WalkArgs<Tab>& A, WalkLds& S, 
                 if (tid & ((1u << lg) - 1u)) r = SAT_SEPARATED;  // the pair's first lane answers
             }
             const bool hit = r == SAT_HIT, dfr = FUSE == 2 && r == SAT_UNDECIDED;
+            if (hit) h = hit_ids(A.tab, s_desc, h);
             const uint32_t at = hit ? atomicAdd(&S.nh, 1u) : 0u, atd = dfr ? atomicAdd(&S.nd, 1u) : 0u;
             __syncthreads();
             if (tid == 0) {
@@ -983,6 +855,179 @@ __device__ __forceinline__ void walk_leaves(const WalkArgs<Tab>& A, WalkLds& S, 
             }
         }
     }
+}
+
+// FUSE 0: overlapping leaf pairs go to the candidate list; FUSE 1: they are
+// tested with the FP32 SAT by the workgroup that found them; FUSE 2: with the FP32
+// filter, the pairs it leaves undecided going to A.defer for the FP64 pass.
+// Kept pairs gather in LDS (RingLds) and leave in blocks of 1,024 and more. Written
+// from their lanes, 8 bytes here and there, with the output slot fetched before the
+// expansion's loop, they were what the middle steps spent most of their time on. Leaf pairs of all tiles share one ring,
+// so that the SAT runs with full waves, and the next tile's pairs are on their way
+// while one is expanded. Folded cloths of 522K / 8.4M triangles, per frame 300 -> 258
+// / 2,263 -> 1,702 us; 128 instanced scenes, 4 frames, 5,758 -> 5,417 us; 8 scenes of
+// coplanar plates 412 -> 366. The 8.4M cloth's last step (32.4M front pairs, 1,360
+// -> 990 us): 605 us for the child runs, 4.8 TB/s past L2, the rest adjacency
+// and SAT, nearly all of it gathers of faces and vertices. Tiles dealt to XCDs in
+// contiguous ranges: no faster (1,709), short fronts 3-8 % slower.
+// Occupancy: the step waits on its child-run loads, so resident waves matter
+// more than loads in flight per wave. E = 3 holds two runs of 8 boxes and
+// would take 153-161 VGPRs (3 waves per SIMD); capped at 128 (4 waves) it
+// keeps the runs in registers (the fused forms spill 2-5 dwords). E = 2 fits
+// 80 VGPRs (6 waves) unspilled.
+#define STEP_FULL 1024  // kept pairs that leave for the front at a time, at least
+
+template <int E, bool FIRST, int FUSE, class Tab>
+__global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(E == 3 ? 4 : E == 2 ? 6 : 1, 8)))
+k_bvtt_step(StepArgs<Tab> A)
+{
+    constexpr uint32_t K = 1u << E;
+    using M = PairMask<E>;
+    using Ring = RingLds<2 * STEP_FULL, 2 * TB>;
+    __shared__ oi_mesh_desc s_desc[MESH_LDS];
+    __shared__ uint32_t s_ibase[MESH_LDS];
+    __shared__ uint32_t s_wsum[4];
+    __shared__ Ring S;
+    // after an overflow the count keeps growing past the buffer (writes were
+    // dropped and the detect will be re-run): read only what exists
+    uint32_t n_in = A.count_in ? *A.count_in : A.n_in;
+    if (n_in > A.cap_in) n_in = A.cap_in;
+    const uint32_t first = blockIdx.x * TB;
+    if (first >= n_in) return;
+    tab_init(A.tab, s_desc, s_ibase);
+    const uint32_t tid = threadIdx.x, stride = gridDim.x * TB;
+    uint32_t n_tests = 0, n_adj = 0;
+    uint32_t n_out = 0, n_cand = 0, out_done = 0, cand_done = 0;  // uniform
+    // a tile's pairs are loaded while the tile before it is worked on
+    uint2 e_next = first + tid < n_in ? A.front_in[first + tid] : make_uint2(0, 0);
+    for (uint32_t base = first; base < n_in; base += stride) {
+        const uint32_t i = base + tid;
+        bool have = i < n_in;
+        const uint2 e = e_next;
+        if (i + stride < n_in) e_next = A.front_in[i + stride];
+        if (have && (e.x >= A.implicit_end || e.y >= A.implicit_end)) {
+            or_u32(A.error, OI_ERR_CORRUPT);  // never dereference a bad entry
+            have = false;
+        }
+        M m = 0;               // bit (x << E) + y: pair (start_a + x, start_b + y) kept
+        bool leafout = false;  // kept pairs are leaf pairs (candidates)
+        Side sa = {0, 0}, sb = {0, 0};
+        uint32_t baseA = 0, baseB = 0;
+        if (have) entry_expand<E, FIRST, Tab>(A.tab, s_desc, s_ibase, e, m, leafout, sa, sb, baseA, baseB,
+                                              n_tests, n_adj);
+        const uint2 p0 = make_uint2(baseA + sa.start, baseB + sb.start);
+        // one scan for both counts: front pairs in the high half, leaf pairs
+        // in the low half (at most 256 x 64 each, so no carry crosses)
+        uint32_t TC;
+        const uint32_t cnt = mask_count(m);
+        const uint32_t oc = block_scan(leafout ? cnt : (cnt << 16), s_wsum, TC);
+        uint32_t at = leafout ? n_cand + (oc & 0xffffu) : n_out + (oc >> 16);
+        n_out += TC >> 16;
+        n_cand += TC & 0xffffu;
+        for (;;) {
+            // what fits into the rings; while one is full enough it is emptied
+            // and the rest follows
+            uint2* ring = leafout ? S.cand : S.out;
+            const uint32_t wrap = leafout ? Ring::CAND - 1u : Ring::OUT - 1u;
+            const uint32_t lim = leafout ? cand_done + Ring::CAND : out_done + Ring::OUT;
+            for (; m && (int32_t)(lim - at) > 0; m &= m - 1, at++) {
+                const uint32_t k = mask_first(m);
+                ring[at & wrap] = make_uint2(p0.x + (k >> E), p0.y + (k & (K - 1u)));
+            }
+            __syncthreads();
+            const uint32_t no = n_out - out_done, nc = n_cand - cand_done;
+            if (no < STEP_FULL && nc < TB) break;
+            if (no >= STEP_FULL) {
+                const uint32_t take = min(no, Ring::OUT);
+                ring_flush(A, S, out_done, take);
+                out_done += take;
+            }
+            if (nc >= TB) {
+                ring_leaves<FUSE>(A, S, s_desc, s_ibase, cand_done, TB, n_adj);
+                cand_done += TB;
+                __syncthreads();
+            }
+        }
+    }
+    if (n_out != out_done) ring_flush(A, S, out_done, n_out - out_done);
+    if (n_cand != cand_done) ring_leaves<FUSE>(A, S, s_desc, s_ibase, cand_done, n_cand - cand_done, n_adj);
+    __syncthreads();
+    uint32_t nt, na;
+    block_scan(n_tests, s_wsum, nt);
+    block_scan(n_adj, s_wsum, na);
+    if (tid == 0) add_stat(A.stat, nt, na, 0u, FUSE ? n_cand : 0u);
+}
+
+// ---------------------------------------------------------------------------
+// k_bvtt_walk: one or two steps of the walk over a short front, 2^e lanes per
+// front pair (lane x tests child x of the first side against the second side's
+// run) instead of a thread per front pair.
+//
+// A short front is bound by latency, not by work: a k_bvtt_step of E = 3 took
+// 13-16 us on fronts of 100 to 10,000 pairs, most of it a few waves running 30 KB
+// of unrolled code (64 box tests, the output loop) once, cold. Here a wave's code
+// is a few hundred instructions, and the children of the first step stay in LDS,
+// where the workgroup's waves share them for the second: a launch, the front's
+// length, its entries and an output slot are fetched once for two steps.
+//
+// A workgroup takes `per` front pairs at a time: phase 0 loads them (and tests
+// them, on the initial front); then, WALK_MID >> 2 e1 pairs per round, so that
+// their children always fit into LDS, phase 1 expands them by e1 levels and phase
+// 2 their children by e2. Kept pairs of the last phase, and leaf pairs, gather in
+// rings (FUSE as in k_bvtt_step). Fronts, candidates, counts per level and
+// statistics are those of the same steps one by one.
+// The rings are small (25 KB a workgroup in all) so that workgroups find room
+// beside a refit; with 64 KB lists the same walks took 16 overlapped frames of two
+// 1M-triangle bodies from 1,111 to 1,310 us.
+// Frame and pairs: two bodies of 1,280 triangles 102 -> 68 us, of 81,920 128 -> 91,
+// of 1M 183 -> 159. Of a walk's 11 us on 100 pairs, 1.8 are the launch and the
+// front's length, 3.4 the entries and their boxes, 2.6 each step.
+// ---------------------------------------------------------------------------
+#define WALK_T TB
+#define WALK_MID 1024   // first-step children per round
+#define WALK_RING 512   // a ring is emptied from WALK_T pairs on
+
+template <class Tab>
+struct WalkArgs {
+    Tab tab;
+    const uint2* front_in;
+    const uint32_t* count_in;  // length of front_in; null: n_in
+    uint32_t n_in;
+    uint32_t cap_in;           // entries front_in can hold
+    uint32_t e1, e2;           // levels of the first and the second step (e2 = 0: one step)
+    uint32_t test_entries;     // test the input pairs themselves (the initial front)
+    uint2* front_out;
+    uint32_t* count_mid;       // two steps: pairs the first step keeps (a count only)
+    uint32_t* count_out;
+    uint32_t cap_out;
+    uint2* cands;
+    uint32_t* cand_count;
+    uint32_t cand_cap;
+    uint32_t* error;
+    oi_detect_stat* stat;
+    uint4* hits;
+    uint32_t* n_hits;
+    uint32_t hits_cap;
+    uint2* defer;
+    uint32_t* defer_count;
+    uint32_t defer_cap;
+    uint32_t implicit_end;
+};
+
+struct WalkLds : RingLds<WALK_RING, WALK_RING> {
+    uint2 q0[WALK_T];
+    uint2 mid[WALK_MID];
+    float box[WALK_T / 64][64 * 6];  // a wave's second-side boxes
+    uint32_t n0, n_mid;              // entries of q0 and mid
+    uint32_t n_out, n_cand;          // pairs ever put into the rings
+};
+
+// orders a wave's LDS accesses (its lanes exchange boxes)
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // One pass of the workgroup over the n pairs of src from the i0-th on, e levels
@@ -1197,12 +1242,12 @@ __global__ void __launch_bounds__(WALK_T) k_bvtt_walk(WalkArgs<Tab> A)
             if (no < full && nc < full) break;
             if (no >= full) {
                 const uint32_t take = min(no, (uint32_t)WALK_RING);
-                walk_flush(A, S, out_done, take);
+                ring_flush(A, S, out_done, take);
                 out_done += take;
             }
             if (nc >= full) {
                 const uint32_t take = min(nc, (uint32_t)WALK_T);
-                walk_leaves<FUSE>(A, S, s_desc, s_ibase, cand_done, take, n_adj);
+                ring_leaves<FUSE>(A, S, s_desc, s_ibase, cand_done, take, n_adj);
                 cand_done += take;
                 __syncthreads();
             }
@@ -1304,18 +1349,19 @@ __global__ void __launch_bounds__(TB) k_bvtt_local(LocalArgs<Tab> A)
                     or_u32(A.error, OI_ERR_CORRUPT);
                     have = false;
                 }
-                u64 mask = 0;
+                PairMask<E> km = 0;
                 bool leafout = false;
                 Side sa = {0, 0}, sb = {0, 0};
                 uint32_t baseA = 0, baseB = 0;
                 if (have) {
                     if (test)
-                        entry_expand<E, true, Tab>(A.tab, s_desc, s_ibase, e, mask, leafout, sa, sb, baseA, baseB,
+                        entry_expand<E, true, Tab>(A.tab, s_desc, s_ibase, e, km, leafout, sa, sb, baseA, baseB,
                                                    n_tests, n_adj);
                     else
-                        entry_expand<E, false, Tab>(A.tab, s_desc, s_ibase, e, mask, leafout, sa, sb, baseA, baseB,
+                        entry_expand<E, false, Tab>(A.tab, s_desc, s_ibase, e, km, leafout, sa, sb, baseA, baseB,
                                                     n_tests, n_adj);
                 }
+                const u64 mask = km;
                 const uint32_t nout = (uint32_t)__popcll(mask);
                 // one scan for both counts (front pairs high, leaf pairs low)
                 uint32_t TC;
@@ -1413,11 +1459,12 @@ struct NarrowArgs {
 // SAT over the defer list (the precision form's second pass).
 enum { NARROW_FP32 = 0, NARROW_FILTER = 1, NARROW_FP64 = 2 };
 
-// The two triangles of candidate c as the SAT takes them: sorted faces and
-// original ids, then the vertices through the model matrices; inside one
-// mesh P is the face with the smaller original id, across meshes the face of
-// the lower mesh. False (nothing to test) for self-mode pairs that share a
-// vertex, counted in n_adj when count_adj.
+// The two triangles of candidate c as the SAT takes them: sorted faces, then the
+// vertices through the model matrices; inside one mesh P is the face with the
+// smaller original id, across meshes the face of the lower mesh. False (nothing to
+// test) for self-mode pairs that share a vertex, counted in n_adj when count_adj.
+// id: the meshes, and inside one mesh the original face ids; across meshes the
+// leaf positions in their place, for hit_ids (few candidates are hits).
 template <class Tab>
 __device__ __forceinline__ bool narrow_gather(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
                                               uint2 c, bool count_adj, uint32_t& n_adj, v3f* P, v3f* Q, uint4& id)
@@ -1427,13 +1474,14 @@ __device__ __forceinline__ bool narrow_gather(const Tab& T, const uint32_t* s_ib
     const MeshRef rb = tab_ref(T, s_desc, s_ibase, c.y, mb);
     const uint32_t sa = c.x - ra.ibase - ((1u << ra.L) - 1u);
     const uint32_t sb = c.y - rb.ibase - ((1u << rb.L) - 1u);
-    // the original ids are read with the faces, and the vertices before the
-    // ids arrive: two dependent rounds of loads per candidate
     uint32_t fa[3], fb[3];
     oi_ld3(ra.sfaces, sa, fa);
     oi_ld3(rb.sfaces, sb, fb);
-    uint32_t oa = oi_g(ra.perm)[sa], ob = oi_g(rb.perm)[sb];
+    uint32_t oa = sa, ob = sb;
     if (ma == mb) {
+        // (read with the faces; the vertices are read before they arrive)
+        oa = oi_g(ra.perm)[sa];
+        ob = oi_g(rb.perm)[sb];
         bool adj = false;
 #pragma unroll
         for (int i = 0; i < 3; i++)
@@ -1444,37 +1492,38 @@ __device__ __forceinline__ bool narrow_gather(const Tab& T, const uint32_t* s_ib
             return false;
         }
     }
-    // all six vertices, then both model matrices, are loaded before any is
-    // used (one round of loads, not one per vertex)
+    // all six vertices, and both model matrices, are loaded before any is used
+    // (one round of loads, not one per vertex)
     float pa[3][3], pb[3][3];
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         oi_ld3(ra.pos, fa[k], pa[k]);
         oi_ld3(rb.pos, fb[k], pb[k]);
     }
-    // (a mesh without a matrix reads a zero block in its place, unused)
-    const float* sxa = ra.xf ? ra.xf : k_no_xf;
-    const float* sxb = rb.xf ? rb.xf : k_no_xf;
-    float xa[16], xb[16];
+    if (__ballot(ra.xf || rb.xf) == 0ull) {
+        // no mesh of this wave has a matrix
 #pragma unroll
-    for (int k = 0; k < 16; k++) {
-        xa[k] = oi_g(sxa)[k];
-        xb[k] = oi_g(sxb)[k];
-    }
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        float o[3];
-        if (ra.xf) {
-            oi_xform(xa, pa[k][0], pa[k][1], pa[k][2], o);
-            P[k] = v3f{o[0], o[1], o[2]};
-        } else {
+        for (int k = 0; k < 3; k++) {
             P[k] = v3f{pa[k][0], pa[k][1], pa[k][2]};
-        }
-        if (rb.xf) {
-            oi_xform(xb, pb[k][0], pb[k][1], pb[k][2], o);
-            Q[k] = v3f{o[0], o[1], o[2]};
-        } else {
             Q[k] = v3f{pb[k][0], pb[k][1], pb[k][2]};
+        }
+    } else {
+        // (a mesh without a matrix reads a zero block in its place, unused)
+        const float* sxa = ra.xf ? ra.xf : k_no_xf;
+        const float* sxb = rb.xf ? rb.xf : k_no_xf;
+        float xa[16], xb[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+            xa[k] = oi_g(sxa)[k];
+            xb[k] = oi_g(sxb)[k];
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            float o[3];
+            oi_xform(xa, pa[k][0], pa[k][1], pa[k][2], o);
+            P[k] = ra.xf ? v3f{o[0], o[1], o[2]} : v3f{pa[k][0], pa[k][1], pa[k][2]};
+            oi_xform(xb, pb[k][0], pb[k][1], pb[k][2], o);
+            Q[k] = rb.xf ? v3f{o[0], o[1], o[2]} : v3f{pb[k][0], pb[k][1], pb[k][2]};
         }
     }
     if (ma == mb && oa > ob) {
@@ -1494,6 +1543,17 @@ __device__ __forceinline__ bool narrow_gather(const Tab& T, const uint32_t* s_ib
     return true;
 }
 
+// a hit's id with the original face ids
+template <class Tab>
+__device__ __forceinline__ uint4 hit_ids(const Tab& T, const oi_mesh_desc* s_desc, uint4 id)
+{
+    if (id.x != id.y) {
+        id.z = oi_g(mesh_perm(T, s_desc, id.x))[id.z];
+        id.w = oi_g(mesh_perm(T, s_desc, id.y))[id.w];
+    }
+    return id;
+}
+
 // FP32 narrow phase of one candidate (the fused BVTT steps use it)
 template <bool FP64, class Tab>
 __device__ __forceinline__ void narrow_one(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
@@ -1506,7 +1566,7 @@ __device__ __forceinline__ void narrow_one(const Tab& T, const uint32_t* s_ibase
     if (!narrow_gather(T, s_ibase, s_desc, c, true, n_adj, P, Q, id)) return;
     if (sat_f32(P, Q)) {
         hit = true;
-        out = id;
+        out = hit_ids(T, s_desc, id);
     }
 }
 
@@ -1524,7 +1584,7 @@ __device__ __forceinline__ void narrow_one_filter(const Tab& T, const uint32_t* 
     const int r = sat_filter(P, Q);
     hit = r == SAT_HIT;
     defer = r == SAT_UNDECIDED;
-    out = id;
+    if (hit) out = hit_ids(T, s_desc, id);
 }
 
 template <int MODE, class Tab>
@@ -1569,6 +1629,7 @@ __global__ void __launch_bounds__(TB) k_narrow(NarrowArgs<Tab> A)
                     hit = sat_f64_counted(P, Q, n_fp64);
                 }
             }
+            if (hit) out = hit_ids(A.tab, s_desc, out);
             if (defer) out = make_uint4(c.x, c.y, 0, 0);
         }
         // one scan for both counts: hits in the high half, deferred pairs in

@@ -761,6 +761,32 @@ def test_detect_walk_dense_and_sparse(api, ctx, orc, expand, mode):
         ctx.set_tuning(narrow_separate=0)
 
 
+@pytest.mark.parametrize("mode", ["fp32", "separate", "fp64"])
+@pytest.mark.parametrize("expand", [1, 2, 3])
+def test_detect_steps_dense_and_sparse(api, ctx, orc, expand, mode):
+    """Long fronts (k_bvtt_step from an entry level of 2^8 nodes a tree and
+    deeper): a sphere against itself, where the kept pairs of one pass overflow the
+    ring in LDS several times over, a cloth in self mode with many leaf pairs a
+    pass, trees of unequal depth, an entry level just above the leaves (a first
+    step of few levels), and a front that leaves most of the last tile empty; with
+    leaf pairs tested in the step, in one k_narrow launch, and through the filter:
+    the oracle's pairs."""
+    say(f"detect steps expand={expand} {mode}")
+    fp64 = mode == "fp64"
+    a, small = M.icosphere(5, 1.0, 0.0, 0), M.box(9, 0.9, 0.0, 1)
+    cl = M.cloth(64, amplitude=0.2, wavelength=0.2, seed=5)
+    ctx.set_tuning(narrow_separate=1 if mode == "separate" else 0)
+    try:
+        for meshes, entry, self_collide in (([a, a], 8, False), ([a, a], 11, False), ([cl], 9, True),
+                                            ([a, small, cl], 8, True)):
+            p, st, trees = gpu_pairs(api, ctx, meshes, entry, expand, self_collide=self_collide, fp64=fp64)
+            want = orc.detect([orc.Tree(x, f, order=t.perm()) for (x, f), t in zip(meshes, trees)],
+                              self_collide=self_collide, fp64=fp64)
+            assert np.array_equal(p, want), (len(meshes), entry)
+    finally:
+        ctx.set_tuning(narrow_separate=0)
+
+
 @pytest.mark.parametrize("entry", [0, 1, 3, 6, 30])
 @pytest.mark.parametrize("expand", [1, 2, 3, 5])
 @pytest.mark.parametrize("mode", [(0, 0), (64, 0), (7, 0), (64, 2), (16, 1),
