@@ -71,7 +71,7 @@ struct oibvh_batch {
     uint32_t morton_bits = 30;
     uint32_t* sort_scratch = nullptr;  // histograms | tile counters | lookback0 | lookback1
     uint32_t* mesh_hist = nullptr;     // digit histograms of the mesh ids, 256 per pass
-    uint32_t tiles = 0, mesh_passes = 0;
+    uint32_t sort_rows = 0, mesh_passes = 0;
     uint2* w_box = nullptr;
     uint32_t n_box = 0;
     uint2* w_morton = nullptr;
@@ -390,8 +390,9 @@ static oibvh_status commit(oibvh_batch* b)
     HIPCHK(c, dalloc(&b->vals_tmp, F));
     b->mesh_passes = n <= 1 ? 0 : n <= 256 ? 1 : n <= 65536 ? 2 : 3;
     if (b->mesh_passes) HIPCHK(c, dalloc(&b->fmesh, F));
-    b->tiles = (uint32_t)((F + oi_sort_tile() - 1) / oi_sort_tile());
-    HIPCHK(c, dalloc(&b->sort_scratch, OI_SORT_HEAD + 512ull * b->tiles));
+    const uint32_t Fn = (uint32_t)F;
+    b->sort_rows = (uint32_t)oi_sort_rows(1, oi_sort_tiles(1, &Fn));
+    HIPCHK(c, dalloc(&b->sort_scratch, OI_SORT_HEAD + 512ull * b->sort_rows));
     {
         std::vector<uint32_t> mh(768, 0u);
         for (uint32_t i = 0; i < n; i++)
@@ -404,7 +405,7 @@ static oibvh_status commit(oibvh_batch* b)
     for (uint32_t i = 0; i < n; i++) {
         const oibvh_batch::Mesh& m = b->meshes[i];
         for (uint32_t k = 0; k < m.nparts; k++) wb.push_back(make_uint2(i, k));
-        const uint32_t mc = (m.F + oi_morton_chunk() - 1) / oi_morton_chunk();
+        const uint32_t mc = (m.F + oi_morton_chunk(F) - 1) / oi_morton_chunk(F);
         for (uint32_t k = 0; k < mc; k++) wm.push_back(make_uint2(i, k));
     }
     oibvh_status r;
@@ -686,11 +687,11 @@ extern "C" oibvh_status oibvh_batch_build(oibvh_batch* b)
     if (m63 && !b->keys_hi) HIPCHK(c, dalloc(&b->keys_hi, F));
     uint32_t* ghist = b->sort_scratch;
     uint32_t* tctr = b->sort_scratch + OI_SORT_HIST;
-    uint32_t* lb[2] = {b->sort_scratch + OI_SORT_HEAD, b->sort_scratch + OI_SORT_HEAD + 256ull * b->tiles};
+    uint32_t* lb[2] = {b->sort_scratch + OI_SORT_HEAD, b->sort_scratch + OI_SORT_HEAD + 256ull * b->sort_rows};
     HIPCHK(c, oi_launch_mesh_box(s, sl.d_bdesc, b->w_box, nullptr, b->n_box, b->partials, b->sort_scratch,
-                                 OI_SORT_HEAD + 256u * b->tiles));
-    HIPCHK(c, oi_launch_morton(s, sl.d_bdesc, b->w_morton, nullptr, b->n_morton, b->partials, b->keys,
-                               m63 ? b->keys_hi : nullptr, ghist, b->fmesh));
+                                 OI_SORT_HEAD + 256u * b->sort_rows));
+    HIPCHK(c, oi_launch_morton(s, sl.d_bdesc, b->w_morton, nullptr, b->n_morton, oi_morton_chunk(F), b->partials,
+                               b->keys, m63 ? b->keys_hi : nullptr, ghist, OI_HIST_REPS, b->fmesh));
     // Morton passes (four over the low word with the keys moving along; for
     // 63-bit keys four more over the high word, looked up by face id), then
     // the mesh-id passes; lookback buffers alternate
@@ -708,8 +709,9 @@ extern "C" oibvh_status oibvh_batch_build(oibvh_batch* b)
         const uint32_t shift = morton ? 8 * (p & 3) : 8 * (p - mpasses);
         uint32_t* ko = (lo && p < 3) ? kout : nullptr;
         const uint32_t* kov = lo ? nullptr : (morton ? b->keys_hi : b->fmesh);
-        HIPCHK(c, oi_launch_sort_pass(s, lo ? kin : nullptr, vin, ko, vout, F, shift, hist, lb[p & 1],
-                                      last ? nullptr : lb[(p + 1) & 1], tctr + p, kov));
+        HIPCHK(c, oi_launch_sort_pass(s, lo ? kin : nullptr, vin, ko, vout, F, shift, hist,
+                                      morton ? OI_HIST_REPS : 1u, lb[p & 1], last ? nullptr : lb[(p + 1) & 1], tctr + p,
+                                      kov));
         std::swap(kin, kout);
         vin = vout;
         vout = (vout == b->vals_tmp) ? b->vals : b->vals_tmp;

@@ -33,8 +33,7 @@
 #include "oibvh_common.h"
 
 #define OI_BLOCK 256
-#define OI_MORTON_CHUNK 2048
-#define OI_HIST_WORDS 3072  // k_morton's digit histograms: 8 x 256 or 3 x 1024 bins
+#define OI_MORTON_T 1024    // threads of k_morton
 
 __device__ __forceinline__ float gmin(float a, float b) { return (b < a) ? b : a; }
 __device__ __forceinline__ float gmax(float a, float b) { return (a < b) ? b : a; }
@@ -146,13 +145,66 @@ struct Xf {
 __device__ __forceinline__ float lo_c(float l, float r) { return (l < r) ? l : r; }
 __device__ __forceinline__ float hi_c(float l, float r) { return (r < l) ? l : r; }
 
+// A wave's lo_c / hi_c in lane order (lane 63 holds it), neighbours first, then
+// pairs of pairs, through the data-parallel primitives of oi_wave_scan_incl; a
+// lane without a left neighbour folds the identity.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_left(float identity, float x)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp((int)__float_as_uint(identity),
+                                                                 (int)__float_as_uint(x), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ float wave_lo(float x)
+{
+    const float id = __builtin_inff();
+    x = lo_c(dpp_left<0x111, 0xf>(id, x), x);
+    x = lo_c(dpp_left<0x112, 0xf>(id, x), x);
+    x = lo_c(dpp_left<0x114, 0xf>(id, x), x);
+    x = lo_c(dpp_left<0x118, 0xf>(id, x), x);
+    x = lo_c(dpp_left<0x142, 0xa>(id, x), x);
+    return lo_c(dpp_left<0x143, 0xc>(id, x), x);
+}
+__device__ __forceinline__ float wave_hi(float x)
+{
+    const float id = -__builtin_inff();
+    x = hi_c(dpp_left<0x111, 0xf>(id, x), x);
+    x = hi_c(dpp_left<0x112, 0xf>(id, x), x);
+    x = hi_c(dpp_left<0x114, 0xf>(id, x), x);
+    x = hi_c(dpp_left<0x118, 0xf>(id, x), x);
+    x = hi_c(dpp_left<0x142, 0xa>(id, x), x);
+    return hi_c(dpp_left<0x143, 0xc>(id, x), x);
+}
+
+// The ordered fold of OI_BLOCK threads' boxes (threads from OI_BLOCK on have
+// none); every thread gets the result.
+__device__ __forceinline__ void fold_box(float (*s_v)[6], float* mn, float* mx)
+{
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    if (wave < OI_BLOCK / 64) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const float lo = wave_lo(mn[k]), hi = wave_hi(mx[k]);
+            if (lane == 63u) {
+                s_v[wave][k] = lo;
+                s_v[wave][3 + k] = hi;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        mn[k] = lo_c(lo_c(s_v[0][k], s_v[1][k]), lo_c(s_v[2][k], s_v[3][k]));
+        mx[k] = hi_c(hi_c(s_v[0][3 + k], s_v[1][3 + k]), hi_c(s_v[2][3 + k], s_v[3][3 + k]));
+    }
+}
+
 __global__ void __launch_bounds__(OI_BLOCK)
 k_mesh_box(BuildTab T, float* __restrict__ partials, uint32_t* __restrict__ clear_u32, uint32_t clear_n)
 {
     const uint32_t tid = threadIdx.x;
     for (uint32_t i = blockIdx.x * OI_BLOCK + tid; i < clear_n; i += gridDim.x * OI_BLOCK) clear_u32[i] = 0u;
 
-    __shared__ float s_v[6][OI_BLOCK];
+    __shared__ float s_v[OI_BLOCK / 64][6];
     const uint2 it = T.item();
     const oi_build_desc D = T.mesh(it.x);
     Xf X;
@@ -181,55 +233,15 @@ k_mesh_box(BuildTab T, float* __restrict__ partials, uint32_t* __restrict__ clea
             }
         }
     }
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        s_v[k][tid] = mn[k];
-        s_v[3 + k][tid] = mx[k];
-    }
-    __syncthreads();
-    for (uint32_t s = 1; s < OI_BLOCK; s <<= 1) {
-        if ((tid & (2u * s - 1u)) == 0) {
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                s_v[k][tid] = lo_c(s_v[k][tid], s_v[k][tid + s]);
-                s_v[3 + k][tid] = hi_c(s_v[3 + k][tid], s_v[3 + k][tid + s]);
-            }
-        }
-        __syncthreads();
-    }
+    fold_box(s_v, mn, mx);
     float* P = partials ? partials + 6u * D.pbase : D.box + 6;
-    if (tid < 6) oi_gw(P)[6u * it.y + tid] = s_v[tid][0];
-}
-
-// Fold the per-block partial boxes (at most OI_BLOCK of them) in block order and
-// then with the default box (+-FLT_MAX) in front; every thread gets the result.
-__device__ void fold_partials(const float* __restrict__ partials, uint32_t nparts, float (*s_v)[OI_BLOCK],
-                              float* bmn, float* bmx)
-{
-    const uint32_t tid = threadIdx.x;
-    const float INF = __builtin_inff();
+    if (tid < 6) {
+        float r = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-        s_v[k][tid] = (tid < nparts) ? partials[6u * tid + k] : INF;
-        s_v[3 + k][tid] = (tid < nparts) ? partials[6u * tid + 3 + k] : -INF;
+        for (int k = 0; k < 6; k++)
+            if ((int)tid == k) r = k < 3 ? mn[k] : mx[k - 3];
+        oi_gw(P)[6u * it.y + tid] = r;
     }
-    __syncthreads();
-    for (uint32_t s = 1; s < OI_BLOCK; s <<= 1) {
-        if ((tid & (2u * s - 1u)) == 0) {
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                s_v[k][tid] = lo_c(s_v[k][tid], s_v[k][tid + s]);
-                s_v[3 + k][tid] = hi_c(s_v[3 + k][tid], s_v[3 + k][tid + s]);
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        bmn[k] = lo_c(__FLT_MAX__, s_v[k][0]);
-        bmx[k] = hi_c(-__FLT_MAX__, s_v[3 + k][0]);
-    }
-    __syncthreads();
 }
 
 // ---------------------------------------------------------------------------
@@ -254,8 +266,7 @@ __device__ __forceinline__ uint32_t quantise10(float p)
     return (q != q) ? 0u : (uint32_t)q;
 }
 
-// Work item (m, c): faces [c * OI_MORTON_CHUNK, (c + 1) * OI_MORTON_CHUNK) of
-// mesh m. Keys go to keys[fbase + face]; the 8-bit digit histograms of the
+// Work item (m, c): faces [c * chunk, (c + 1) * chunk) of mesh m, chunk = 1024 NJ. Keys go to keys[fbase + face]; the 8-bit digit histograms of the
 // keys accumulate in ghist + m * hstride (hstride 0: one set for all keys of
 // the launch); fmesh (if not null) receives the mesh id of each face
 // (fmesh[fbase + face] = m). The mesh-box partials are read from partials +
@@ -288,8 +299,8 @@ __device__ __forceinline__ uint32_t quantise21(float p)
 __device__ __forceinline__ void hist_add(uint32_t* h, uint32_t bin, bool active)
 {
     const uint32_t lane = threadIdx.x & 63u;
-    // the bin of the lane below (lane 0 reads its own; it is always a head)
-    const uint32_t below = (uint32_t)__shfl_up((int)bin, 1u, 64);
+    // the bin of the lane below (wave_shr:1; lane 0 reads its own and is always a head)
+    const uint32_t below = (uint32_t)__builtin_amdgcn_update_dpp((int)bin, (int)bin, 0x138, 0xf, 0xf, false);
     const unsigned long long act = __ballot(active);
     const bool below_active = lane > 0 && ((act >> (lane - 1u)) & 1ull);
     const bool head = active && (!below_active || below != bin);
@@ -306,13 +317,19 @@ __device__ __forceinline__ void hist_add(uint32_t* h, uint32_t bin, bool active)
 // keys_hi == null: 30-bit keys and the histograms of 4 8-bit digits (hbits 8)
 // or of 3 10-bit digits (hbits 10); else 63-bit keys split into keys (low
 // word) and keys_hi (high word) and 8 8-bit digit histograms. Digit d's
-// histogram is ghist[d << hbits .. (d + 1) << hbits).
-__global__ void __launch_bounds__(OI_BLOCK)
+// histogram is ghist[d << hbits .. (d + 1) << hbits), in `hreps` copies OI_HIST_WORDS
+// apart (a workgroup adds to copy blockIdx.x mod hreps; a reader sums them).
+// Bound by its chain of waits (faces, vertices, box, LDS histograms, additions to the
+// shared ones): with 256 threads of 8 faces each, the box folded before the first
+// load and one shared histogram, 13K faces took 14 us and 1M 24; 16 waves of 1 to 4
+// faces a lane take 5.8 and 13.
+template <int NJ>
+__global__ void __launch_bounds__(OI_MORTON_T)
 k_morton(BuildTab T, const float* __restrict__ partials, uint32_t* __restrict__ keys, uint32_t* __restrict__ keys_hi,
-         uint32_t* __restrict__ ghist, uint32_t hstride, uint32_t* __restrict__ fmesh, uint32_t hbits)
+         uint32_t* __restrict__ ghist, uint32_t hstride, uint32_t hreps, uint32_t* __restrict__ fmesh, uint32_t hbits)
 {
     __shared__ uint32_t s_h[OI_HIST_WORDS];
-    __shared__ float s_v[6][OI_BLOCK];
+    __shared__ float s_v[OI_BLOCK / 64][6];
     const uint32_t tid = threadIdx.x;
     const uint2 it = T.item();
     const oi_build_desc D = T.mesh(it.x);
@@ -320,27 +337,27 @@ k_morton(BuildTab T, const float* __restrict__ partials, uint32_t* __restrict__ 
     X.load(D.xf);
     const bool h10 = hbits == 10u;
     const uint32_t nd = keys_hi ? 8u : h10 ? 3u : 4u;
-    for (uint32_t i = tid; i < OI_HIST_WORDS; i += OI_BLOCK) s_h[i] = 0u;
-    float bmn[3], bmx[3];
-    fold_partials(partials ? partials + 6u * D.pbase : D.box + 6, D.nparts, s_v, bmn, bmx);
-    ghist += it.x * hstride;
-    if (it.y == 0 && tid < 3) {
-        oi_gw(D.box)[tid] = bmn[tid];
-        oi_gw(D.box)[3 + tid] = bmx[tid];
-    }
-    const uint32_t f0 = it.y * OI_MORTON_CHUNK;
-    const uint32_t f1 = min(D.F, f0 + OI_MORTON_CHUNK);  // f0 < f1: a work item holds a face
-    // a thread's faces i = f0 + tid + 256 j: every face load is issued, then
-    // every vertex load, then the keys are formed (two rounds of memory
-    // latency per thread instead of two per face); faces past f1 load face f0
-    // and are dropped
-    constexpr int NJ = OI_MORTON_CHUNK / OI_BLOCK;
+    const uint32_t f0 = it.y * (OI_MORTON_T * NJ);
+    const uint32_t f1 = min(D.F, f0 + OI_MORTON_T * NJ);  // f0 < f1: a work item holds a face
+    // a thread's faces i = f0 + tid + 1024 j: every face load is issued, then
+    // every vertex load, and while these are on their way the mesh's box is
+    // folded; then the keys are formed. Faces past f1 load face f0 and are dropped
     uint32_t fv[NJ][3];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
-        const uint32_t i = f0 + tid + (uint32_t)j * OI_BLOCK;
+        const uint32_t i = f0 + tid + (uint32_t)j * OI_MORTON_T;
         oi_ld3(D.faces, i < f1 ? i : f0, fv[j]);
     }
+    // the mesh's partial boxes (at most OI_BLOCK of them), folded in order and
+    // then with the default box (+-FLT_MAX) in front
+    const float* part = partials ? partials + 6u * D.pbase : D.box + 6;
+    float bmn[3], bmx[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        bmn[k] = (tid < D.nparts) ? oi_g(part)[6u * tid + k] : __builtin_inff();
+        bmx[k] = (tid < D.nparts) ? oi_g(part)[6u * tid + 3 + k] : -__builtin_inff();
+    }
+    for (uint32_t i = tid; i < OI_HIST_WORDS; i += OI_MORTON_T) s_h[i] = 0u;
     float p[NJ][9];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
@@ -348,9 +365,23 @@ k_morton(BuildTab T, const float* __restrict__ partials, uint32_t* __restrict__ 
         oi_ld3(D.pos, fv[j][1], &p[j][3]);
         oi_ld3(D.pos, fv[j][2], &p[j][6]);
     }
+    fold_box(s_v, bmn, bmx);  // (its barrier also orders the cleared histograms)
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        bmn[k] = lo_c(__FLT_MAX__, bmn[k]);
+        bmx[k] = hi_c(-__FLT_MAX__, bmx[k]);
+    }
+    ghist += it.x * hstride + (blockIdx.x % hreps) * OI_HIST_WORDS;
+    if (it.y == 0 && tid == 0) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            oi_gw(D.box)[k] = bmn[k];
+            oi_gw(D.box)[3 + k] = bmx[k];
+        }
+    }
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
-        const uint32_t i = f0 + tid + (uint32_t)j * OI_BLOCK;
+        const uint32_t i = f0 + tid + (uint32_t)j * OI_MORTON_T;
         const bool live = i < f1;
         float a[3], b[3], c[3];
         X.apply(&p[j][0], a);
@@ -382,8 +413,12 @@ k_morton(BuildTab T, const float* __restrict__ partials, uint32_t* __restrict__ 
         }
         // every lane of the wave takes part (ballots), dead lanes add nothing
         if (h10) {
-#pragma unroll
-            for (int d = 0; d < 3; d++) hist_add(s_h + 1024 * d, (key >> (10 * d)) & 0x3ffu, live);
+            // (the low digits of neighbours mostly differ: no runs to join)
+            if (live) {
+                atomicAdd(&s_h[key & 0x3ffu], 1u);
+                atomicAdd(&s_h[1024u + ((key >> 10) & 0x3ffu)], 1u);
+            }
+            hist_add(s_h + 2048, key >> 20, live);
         } else {
 #pragma unroll
             for (int d = 0; d < 4; d++) hist_add(s_h + 256 * d, (key >> (8 * d)) & 0xffu, live);
@@ -395,42 +430,49 @@ k_morton(BuildTab T, const float* __restrict__ partials, uint32_t* __restrict__ 
     }
     __syncthreads();
     const uint32_t words = nd << hbits;
-    for (uint32_t i = tid; i < words; i += OI_BLOCK) {
+    for (uint32_t i = tid; i < words; i += OI_MORTON_T) {
         const uint32_t c = s_h[i];
         if (c) atomicAdd(&ghist[i], c);
     }
 }
 
 // ---------------------------------------------------------------------------
-// k_sort_pass<DB>: one stable LSD pass over a DB-bit digit (8 or 10),
-// onesweep style, over up to
-// OI_SORT_SEGS independent segments of the concatenated key arrays (one per
-// tree when several trees are built in one launch).
-// A tile is 16 waves x 8 rounds x 64 lanes = 8192 keys of one segment in
-// input order (wave w owns keys [512w, 512w + 512) of the tile, round j lane l
-// holds key 512w + 64j + l): fewer, larger tiles than one wave per SIMD would
-// give shorten the look-back chains. Keys are ranked per wave with 8 ballots
-// per round (DB ballots; stable: earlier rounds and lower lanes come first), staged
+// k_sort_pass<DB, ITEMS>: one stable LSD pass over a DB-bit digit (8 or 10),
+// onesweep style, over up to OI_SORT_SEGS independent segments of the
+// concatenated key arrays (one per tree when several trees are built in one launch).
+// A tile is 16 waves x ITEMS rounds x 64 lanes (1,024 to 8,192 keys) of one segment
+// in input order (wave w owns keys [64 ITEMS w, 64 ITEMS (w + 1)) of the tile,
+// round j lane l holds the 64j + l-th of them). Keys are ranked per wave with DB
+// ballots per round (stable: earlier rounds and lower lanes come first), staged
 // through LDS in tile-local sorted order and written out in runs. Segment s
 // owns the workgroups and tile ids [tile0[s], tile0[s + 1]); a workgroup takes
 // its tile from its segment's atomic counter (tile_counter[s]), so every tile
 // a look-back waits on is already running, and the look-back ends at the
 // segment's own first tile.
 // Look-back status word: bits 31:30 = 1 aggregate / 2 inclusive prefix,
-// bits 29:0 = count. A digit that no key of the segment has (its histogram
+// bits 29:0 = count. A tile's word counts from the start of its group of LB_GROUP
+// tiles; the group's last tile publishes the group's word (row tiles + group, from
+// the start of the segment), so that a tile reads the words of its group before it,
+// and then group words. A digit that no key of the segment has (its histogram
 // entry is 0) is neither published nor looked back on. Values default to the
 // key's index in the concatenated arrays. With key_of_val the key of a value v
 // is key_of_val[v] (a batch's mesh-id passes: a stable partition of the
 // Morton-sorted faces of all meshes back into their meshes).
+// A pass is a chain of waits: of 25 us on 1M keys (123 tiles of 8,192, one window of
+// look-back after the other over all tiles) the ranking took 5, the look-back 9, the
+// keys' and counts' loads 3.5. Now 19 (245 tiles of 4,096), and 7.9 instead of 14 on
+// 13K keys (13 tiles, before 2). The statuses cross XCDs and their traffic counts: with
+// 16 instead of 8 per round trip a build of 1M triangles took 111 instead of 105 us,
+// and with groups of 16 and 8 tiles 99.
 // ---------------------------------------------------------------------------
 #define RS_WAVES 16
 #define RS_THREADS (64 * RS_WAVES)
-#define RS_ITEMS 8
-#define RS_TILE (RS_THREADS * RS_ITEMS)
+#define RS_ITEMS_MAX 8
 #define LB_AGG (1u << 30)
 #define LB_PRE (2u << 30)
 #define LB_CNT 0x3fffffffu
 #define LB_WIN 8  // look-back statuses loaded per round trip
+#define LB_GROUP OI_SORT_GROUP  // tiles of a look-back group
 #define OI_SORT_SEGS 4
 
 struct SortSegs {
@@ -441,42 +483,71 @@ struct SortSegs {
     uint32_t n[OI_SORT_SEGS];           // its keys
 };
 
-// block-wide exclusive scan over NW waves (one uint32 per thread)
-template <int NW>
-__device__ __forceinline__ uint32_t block_excl_scan_w(uint32_t v, uint32_t* s_wsum, uint32_t& total)
+// exclusive prefixes over the workgroup of two counts per thread
+__device__ __forceinline__ uint2 block_excl_scan2(uint2 v, uint2* s_wsum)
 {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t x = oi_wave_scan_incl(v);
+    const uint2 x = make_uint2(oi_wave_scan_incl(v.x), oi_wave_scan_incl(v.y));
     if (lane == 63) s_wsum[wave] = x;
     __syncthreads();
-    uint32_t before = 0, tot = 0;
+    uint2 before = make_uint2(x.x - v.x, x.y - v.y);
 #pragma unroll
-    for (int w = 0; w < NW; w++) {
-        const uint32_t t = s_wsum[w];
-        before += (w < (int)wave) ? t : 0u;
-        tot += t;
+    for (int w = 0; w < RS_WAVES; w++) {
+        const uint2 t = s_wsum[w];
+        before.x += (w < (int)wave) ? t.x : 0u;
+        before.y += (w < (int)wave) ? t.y : 0u;
     }
-    total = tot;
-    __syncthreads();
-    return before + x - v;
+    return before;
 }
 
+// Sum of digit `d` over the `n` entries (tiles of a group, or groups) before entry
+// `at`. The statuses of LB_WIN entries at - 1, at - 2, ... are loaded in one round trip
+// (the loads cross XCDs) and consumed in order, summing counts until an inclusive
+// prefix or the n-th; an entry not yet published ends the window, which is loaded
+// again from there.
 template <int DB>
+__device__ __forceinline__ uint32_t look_back(const uint32_t* lookback, uint32_t at, uint32_t n, uint32_t d)
+{
+    uint32_t sum = 0;
+    while (n) {
+        uint32_t st[LB_WIN];
+#pragma unroll
+        for (uint32_t w = 0; w < LB_WIN; w++)
+            st[w] = w < n ? ld_acq_relaxed(lookback + ((at - 1u - w) << DB) + d) : 0u;
+        uint32_t used = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < LB_WIN; w++) {
+            if (used != w || w >= n) continue;
+            const uint32_t fl = st[w] & ~LB_CNT;
+            if (fl == 0u) continue;
+            sum += st[w] & LB_CNT;
+            used = w + 1u;
+            if (fl == LB_PRE) n = w + 1u;  // none before it is wanted
+        }
+        at -= used;
+        n -= used;
+        if (n && used != LB_WIN) __builtin_amdgcn_s_sleep(1);
+    }
+    return sum;
+}
+
+template <int DB, int ITEMS>
 __global__ void __launch_bounds__(RS_THREADS)
 k_sort_pass(const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
             uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, SortSegs S, uint32_t shift,
-            const uint32_t* __restrict__ ghist, uint32_t* lookback, uint32_t* lookback_next,
+            const uint32_t* __restrict__ ghist, uint32_t hreps, uint32_t* lookback, uint32_t* lookback_next,
             uint32_t* tile_counter, const uint32_t* __restrict__ key_of_val)
 {
     constexpr uint32_t NB = 1u << DB;  // bins; at most RS_THREADS
+    constexpr uint32_t TILE = RS_THREADS * ITEMS;
     static_assert(NB <= RS_THREADS, "one digit per thread");
     __shared__ uint32_t s_tile;
     __shared__ uint32_t s_whist[RS_WAVES][NB];
     __shared__ uint32_t s_lstart[NB];
     __shared__ uint32_t s_gbase[NB];
-    __shared__ uint32_t s_wsum[RS_WAVES];
-    __shared__ uint32_t s_keys[RS_TILE];
-    __shared__ uint32_t s_vals[RS_TILE];
+    __shared__ uint2 s_wsum[RS_WAVES];
+    __shared__ uint32_t s_keys[TILE];
+    __shared__ uint32_t s_vals[TILE];
 
     // threads tid < NB also own digit tid
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -495,42 +566,58 @@ k_sort_pass(const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ v
     }
     if (tid == 0)
         s_tile = __hip_atomic_fetch_add(tile_counter + seg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // the histogram entry is loaded while the tile id is in flight
-    const uint32_t hcnt = dig ? ghist[seg * S.hstride + tid] : 0u;
     for (uint32_t i = tid; i < RS_WAVES * NB; i += RS_THREADS) (&s_whist[0][0])[i] = 0u;
     __syncthreads();
     const uint32_t tile = s_tile;
     const uint32_t gt = seg0 + tile;  // tile id over all segments
-    const uint32_t base = tile * RS_TILE;
-    if (lookback_next && dig) lookback_next[gt * NB + tid] = 0u;
+    const uint32_t base = tile * TILE;
 
-    // exclusive prefix of the segment's digit histogram
-    uint32_t gtot;
-    const uint32_t gexcl = block_excl_scan_w<RS_WAVES>(hcnt, s_wsum, gtot);
-
-    uint32_t k[RS_ITEMS], v[RS_ITEMS], rk[RS_ITEMS];
-    const uint32_t wbase = base + wave * (64u * RS_ITEMS);
+    uint32_t k[ITEMS], v[ITEMS], rk[ITEMS];
+    const uint32_t wbase = base + wave * (64u * ITEMS);
 #pragma unroll
-    for (int j = 0; j < RS_ITEMS; j++) {
+    for (int j = 0; j < ITEMS; j++) {
         const uint32_t idx = wbase + 64u * j + lane;
         const bool ok = idx < n;
         const uint32_t gi = sbase + idx;
         v[j] = ok ? (vals_in ? vals_in[gi] : gi) : 0u;
         k[j] = ok ? (key_of_val ? key_of_val[v[j]] : keys_in[gi]) : 0u;
     }
+    // (the digit's count over the segment is on its way with the keys)
+    uint32_t hcnt = 0;
+    if (dig) {
+        const uint32_t* h = ghist + seg * S.hstride + tid;
+        if (hreps == OI_HIST_REPS) {
+            uint32_t c[OI_HIST_REPS];
+#pragma unroll
+            for (uint32_t r = 0; r < OI_HIST_REPS; r++) c[r] = h[r * OI_HIST_WORDS];
+#pragma unroll
+            for (uint32_t r = 0; r < OI_HIST_REPS; r++) hcnt += c[r];
+        } else {
+            hcnt = h[0];
+        }
+        if (lookback_next) {
+            lookback_next[gt * NB + tid] = 0u;
+            if (tile % LB_GROUP == 0u)
+                lookback_next[(S.tile0[S.ns] + seg0 / LB_GROUP + seg + tile / LB_GROUP) * NB + tid] = 0u;
+        }
+    }
     const unsigned long long lt = (1ull << lane) - 1ull;
 #pragma unroll
-    for (int j = 0; j < RS_ITEMS; j++) {
+    for (int j = 0; j < ITEMS; j++) {
         const uint32_t idx = wbase + 64u * j + lane;
         const bool ok = idx < n;
         const uint32_t d = (k[j] >> shift) & (NB - 1u);
-        unsigned long long peers = __ballot(ok);
+        const unsigned long long live = __ballot(ok);
+        uint32_t p0 = (uint32_t)live, p1 = (uint32_t)(live >> 32);
 #pragma unroll
         for (int b = 0; b < DB; b++) {
-            const bool bit = (d >> b) & 1u;
-            const unsigned long long m = __ballot(bit);
-            peers &= bit ? m : ~m;
+            // lanes whose bit b equals this lane's
+            const uint32_t bit = (uint32_t)((int32_t)(d << (31 - b)) >> 31);
+            const unsigned long long m = __ballot(bit != 0u);
+            p0 &= ~((uint32_t)m ^ bit);
+            p1 &= ~((uint32_t)(m >> 32) ^ bit);
         }
+        const unsigned long long peers = ((unsigned long long)p1 << 32) | p0;
         const uint32_t prev = s_whist[wave][d];
         const uint32_t cnt = (uint32_t)__popcll(peers);
         rk[j] = prev + (uint32_t)__popcll(peers & lt);
@@ -548,55 +635,34 @@ k_sort_pass(const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ v
             tot += c;
         }
     }
-    // publish this tile's aggregate (or inclusive prefix for the segment's
-    // first tile)
-    uint32_t* my = lookback + gt * NB + tid;
+    // publish this tile's count (a group's first tile has none before it)
     const bool live = dig && hcnt != 0u;
-    if (live) st_relaxed(my, (tile == 0 ? LB_PRE : LB_AGG) | tot);
-    uint32_t ltot;
-    const uint32_t lstart = block_excl_scan_w<RS_WAVES>(tot, s_wsum, ltot);
-    if (dig) s_lstart[tid] = lstart;
-    // decoupled look-back over the segment's preceding tiles for digit tid:
-    // the statuses of LB_WIN tiles i, i - 1, ... are loaded in one round trip
-    // (the loads cross XCDs) and consumed in order, summing aggregates until
-    // an inclusive prefix; a tile not yet published ends the window, which is
-    // loaded again from there. The segment's first tile publishes its prefix
-    // at once, so every walk ends there at the latest (statuses loaded beyond
-    // it are not consumed).
+    if (live) st_relaxed(lookback + gt * NB + tid, (tile % LB_GROUP == 0 ? LB_PRE : LB_AGG) | tot);
+    // exclusive prefixes of the tile's and of the segment's digit counts
+    const uint2 ex = block_excl_scan2(make_uint2(tot, hcnt), s_wsum);
+    if (dig) s_lstart[tid] = ex.x;
+    // look-back for digit tid: the group's tiles before this one, then, in the
+    // group's last tile, publishing the group's count, the groups before it
     uint32_t excl = 0;
-    if (tile > 0 && live) {
-        int32_t i = (int32_t)gt - 1;
-        bool done = false;
-        while (!done) {
-            uint32_t st[LB_WIN];
-#pragma unroll
-            for (int w = 0; w < LB_WIN; w++) {
-                const int32_t t = i - w;
-                st[w] = t >= 0 ? ld_acq_relaxed(lookback + (uint32_t)t * NB + tid) : 0u;
-            }
-            int32_t used = LB_WIN;
-#pragma unroll
-            for (int w = 0; w < LB_WIN; w++) {
-                if (used != LB_WIN || done) continue;
-                const uint32_t fl = st[w] & ~LB_CNT;
-                if (fl == 0u) {
-                    used = w;
-                } else {
-                    excl += st[w] & LB_CNT;
-                    if (fl == LB_PRE) done = true;
-                }
-            }
-            if (done) break;
-            i -= used;
-            if (used != LB_WIN) __builtin_amdgcn_s_sleep(1);
+    if (live) {
+        const uint32_t in_group = tile % LB_GROUP;
+        excl = look_back<DB>(lookback, gt, in_group, tid);
+        const uint32_t g0 = seg0 / LB_GROUP + seg, grp = tile / LB_GROUP;
+        uint32_t* const groups = lookback + (uint64_t)S.tile0[S.ns] * NB;
+        uint32_t* const mine = groups + (g0 + grp) * NB + tid;
+        const bool last = in_group == LB_GROUP - 1u;
+        if (last) st_relaxed(mine, (grp == 0 ? LB_PRE : LB_AGG) | (excl + tot));
+        if (grp > 0) {
+            const uint32_t before = look_back<DB>(groups, g0 + grp, grp, tid);
+            excl += before;
+            if (last) st_relaxed(mine, LB_PRE | (excl + tot));
         }
-        st_relaxed(my, LB_PRE | (excl + tot));
     }
-    if (dig) s_gbase[tid] = sbase + gexcl + excl;
+    if (dig) s_gbase[tid] = sbase + ex.y + excl;
     __syncthreads();
     // stage in tile-local sorted order
 #pragma unroll
-    for (int j = 0; j < RS_ITEMS; j++) {
+    for (int j = 0; j < ITEMS; j++) {
         const uint32_t idx = wbase + 64u * j + lane;
         if (idx < n) {
             const uint32_t d = (k[j] >> shift) & (NB - 1u);
@@ -606,7 +672,7 @@ k_sort_pass(const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ v
         }
     }
     __syncthreads();
-    const uint32_t cnt_tile = (n - base < RS_TILE) ? (n - base) : RS_TILE;
+    const uint32_t cnt_tile = (n - base < TILE) ? (n - base) : TILE;
     for (uint32_t i = tid; i < cnt_tile; i += RS_THREADS) {
         const uint32_t key = s_keys[i];
         const uint32_t d = (key >> shift) & (NB - 1u);
@@ -1271,7 +1337,36 @@ hipError_t oi_launch_mesh_box(hipStream_t st, const oi_build_desc* d, const uint
     return hipGetLastError();
 }
 
-uint32_t oi_morton_chunk() { return OI_MORTON_CHUNK; }
+// Faces a workgroup of k_morton takes in a launch over F faces: 1, 2 or 4 a thread.
+// About one workgroup per CU, so that small launches spread and large ones add fewer
+// histograms to the shared ones: 1M faces 15 us with 2 a thread, 13 with 4.
+uint32_t oi_morton_chunk(uint64_t F)
+{
+    return OI_MORTON_T * (F <= 256ull * OI_MORTON_T ? 1u : F <= 512ull * OI_MORTON_T ? 2u : 4u);
+}
+
+static hipError_t launch_morton(hipStream_t st, uint32_t chunk, uint32_t nblocks, const BuildTab& t,
+                                const float* partials, uint32_t* keys, uint32_t* keys_hi, uint32_t* ghist,
+                                uint32_t hstride, uint32_t hreps, uint32_t* fmesh, uint32_t hbits)
+{
+    if ((hbits != 8 && hbits != 10) || (keys_hi && hbits != 8) || hreps == 0) return hipErrorInvalidValue;
+    switch (chunk) {
+    case OI_MORTON_T:
+        hipLaunchKernelGGL(k_morton<1>, dim3(nblocks), dim3(OI_MORTON_T), 0, st, t, partials, keys, keys_hi, ghist,
+                           hstride, hreps, fmesh, hbits);
+        break;
+    case 2 * OI_MORTON_T:
+        hipLaunchKernelGGL(k_morton<2>, dim3(nblocks), dim3(OI_MORTON_T), 0, st, t, partials, keys, keys_hi, ghist,
+                           hstride, hreps, fmesh, hbits);
+        break;
+    case 4 * OI_MORTON_T:
+        hipLaunchKernelGGL(k_morton<4>, dim3(nblocks), dim3(OI_MORTON_T), 0, st, t, partials, keys, keys_hi, ghist,
+                           hstride, hreps, fmesh, hbits);
+        break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
 
 hipError_t oi_launch_set_xf(hipStream_t st, float* dst, const float* mat4)
 {
@@ -1281,15 +1376,14 @@ hipError_t oi_launch_set_xf(hipStream_t st, float* dst, const float* mat4)
     return hipGetLastError();
 }
 
-// keys_hi: null for 30-bit keys, else the high words of 63-bit keys
+// keys_hi: null for 30-bit keys, else the high words of 63-bit keys; chunk: the
+// work items' (oi_morton_chunk)
 hipError_t oi_launch_morton(hipStream_t st, const oi_build_desc* d, const uint2* work, const oi_build_desc* one,
-                            uint32_t nblocks, const float* partials, uint32_t* keys, uint32_t* keys_hi,
-                            uint32_t* ghist, uint32_t* fmesh, uint32_t hbits)
+                            uint32_t nblocks, uint32_t chunk, const float* partials, uint32_t* keys,
+                            uint32_t* keys_hi, uint32_t* ghist, uint32_t hreps, uint32_t* fmesh, uint32_t hbits)
 {
-    if ((hbits != 8 && hbits != 10) || (keys_hi && hbits != 8)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_morton, dim3(nblocks), dim3(OI_BLOCK), 0, st, make_btab(d, work, one), partials, keys,
-                       keys_hi, ghist, 0u, fmesh, hbits);
-    return hipGetLastError();
+    return launch_morton(st, chunk, nblocks, make_btab(d, work, one), partials, keys, keys_hi, ghist, 0u, hreps,
+                         fmesh, hbits);
 }
 
 // n (<= OI_INLINE_MESHES) meshes in the kernel arguments, mesh m owning the
@@ -1306,14 +1400,12 @@ hipError_t oi_launch_mesh_box_inline(hipStream_t st, const oi_build_desc* meshes
 }
 
 hipError_t oi_launch_morton_inline(hipStream_t st, const oi_build_desc* meshes, uint32_t n, const uint32_t* boff,
-                                   uint32_t* keys, uint32_t* keys_hi, uint32_t* ghist, uint32_t hstride,
-                                   uint32_t hbits)
+                                   uint32_t chunk, uint32_t* keys, uint32_t* keys_hi, uint32_t* ghist,
+                                   uint32_t hstride, uint32_t hreps, uint32_t hbits)
 {
     if (n == 0 || n > OI_INLINE_MESHES) return hipErrorInvalidValue;
-    if ((hbits != 8 && hbits != 10) || (keys_hi && hbits != 8)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_morton, dim3(boff[n]), dim3(OI_BLOCK), 0, st, make_btab_inline(meshes, n, boff), nullptr,
-                       keys, keys_hi, ghist, hstride, nullptr, hbits);
-    return hipGetLastError();
+    return launch_morton(st, chunk, boff[n], make_btab_inline(meshes, n, boff), nullptr, keys, keys_hi, ghist,
+                         hstride, hreps, nullptr, hbits);
 }
 
 hipError_t oi_launch_set_mesh_pos(hipStream_t st, oi_build_desc* bd, oi_mesh_desc* md, uint32_t m, const float* pos)
@@ -1322,37 +1414,70 @@ hipError_t oi_launch_set_mesh_pos(hipStream_t st, oi_build_desc* bd, oi_mesh_des
     return hipGetLastError();
 }
 
-uint32_t oi_sort_tile() { return RS_TILE; }
+// Keys a thread of k_sort_pass takes, over ns segments of n[] keys: 1, 2, 4 or 8, the
+// fewest that leave at most 128 tiles (256 with 4). More tiles rank fewer keys each
+// but read more look-back statuses: builds of 122K, 250K and 518K triangles take 55.1,
+// 63.5 and 77.1 us, and up to 256 tiles of fewer keys 55.3, 68.3 and 79.7; of 1M 99.2
+// with 4 keys a thread, 103.9 with 8.
+static uint32_t sort_items(uint32_t ns, const uint32_t* n)
+{
+    for (uint32_t it = 1; it < RS_ITEMS_MAX; it *= 2) {
+        uint64_t tiles = 0;
+        for (uint32_t k = 0; k < ns; k++) tiles += ((uint64_t)n[k] + RS_THREADS * it - 1) / (RS_THREADS * it);
+        if (tiles <= (it < 4 ? OI_SORT_WGS / 2 : OI_SORT_WGS)) return it;
+    }
+    return RS_ITEMS_MAX;
+}
+
+uint32_t oi_sort_tiles(uint32_t ns, const uint32_t* n)
+{
+    const uint32_t tile = RS_THREADS * sort_items(ns, n);
+    uint32_t tiles = 0;
+    for (uint32_t k = 0; k < ns; k++) tiles += (uint32_t)(((uint64_t)n[k] + tile - 1) / tile);
+    return tiles;
+}
+
+// rows of a look-back buffer: one per tile, then one per group
+uint64_t oi_sort_rows(uint32_t ns, uint64_t tiles) { return tiles + tiles / LB_GROUP + ns; }
+
+uint64_t oi_sort_tiles_max(uint64_t cap)
+{
+    const uint64_t fine = (cap + RS_THREADS - 1) / RS_THREADS;
+    const uint64_t coarse = (cap + RS_THREADS * RS_ITEMS_MAX - 1) / (RS_THREADS * RS_ITEMS_MAX);
+    return fine < OI_SORT_WGS ? fine : coarse > OI_SORT_WGS ? coarse : OI_SORT_WGS;
+}
 
 hipError_t oi_launch_sort_pass_segs(hipStream_t st, const uint32_t* keys_in, const uint32_t* vals_in,
                                     uint32_t* keys_out, uint32_t* vals_out, uint32_t ns, const uint32_t* base,
                                     const uint32_t* n, uint32_t shift, const uint32_t* ghist, uint32_t hstride,
-                                    uint32_t* lookback, uint32_t* lookback_next, uint32_t* tile_counter,
-                                    const uint32_t* key_of_val, uint32_t bits);
+                                    uint32_t hreps, uint32_t* lookback, uint32_t* lookback_next,
+                                    uint32_t* tile_counter, const uint32_t* key_of_val, uint32_t bits);
 
 hipError_t oi_launch_sort_pass(hipStream_t st, const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
-                               uint32_t* vals_out, uint32_t n, uint32_t shift, const uint32_t* ghist,
+                               uint32_t* vals_out, uint32_t n, uint32_t shift, const uint32_t* ghist, uint32_t hreps,
                                uint32_t* lookback, uint32_t* lookback_next, uint32_t* tile_counter,
                                const uint32_t* key_of_val, uint32_t bits)
 {
     const uint32_t base = 0;
-    return oi_launch_sort_pass_segs(st, keys_in, vals_in, keys_out, vals_out, 1, &base, &n, shift, ghist, 0,
+    return oi_launch_sort_pass_segs(st, keys_in, vals_in, keys_out, vals_out, 1, &base, &n, shift, ghist, 0, hreps,
                                     lookback, lookback_next, tile_counter, key_of_val, bits);
 }
 
 uint32_t oi_sort_segs_max() { return OI_SORT_SEGS; }
 
 // ns segments: segment s is keys [base[s], base[s] + n[s]) of the arrays, its
-// digit histogram at ghist + s * hstride, its tile counter tile_counter[s];
-// look-back statuses are indexed by the tile id over all segments (sum of
-// ceil(n[s] / tile) tiles)
+// digit histogram at ghist + s * hstride (hreps copies, 1 or OI_HIST_REPS), its tile
+// counter tile_counter[s]; look-back statuses are indexed by the tile id over all
+// segments (oi_sort_tiles of them)
 hipError_t oi_launch_sort_pass_segs(hipStream_t st, const uint32_t* keys_in, const uint32_t* vals_in,
                                     uint32_t* keys_out, uint32_t* vals_out, uint32_t ns, const uint32_t* base,
                                     const uint32_t* n, uint32_t shift, const uint32_t* ghist, uint32_t hstride,
-                                    uint32_t* lookback, uint32_t* lookback_next, uint32_t* tile_counter,
-                                    const uint32_t* key_of_val, uint32_t bits)
+                                    uint32_t hreps, uint32_t* lookback, uint32_t* lookback_next,
+                                    uint32_t* tile_counter, const uint32_t* key_of_val, uint32_t bits)
 {
-    if (ns == 0 || ns > OI_SORT_SEGS || (bits != 8 && bits != 10)) return hipErrorInvalidValue;
+    if (ns == 0 || ns > OI_SORT_SEGS || (bits != 8 && bits != 10) || (hreps != 1 && hreps != OI_HIST_REPS))
+        return hipErrorInvalidValue;
+    const uint32_t items = sort_items(ns, n), tile = RS_THREADS * items;
     SortSegs S{};
     S.ns = ns;
     S.hstride = hstride;
@@ -1362,15 +1487,27 @@ hipError_t oi_launch_sort_pass_segs(hipStream_t st, const uint32_t* keys_in, con
         S.tile0[k] = tiles;
         S.base[k] = base[k];
         S.n[k] = n[k];
-        tiles += (n[k] + RS_TILE - 1) / RS_TILE;
+        tiles += (uint32_t)(((uint64_t)n[k] + tile - 1) / tile);
     }
     S.tile0[ns] = tiles;
-    if (bits == 10)
-        hipLaunchKernelGGL(k_sort_pass<10>, dim3(tiles), dim3(RS_THREADS), 0, st, keys_in, vals_in, keys_out,
-                           vals_out, S, shift, ghist, lookback, lookback_next, tile_counter, key_of_val);
-    else
-        hipLaunchKernelGGL(k_sort_pass<8>, dim3(tiles), dim3(RS_THREADS), 0, st, keys_in, vals_in, keys_out,
-                           vals_out, S, shift, ghist, lookback, lookback_next, tile_counter, key_of_val);
+#define PASS(DB, IT)                                                                                              \
+    hipLaunchKernelGGL((k_sort_pass<DB, IT>), dim3(tiles), dim3(RS_THREADS), 0, st, keys_in, vals_in, keys_out,   \
+                       vals_out, S, shift, ghist, hreps, lookback, lookback_next, tile_counter, key_of_val)
+    switch (items) {
+    case 1:
+        if (bits == 10) PASS(10, 1); else PASS(8, 1);
+        break;
+    case 2:
+        if (bits == 10) PASS(10, 2); else PASS(8, 2);
+        break;
+    case 4:
+        if (bits == 10) PASS(10, 4); else PASS(8, 4);
+        break;
+    default:
+        if (bits == 10) PASS(10, 8); else PASS(8, 8);
+        break;
+    }
+#undef PASS
     return hipGetLastError();
 }
 

@@ -51,6 +51,11 @@ __device__ __forceinline__ uint32_t oi_wave_scan_incl(uint32_t x)
 }
 #endif
 
+#define OI_HIST_WORDS 3072u  // one copy of a build's digit histograms: 8 x 256 or 3 x 1024 bins
+#define OI_HIST_REPS 8u      // copies of them
+#define OI_SORT_WGS 256u     // tiles a sort pass is divided into, if it has keys enough
+#define OI_SORT_GROUP 8u     // tiles of a look-back group
+
 // ---------------------------------------------------------------------------
 // device descriptors
 // ---------------------------------------------------------------------------

@@ -565,32 +565,32 @@ static oibvh_status sort_hits(oi_detector* d)
             dg.nd++;
         }
     }
-    const uint32_t tiles = (n + oi_sort_tile() - 1) / oi_sort_tile();
+    const uint32_t rows = (uint32_t)oi_sort_rows(1, oi_sort_tiles(1, &n));
     if (d->sort_cap < n) {
         // sized with headroom, so that the next queries rarely grow them
         const uint64_t cap = std::min<uint64_t>((1ull << 30) - 1, (uint64_t)n + (n >> 2));
-        const uint64_t ctiles = (cap + oi_sort_tile() - 1) / oi_sort_tile();
+        const uint64_t crows = oi_sort_rows(1, oi_sort_tiles_max(cap));
         dfree(d->sort_words);
         dfree(d->sort_vals);
         dfree(d->sort_scratch);
         d->sort_cap = 0;
         HIPCHK(c, dalloc(&d->sort_words, 4 * cap));
         HIPCHK(c, dalloc(&d->sort_vals, 2 * cap));
-        HIPCHK(c, dalloc(&d->sort_scratch, 256ull * OI_HIT_DIGITS + OI_HIT_DIGITS + 512ull * ctiles));
+        HIPCHK(c, dalloc(&d->sort_scratch, 256ull * OI_HIT_DIGITS + OI_HIT_DIGITS + 512ull * crows));
         d->sort_cap = (uint32_t)cap;
     }
     if ((r = grow(c, d->d_sorted, d->d_sorted_cap, n, gen)) != OIBVH_OK) return r;
     uint32_t* hist = d->sort_scratch;
     uint32_t* tctr = hist + 256u * OI_HIT_DIGITS;
-    uint32_t* lb[2] = {tctr + OI_HIT_DIGITS, tctr + OI_HIT_DIGITS + 256ull * tiles};
+    uint32_t* lb[2] = {tctr + OI_HIT_DIGITS, tctr + OI_HIT_DIGITS + 256ull * rows};
     uint32_t* vals[2] = {d->sort_vals, d->sort_vals + d->sort_cap};
     hipStream_t st = c->stream;
     // histograms, tile counters and the first look-back buffer start at zero
-    HIPCHK(c, oi_launch_zero_u32(st, hist, 256u * OI_HIT_DIGITS + OI_HIT_DIGITS + 256u * tiles));
+    HIPCHK(c, oi_launch_zero_u32(st, hist, 256u * OI_HIT_DIGITS + OI_HIT_DIGITS + 256u * rows));
     HIPCHK(c, oi_launch_hits_digits(st, d->hits, n, d->sort_words, hist, &dg));
     const uint32_t* order = nullptr;  // identity
     for (uint32_t p = 0; p < dg.nd; p++) {
-        HIPCHK(c, oi_launch_sort_pass(st, nullptr, order, nullptr, vals[p & 1], n, dg.shift[p], hist + 256u * p,
+        HIPCHK(c, oi_launch_sort_pass(st, nullptr, order, nullptr, vals[p & 1], n, dg.shift[p], hist + 256u * p, 1u,
                                       lb[p & 1], p + 1 < dg.nd ? lb[(p + 1) & 1] : nullptr, tctr + p,
                                       d->sort_words + (uint64_t)n * dg.word[p]));
         order = vals[p & 1];

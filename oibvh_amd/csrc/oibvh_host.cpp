@@ -145,7 +145,6 @@ struct oibvh_tree {
     uint32_t* keys_alt = nullptr;
     uint32_t* vals_tmp = nullptr;
     uint32_t* sort_scratch = nullptr;
-    uint32_t tiles = 0;
     uint32_t morton_bits = 30;
     float* box = nullptr;        // 6 floats + per-block partial boxes
     float* xf = nullptr;         // model matrix (16 floats, device)
@@ -504,23 +503,24 @@ oibvh_status oi_enqueue_build(oibvh_ctx* c, const oi_build_desc& d, const oi_bui
                               hipStream_t stream)
 {
     const uint32_t F = d.F;
-    const uint32_t tiles = (F + oi_sort_tile() - 1) / oi_sort_tile();
+    const uint32_t rows = (uint32_t)oi_sort_rows(1, oi_sort_tiles(1, &F));
     const bool m63 = s.keys_hi != nullptr;
     uint32_t* ghist = s.sort;
-    uint32_t* tctr = s.sort + OI_SORT_HIST;
-    uint32_t* lb[2] = {s.sort + OI_SORT_HEAD, s.sort + OI_SORT_HEAD + (uint64_t)OI_SORT_LB * tiles};
+    const uint32_t chunk = oi_morton_chunk(F), mblocks = (F + chunk - 1) / chunk;
+    const uint32_t hreps = oi_hist_reps(mblocks), hwords = hreps * OI_HIST_WORDS;
+    uint32_t* tctr = ghist + hwords;
+    uint32_t* lb[2] = {tctr + OI_SORT_CTRS, tctr + OI_SORT_CTRS + (uint64_t)OI_SORT_LB * rows};
     hipStream_t st = stream ? stream : c->stream;
-    // the mesh-box launch also clears the histograms, tile counters and the
-    // first look-back buffer (a kernel, not a memset: capturable)
-    HIPCHK(c, oi_launch_mesh_box(st, nullptr, nullptr, &d, d.nparts, d.box + 6, s.sort,
-                                 OI_SORT_HEAD + OI_SORT_LB * tiles));
-    const uint32_t mblocks = (F + oi_morton_chunk() - 1) / oi_morton_chunk();
     // 30-bit keys: three passes of 10-bit digits; 63-bit keys: four 8-bit
     // passes over the low word (keys move with the values), then four over
     // the high word looked up by face id. Values end in perm.
     const uint32_t bits = m63 ? 8u : OI_M30_BITS;
-    HIPCHK(c, oi_launch_morton(st, nullptr, nullptr, &d, mblocks, d.box + 6, s.keys, s.keys_hi, ghist, nullptr,
-                               bits));
+    // the mesh-box launch also clears the histograms, tile counters and the
+    // first look-back buffer (a kernel, not a memset: capturable)
+    HIPCHK(c, oi_launch_mesh_box(st, nullptr, nullptr, &d, d.nparts, d.box + 6, s.sort,
+                                 hwords + OI_SORT_CTRS + (rows << bits)));
+    HIPCHK(c, oi_launch_morton(st, nullptr, nullptr, &d, mblocks, chunk, d.box + 6, s.keys, s.keys_hi, ghist, hreps,
+                               nullptr, bits));
     const int np = m63 ? 8 : OI_M30_PASSES, nlo = m63 ? 4 : OI_M30_PASSES;
     for (int p = 0; p < np; p++) {
         const bool lo = p < nlo;
@@ -530,8 +530,8 @@ oibvh_status oi_enqueue_build(oibvh_ctx* c, const oi_build_desc& d, const oi_bui
         uint32_t* vout = ((np - 1 - p) & 1) ? s.vals_tmp : d.perm;
         const uint32_t* vin = p == 0 ? nullptr : (((np - p) & 1) ? s.vals_tmp : d.perm);
         const uint32_t shift = bits * (uint32_t)(p % nlo);
-        HIPCHK(c, oi_launch_sort_pass(st, kin, vin, kout, vout, F, shift, ghist + (p << bits), lb[p & 1],
-                                      p + 1 < np ? lb[(p + 1) & 1] : nullptr, tctr + p, lo ? nullptr : s.keys_hi,
+        HIPCHK(c, oi_launch_sort_pass(st, kin, vin, kout, vout, F, shift, ghist + (p << bits), hreps,
+                                      lb[p & 1], p + 1 < np ? lb[(p + 1) & 1] : nullptr, tctr + p, lo ? nullptr : s.keys_hi,
                                       bits));
     }
     const uint32_t h = oi_reduce_height(M, d.L);
@@ -550,14 +550,13 @@ static oibvh_status build_scratch(oibvh_tree* t, oi_build_scratch* out)
 {
     oibvh_ctx* c = t->ctx;
     const uint32_t F = t->F;
-    const uint32_t tiles = (F + oi_sort_tile() - 1) / oi_sort_tile();
+    const uint64_t rows = oi_sort_rows(1, oi_sort_tiles(1, &F));
     const bool m63 = t->morton_bits == 63;
     if (!t->keys) {
         HIPCHK(c, dalloc(&t->keys, F));
         HIPCHK(c, dalloc(&t->keys_alt, F));
         HIPCHK(c, dalloc(&t->vals_tmp, F));
-        t->tiles = tiles;
-        HIPCHK(c, dalloc(&t->sort_scratch, OI_SORT_HEAD + 2ull * OI_SORT_LB * tiles));
+        HIPCHK(c, dalloc(&t->sort_scratch, OI_SORT_HEAD + 2ull * OI_SORT_LB * rows));
     }
     if (m63 && !t->keys_hi) HIPCHK(c, dalloc(&t->keys_hi, F));
     *out = oi_build_scratch{t->keys, t->keys_alt, m63 ? t->keys_hi : nullptr, t->vals_tmp, t->sort_scratch};
@@ -1023,12 +1022,12 @@ static oibvh_status scene_refit(oibvh_scene* s, const oi_seed_args* seed, bool* 
 #define OI_SCENE_BUILD_GROUP 4
 #define OI_SCENE_CTRS (8u * OI_SCENE_BUILD_GROUP)
 
-// The scene build's scratch for a group of n trees with F faces and `tiles`
-// sort tiles in all (grown on demand, after the context's streams drain).
-static oibvh_status scene_build_scratch(oibvh_scene* s, uint64_t F, uint32_t n, uint32_t tiles, bool m63)
+// The scene build's scratch for a group of n trees with F faces and `rows`
+// look-back rows in all (grown on demand, after the context's streams drain).
+static oibvh_status scene_build_scratch(oibvh_scene* s, uint64_t F, uint32_t n, uint32_t rows, bool m63)
 {
     oibvh_ctx* c = s->ctx;
-    const uint64_t words = (uint64_t)n * OI_SORT_HIST + OI_SCENE_CTRS + 2ull * OI_SORT_LB * tiles;
+    const uint64_t words = (uint64_t)n * OI_SORT_HIST + OI_SCENE_CTRS + 2ull * OI_SORT_LB * rows;
     const bool grow = F > s->b_cap || words > s->b_sort_cap || (m63 && F > s->b_hi_cap);
     if (!grow) return OIBVH_OK;
     HIPCHK(c, oi_ctx_quiesce(c));
@@ -1063,7 +1062,7 @@ static oibvh_status scene_build_scratch(oibvh_scene* s, uint64_t F, uint32_t n, 
 // Morton width, their build descriptors over the concatenated faces and the
 // launch geometry.
 struct SceneBuildGroup {
-    uint32_t n = 0, tiles = 0;
+    uint32_t n = 0, rows = 0, chunk = 0;
     bool m63 = false;
     int M = 0;
     uint64_t F = 0;
@@ -1075,7 +1074,9 @@ struct SceneBuildGroup {
 
 static void plan_group(const oibvh_ctx* c, oibvh_tree* const* trees, uint32_t n, SceneBuildGroup& g)
 {
-    const uint32_t tile = oi_sort_tile(), chunk = oi_morton_chunk();
+    uint64_t Ft = 0;
+    for (uint32_t k = 0; k < n; k++) Ft += trees[k]->F;
+    g.chunk = oi_morton_chunk(Ft);
     g.n = n;
     g.m63 = trees[0]->morton_bits == 63;
     for (uint32_t k = 0; k < n; k++) {
@@ -1085,10 +1086,10 @@ static void plan_group(const oibvh_ctx* c, oibvh_tree* const* trees, uint32_t n,
         g.base[k] = (uint32_t)g.F;
         g.nf[k] = d.F;
         g.box_off[k + 1] = g.box_off[k] + d.nparts;
-        g.mort_off[k + 1] = g.mort_off[k] + (d.F + chunk - 1) / chunk;
-        g.tiles += (d.F + tile - 1) / tile;
+        g.mort_off[k + 1] = g.mort_off[k] + (d.F + g.chunk - 1) / g.chunk;
         g.F += d.F;
     }
+    g.rows = (uint32_t)oi_sort_rows(n, oi_sort_tiles(n, g.nf));
     g.M = (int)c->leaves_per_thread;
     if (!g.M) g.M = oi_default_lpt(g.F, c->cus);
     for (uint32_t k = 0; k < n; k++) {
@@ -1105,22 +1106,23 @@ static void plan_group(const oibvh_ctx* c, oibvh_tree* const* trees, uint32_t n,
 static oibvh_status enqueue_group(oibvh_scene* s, const SceneBuildGroup& g)
 {
     oibvh_ctx* c = s->ctx;
-    const uint32_t n = g.n, tiles = g.tiles;
+    const uint32_t n = g.n, rows = g.rows;
     hipStream_t st = c->stream;
     uint32_t* ghist = s->b_sort;
-    uint32_t* ctrs = ghist + (uint64_t)n * OI_SORT_HIST;
-    uint32_t* lb[2] = {ctrs + OI_SCENE_CTRS, ctrs + OI_SCENE_CTRS + (uint64_t)OI_SORT_LB * tiles};
-    // the mesh-box launch also clears the histograms, counters and the first
-    // look-back buffer (a kernel, not a memset: capturable)
-    HIPCHK(c, oi_launch_mesh_box_inline(st, g.d, n, g.box_off, ghist,
-                                        n * OI_SORT_HIST + OI_SCENE_CTRS + OI_SORT_LB * tiles));
+    const uint32_t hreps = oi_hist_reps(g.mort_off[n]), hwords = hreps * OI_HIST_WORDS;
+    uint32_t* ctrs = ghist + (uint64_t)n * hwords;
+    uint32_t* lb[2] = {ctrs + OI_SCENE_CTRS, ctrs + OI_SCENE_CTRS + (uint64_t)OI_SORT_LB * rows};
     // 30-bit keys: three passes of 10-bit digits; 63-bit keys: four 8-bit
     // passes over the low words, then four over the high words looked up by
     // value. The sorted values (face ids over the concatenated faces) end in
     // b_vals.
     const uint32_t bits = g.m63 ? 8u : OI_M30_BITS;
-    HIPCHK(c, oi_launch_morton_inline(st, g.d, n, g.mort_off, s->b_keys, g.m63 ? s->b_keys_hi : nullptr, ghist,
-                                      OI_SORT_HIST, bits));
+    // the mesh-box launch also clears the histograms, counters and the first
+    // look-back buffer (a kernel, not a memset: capturable)
+    HIPCHK(c, oi_launch_mesh_box_inline(st, g.d, n, g.box_off, ghist,
+                                        n * hwords + OI_SCENE_CTRS + (rows << bits)));
+    HIPCHK(c, oi_launch_morton_inline(st, g.d, n, g.mort_off, g.chunk, s->b_keys, g.m63 ? s->b_keys_hi : nullptr,
+                                      ghist, hwords, hreps, bits));
     const int np = g.m63 ? 8 : OI_M30_PASSES, nlo = g.m63 ? 4 : OI_M30_PASSES;
     for (int p = 0; p < np; p++) {
         const bool lo = p < nlo;
@@ -1130,7 +1132,7 @@ static oibvh_status enqueue_group(oibvh_scene* s, const SceneBuildGroup& g)
         uint32_t* vout = ((np - 1 - p) & 1) ? s->b_vals_tmp : s->b_vals;
         const uint32_t* vin = p == 0 ? nullptr : (((np - p) & 1) ? s->b_vals_tmp : s->b_vals);
         HIPCHK(c, oi_launch_sort_pass_segs(st, kin, vin, kout, vout, n, g.base, g.nf, bits * (uint32_t)(p % nlo),
-                                           ghist + (p << bits), OI_SORT_HIST, lb[p & 1],
+                                           ghist + (p << bits), hwords, hreps, lb[p & 1],
                                            p + 1 < np ? lb[(p + 1) & 1] : nullptr, ctrs + p * OI_SCENE_BUILD_GROUP,
                                            lo ? nullptr : s->b_keys_hi, bits));
     }
@@ -1160,7 +1162,7 @@ extern "C" oibvh_status oibvh_scene_build(oibvh_scene* s)
     const uint32_t per = std::min<uint32_t>(OI_SCENE_BUILD_GROUP, std::min(oi_inline_meshes(), oi_sort_segs_max()));
     std::vector<SceneBuildGroup> groups;
     uint64_t Fmax = 0;
-    uint32_t nmax = 0, tmax = 0;
+    uint32_t nmax = 0, rmax = 0;
     bool m63 = false;
     for (size_t i = 0; i < s->trees.size();) {
         uint32_t n = 1;
@@ -1171,12 +1173,12 @@ extern "C" oibvh_status oibvh_scene_build(oibvh_scene* s)
         if (g.F > 0xffffffffull) return oi_set_err(c, OIBVH_ERR_CAPACITY, "scene build: too many faces in one group");
         Fmax = std::max(Fmax, g.F);
         nmax = std::max(nmax, g.n);
-        tmax = std::max(tmax, g.tiles);
+        rmax = std::max(rmax, g.rows);
         m63 = m63 || g.m63;
         i += n;
     }
     if (groups.empty()) return OIBVH_OK;
-    oibvh_status r = scene_build_scratch(s, Fmax, nmax, tmax, m63);
+    oibvh_status r = scene_build_scratch(s, Fmax, nmax, rmax, m63);
     if (r != OIBVH_OK) return r;
     for (const SceneBuildGroup& g : groups)
         if ((r = enqueue_group(s, g)) != OIBVH_OK) return r;

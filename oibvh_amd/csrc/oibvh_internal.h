@@ -17,35 +17,44 @@
 extern "C" {
 hipError_t oi_launch_mesh_box(hipStream_t, const oi_build_desc*, const uint2*, const oi_build_desc*, uint32_t, float*,
                               uint32_t*, uint32_t);
-uint32_t oi_morton_chunk();
+uint32_t oi_morton_chunk(uint64_t F);
 hipError_t oi_launch_mesh_box_inline(hipStream_t, const oi_build_desc*, uint32_t, const uint32_t*, uint32_t*,
                                      uint32_t);
 // hbits: digit width of the histograms the Morton launch accumulates (8, or
 // 10 for 30-bit keys)
-hipError_t oi_launch_morton_inline(hipStream_t, const oi_build_desc*, uint32_t, const uint32_t*, uint32_t*,
-                                   uint32_t*, uint32_t*, uint32_t, uint32_t hbits = 8);
-hipError_t oi_launch_morton(hipStream_t, const oi_build_desc*, const uint2*, const oi_build_desc*, uint32_t,
-                            const float*, uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t hbits = 8);
+hipError_t oi_launch_morton_inline(hipStream_t, const oi_build_desc*, uint32_t, const uint32_t*, uint32_t, uint32_t*,
+                                   uint32_t*, uint32_t*, uint32_t, uint32_t, uint32_t hbits = 8);
+hipError_t oi_launch_morton(hipStream_t, const oi_build_desc*, const uint2*, const oi_build_desc*, uint32_t, uint32_t,
+                            const float*, uint32_t*, uint32_t*, uint32_t*, uint32_t, uint32_t*, uint32_t hbits = 8);
 
-// sort scratch: digit histograms (8 x 256 or 3 x 1024 bins) | per-pass tile
-// counters | two look-back buffers of OI_SORT_LB words per tile (256 per
-// tile suffice for 8-bit digits)
-#define OI_SORT_HIST 3072u
+// sort scratch: OI_HIST_REPS copies of the digit histograms (8 x 256 or 3 x 1024
+// bins) | per-pass tile counters | two look-back buffers of oi_sort_rows rows of
+// OI_SORT_LB words (256 for 8-bit digits)
+#define OI_SORT_HIST (OI_HIST_REPS * OI_HIST_WORDS)
 #define OI_SORT_CTRS 16u
 #define OI_SORT_HEAD (OI_SORT_HIST + OI_SORT_CTRS)
 #define OI_SORT_LB 1024u
 // 30-bit Morton keys of a tree or scene build: three passes of 10-bit digits
 #define OI_M30_PASSES 3
 #define OI_M30_BITS 10u
-uint32_t oi_sort_tile();
+// Copies of the digit histograms a Morton launch of `wgs` workgroups adds to. A copy
+// costs a clear of 12 KB and a load per pass; without copies the additions of 489
+// workgroups to one cache line took 5 of 24 us (1M triangles).
+static inline uint32_t oi_hist_reps(uint32_t wgs) { return wgs < 64u ? 1u : OI_HIST_REPS; }
+// tiles of a pass over ns segments of n[] keys, and the most of one over at most
+// cap keys in one segment
+uint32_t oi_sort_tiles(uint32_t ns, const uint32_t* n);
+uint64_t oi_sort_tiles_max(uint64_t cap);
+// rows of 2^bits words in a look-back buffer of a pass of `tiles` tiles
+uint64_t oi_sort_rows(uint32_t ns, uint64_t tiles);
 hipError_t oi_launch_sort_pass(hipStream_t, const uint32_t*, const uint32_t*, uint32_t*, uint32_t*, uint32_t,
-                               uint32_t, const uint32_t*, uint32_t*, uint32_t*, uint32_t*, const uint32_t*,
+                               uint32_t, const uint32_t*, uint32_t, uint32_t*, uint32_t*, uint32_t*, const uint32_t*,
                                uint32_t bits = 8);
 uint32_t oi_sort_segs_max();
 // bits: digit width, 8 or 10 (look-back buffers of 2^bits words per tile)
 hipError_t oi_launch_sort_pass_segs(hipStream_t, const uint32_t*, const uint32_t*, uint32_t*, uint32_t*, uint32_t,
-                                    const uint32_t*, const uint32_t*, uint32_t, const uint32_t*, uint32_t, uint32_t*,
-                                    uint32_t*, uint32_t*, const uint32_t*, uint32_t bits = 8);
+                                    const uint32_t*, const uint32_t*, uint32_t, const uint32_t*, uint32_t, uint32_t,
+                                    uint32_t*, uint32_t*, uint32_t*, const uint32_t*, uint32_t bits = 8);
 uint32_t oi_reduce_height(int, uint32_t);
 hipError_t oi_launch_reduce(hipStream_t, int, const oi_build_desc*, const uint2*, const oi_build_desc*, uint32_t,
                             const uint32_t*, uint32_t, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr,
@@ -174,8 +183,8 @@ oibvh_status oi_set_err(oibvh_ctx* ctx, oibvh_status st, const char* fmt, ...);
 
 // device scratch of one build: sort keys (two buffers, plus the high words
 // of 63-bit keys or null), the values' ping-pong buffer and the sort's
-// histograms, tile counters and look-back tiles (OI_SORT_HEAD + 512 words
-// per sort tile)
+// histograms, tile counters and look-back buffers (OI_SORT_HEAD + 2 OI_SORT_LB
+// words per look-back row)
 struct oi_build_scratch {
     uint32_t* keys;
     uint32_t* keys_alt;

@@ -20,15 +20,16 @@
 
 // layout of the scratch (32-bit words), each part 256-byte aligned:
 // keys | keys_alt | vals_tmp (F each) | sort head + look-back (OI_SORT_HEAD +
-// 2 OI_SORT_LB words per sort tile) | Morton box + mesh-box partials (6 + 6 * 256)
+// 2 OI_SORT_LB words per look-back row) | Morton box + mesh-box partials (6 + 6 * 256)
 #define OI_NA_ALIGN 64u
 #define OI_NA_ROUND(x) (((x) + OI_NA_ALIGN - 1u) & ~(OI_NA_ALIGN - 1u))
-// the sort's tile is 8192 keys; the run-time check below refuses a build
-// whose parts do not fit (should that tile ever shrink)
-#define OI_NA_TILE_MIN 8192u
+// a sort of at most 4,096 x OI_SORT_WGS keys has at most OI_SORT_WGS tiles (the
+// run-time check below refuses a build whose parts do not fit)
+static_assert(OIBVH_NOALLOC_MAX_FACES <= 4096u * OI_SORT_WGS, "sort tiles");
+#define OI_NA_ROWS (OI_SORT_WGS + OI_SORT_WGS / OI_SORT_GROUP + 1u)
 #define OI_NA_WORDS                                                                                  \
     (3u * OI_NA_ROUND(OIBVH_NOALLOC_MAX_FACES) +                                                     \
-     OI_NA_ROUND(OI_SORT_HEAD + 2u * OI_SORT_LB * ((OIBVH_NOALLOC_MAX_FACES + OI_NA_TILE_MIN - 1u) / OI_NA_TILE_MIN)) + \
+     OI_NA_ROUND(OI_SORT_HEAD + 2u * OI_SORT_LB * OI_NA_ROWS) +                                      \
      OI_NA_ROUND(6u + 6u * 256u))
 
 static __device__ __align__(256) uint32_t scratch[OI_NA_WORDS];
@@ -69,8 +70,8 @@ extern "C" oibvh_status oibvh_build_noalloc(oibvh_ctx* ctx, const float* xyz, ui
     if (F > OIBVH_NOALLOC_MAX_FACES)
         return oi_set_err(ctx, OIBVH_ERR_CAPACITY, "oibvh_build_noalloc: %u faces exceed the maximum of %u", F,
                           OIBVH_NOALLOC_MAX_FACES);
-    const uint32_t tiles = (F + oi_sort_tile() - 1) / oi_sort_tile();
-    const uint64_t need = 3ull * OI_NA_ROUND(F) + OI_NA_ROUND(OI_SORT_HEAD + 2ull * OI_SORT_LB * tiles) +
+    const uint32_t rows = (uint32_t)oi_sort_rows(1, oi_sort_tiles(1, &F));
+    const uint64_t need = 3ull * OI_NA_ROUND(F) + OI_NA_ROUND(OI_SORT_HEAD + 2ull * OI_SORT_LB * rows) +
                           OI_NA_ROUND(6u + 6u * 256u);
     if (need > OI_NA_WORDS)
         return oi_set_err(ctx, OIBVH_ERR_CAPACITY, "oibvh_build_noalloc: %llu scratch words needed, %u held",
@@ -92,7 +93,7 @@ extern "C" oibvh_status oibvh_build_noalloc(oibvh_ctx* ctx, const float* xyz, ui
     s.vals_tmp = w;
     w += OI_NA_ROUND(F);
     s.sort = w;
-    w += OI_NA_ROUND(OI_SORT_HEAD + 2u * OI_SORT_LB * tiles);
+    w += OI_NA_ROUND(OI_SORT_HEAD + 2u * OI_SORT_LB * rows);
     s.keys_hi = nullptr;  // 30-bit keys (the reference's morton3D)
     oi_build_desc d{};
     d.pos = xyz;

@@ -152,6 +152,32 @@ def cell_cluster(F, seed):
     return xyz, f
 
 
+@pytest.mark.parametrize("m63", [False, True])
+@pytest.mark.parametrize("sizes", [[1023], [1024], [8 * 1024], [8 * 1024 + 1], [128 * 1024], [128 * 1024 + 1],
+                                   [256 * 1024 + 1], [1024 * 1024 + 1], [9000, 1, 70001, 17 * 1024],
+                                   [120000, 9 * 1024, 1025, 200000]])
+def test_build_sort_tile_edges(api, ctx, orc, sizes, m63):
+    """The sort's tiles (1,024 to 8,192 keys), look-back groups (8 tiles) and the
+    Morton launch's workgroups at their edges, alone and as segments of one launch:
+    a permutation that sorts the oracle's keys stably, equal to the oracle's."""
+    say(f"build sort tiles {sizes} m63={m63}")
+    meshes = [soup(F, 31 + F) for F in sizes]
+    sc = api.Scene(ctx)
+    trees = []
+    for x, f in meshes:
+        t = api.OibvhTree(ctx, x, f)
+        t.set_morton_bits(63 if m63 else 30)
+        t.build()
+        sc.addOibvhTree(t)
+        trees.append(t)
+    want = [orc.Tree(x, f, order="morton63" if m63 else "morton").order for x, f in meshes]
+    for again in (False, True):
+        if again:
+            sc.build()
+        for t, w, F in zip(trees, want, sizes):
+            assert np.array_equal(t.perm(), w), (F, again)
+
+
 @pytest.mark.parametrize("F", [1, 2, 5, 257, 4097, 65537, 300001])
 def test_build_morton63_soup_bit_exact(api, ctx, orc, F):
     say(f"build 63-bit soup F={F}")
