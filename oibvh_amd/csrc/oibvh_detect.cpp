@@ -266,12 +266,13 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
     // undecided collected in the candidate buffer for one FP64 pass
     d->fused = !c->narrow_separate && (!fp64 || (J == 0 && T >= d->n_levels));
     const int fuse = d->fused ? (fp64 ? 2 : 1) : 0;
-    // Workgroups per step. A step of two levels fits six workgroups on a CU;
+    // Workgroups per step. A step of up to two levels fits six workgroups on a CU;
     // with six instead of four the folded cloth of 8.4M triangles takes 1,743
     // instead of 1,849 us a frame, one of 522K 264 instead of 279. With the FP32
     // filter in the step four are faster (331 against 339 us on coplanar scenes),
     // and beside the next frame's refit they leave it room.
-    const uint32_t grid = c->trav_blocks || fuse != 1 || d->stream ? oi_grid_for(c) : (uint32_t)std::max(1, c->cus) * 6u;
+    const uint32_t grid = oi_grid_for(c);
+    const uint32_t grid2 = c->trav_blocks || fuse != 1 || d->stream ? grid : (uint32_t)std::max(1, c->cus) * 6u;
     // `done` rides on the last launch: k_narrow, else the tail walk, else
     // the last step, else the head walk
     const bool narrow = !d->fused || fp64, tail = T < d->n_levels, steps = T > J;
@@ -323,7 +324,7 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
             k = o;
             continue;
         }
-        HIPCHK(c, oi_launch_bvtt_step(st, grid, &d->tab, k == 0, in, k ? d->counts + k : nullptr, d->n_front,
+        HIPCHK(c, oi_launch_bvtt_step(st, d->step_e[k] < 3 ? grid2 : grid, &d->tab, k == 0, in, k ? d->counts + k : nullptr, d->n_front,
                                       k ? d->front_cap : d->n_front, d->front[rd], d->counts + k + 1,
                                       d->front_cap, d->cands, &d->ctl->cands, d->cand_cap, d->hits, d->hits_cap,
                                       d->ctl, d->step_e[k], d->implicit_end, fuse,
