@@ -976,15 +976,21 @@ k_bvtt_step(StepArgs<Tab> A)
 // 2 their children by e2. Kept pairs of the last phase, and leaf pairs, gather in
 // rings (FUSE as in k_bvtt_step). Fronts, candidates, counts per level and
 // statistics are those of the same steps one by one.
-// The rings are small (25 KB a workgroup in all) so that workgroups find room
+// A round of three levels is 32 pairs, one pass of the workgroup (WALK_MID; 16 pairs
+// left half of its lanes idle: 161 -> 152 us a frame of two 1M-triangle bodies, 16
+// overlapped frames 1,108 -> 1,068). On fronts of 16K pairs and more, twice the
+// workgroups hide more of the chain (152 -> 144); on shorter ones their additions to
+// the shared counters cost more than that (132 against 127 us, five rigid bodies).
+// The rings are small (33 KB a workgroup in all) so that workgroups find room
 // beside a refit; with 64 KB lists the same walks took 16 overlapped frames of two
 // 1M-triangle bodies from 1,111 to 1,310 us.
 // Frame and pairs: two bodies of 1,280 triangles 102 -> 68 us, of 81,920 128 -> 91,
-// of 1M 183 -> 159. Of a walk's 11 us on 100 pairs, 1.8 are the launch and the
+// of 1M 183 -> 144. Of a walk's 11 us on 100 pairs, 1.8 are the launch and the
 // front's length, 3.4 the entries and their boxes, 2.6 each step.
 // ---------------------------------------------------------------------------
 #define WALK_T TB
-#define WALK_MID 1024   // first-step children per round
+#define WALK_MID 2048   // first-step children per round
+#define WALK_LONG 16384 // fronts from here on are walked by the whole launch
 #define WALK_RING 512   // a ring is emptied from WALK_T pairs on
 
 template <class Tab>
@@ -1012,6 +1018,7 @@ struct WalkArgs {
     uint32_t* defer_count;
     uint32_t defer_cap;
     uint32_t implicit_end;
+    uint32_t wgs;              // workgroups that walk a front shorter than WALK_LONG
 };
 
 struct WalkLds : RingLds<WALK_RING, WALK_RING> {
@@ -1125,9 +1132,10 @@ __global__ void __launch_bounds__(WALK_T) k_bvtt_walk(WalkArgs<Tab> A)
     // from one pair and read the same nodes, but a long run of them would leave
     // one workgroup with all the work of a dense spot. (Shallow steps leave little
     // work per pair, mostly leaf tests, which run in fewer, fuller workgroups.)
-    const uint32_t lgg = n_in >= 32u * gridDim.x ? 5u : n_in >= 8u * gridDim.x || A.e1 + A.e2 <= 2u ? 3u : 0u;
-    if ((blockIdx.x << lgg) >= n_in) return;
-    const uint32_t share = gridDim.x << lgg;
+    const uint32_t wgs = n_in >= WALK_LONG ? gridDim.x : A.wgs;
+    const uint32_t lgg = n_in >= 32u * wgs ? 5u : n_in >= 8u * wgs || A.e1 + A.e2 <= 2u ? 3u : 0u;
+    if (blockIdx.x >= wgs || (blockIdx.x << lgg) >= n_in) return;
+    const uint32_t share = wgs << lgg;
     const uint32_t per = min((n_in + share - 1u) / share << lgg, (uint32_t)WALK_T);
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     if (tid == 0) S.n0 = S.n_mid = S.n_out = S.n_cand = 0;
@@ -1198,7 +1206,7 @@ __global__ void __launch_bounds__(WALK_T) k_bvtt_walk(WalkArgs<Tab> A)
                         __syncthreads();
                         if (tid == 0) S.n0 = 0;
                         __syncthreads();
-                        b0 += gridDim.x * per;
+                        b0 += wgs * per;
                         r0 = 0;
                     }
                 }
@@ -1826,7 +1834,8 @@ static hipError_t launch_walk(hipStream_t st, uint32_t grid, const Tab& tab, con
     a.defer_count = &ctl->deferred;
     a.defer_cap = cand_cap;
     a.implicit_end = implicit_end;
-    const dim3 g(grid), b(WALK_T);
+    a.wgs = grid;
+    const dim3 g(std::max(grid, w.wgs_long)), b(WALK_T);
     switch (fused) {
     case 0: launch_done((k_bvtt_walk<0, Tab>), g, b, st, w.done, a); break;
     case 1: launch_done((k_bvtt_walk<1, Tab>), g, b, st, w.done, a); break;
@@ -1950,7 +1959,8 @@ hipError_t oi_launch_bvtt_step(hipStream_t st, uint32_t grid, const oi_tab_args*
                        expand, implicit_end, fused, done);
 }
 
-// one or two steps over a short front (k_bvtt_walk), `grid` workgroups
+// one or two steps over a short front (k_bvtt_walk), `grid` workgroups (w->wgs_long,
+// if more, over a long one)
 hipError_t oi_launch_bvtt_walk(hipStream_t st, uint32_t grid, const oi_tab_args* t, const oi_walk_args* w,
                                uint2* cands, uint32_t* cand_count, uint32_t cand_cap, uint4* hits, uint32_t hits_cap,
                                oi_detect_ctl* ctl, uint32_t implicit_end, int fused)

@@ -227,6 +227,7 @@ struct oi_walk_args {
     uint32_t* count_mid;       // with e2: counts the first step's kept pairs
     uint32_t* count_out;
     uint32_t cap_out;
+    uint32_t wgs_long;         // workgroups for a long front (0: as for a short one)
     hipEvent_t done;           // recorded when the launch completes (null: none)
 };
 

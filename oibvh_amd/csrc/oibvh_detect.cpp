@@ -139,6 +139,9 @@ oibvh_status oi_det_set_front(oi_detector* d, const std::vector<uint2>& front)
 #define OI_WALK_MAX3 65536u
 #define OI_WALK_MAX 2048u
 #define OI_WALK_TESTS (1u << 21)
+// guessed lengths from here on get workgroups for a long front (beside the next
+// frame's refit they would take its room)
+#define OI_WALK_LONG 16384u
 static void plan_walk(oi_detector* d)
 {
     std::memset(d->step_walk, 0, sizeof d->step_walk);
@@ -147,10 +150,10 @@ static void plan_walk(oi_detector* d)
     uint64_t est = d->n_front;
     auto grown = [&](uint32_t k) { return est * (self ? (1u << d->step_e[k]) + 3u : d->step_e[k] + 1u); };
     for (uint32_t k = 0; k < d->n_levels && est <= (d->step_e[k] == 3 ? OI_WALK_MAX3 : OI_WALK_MAX); k++) {
-        d->step_walk[k] = 1;
+        d->step_walk[k] = est >= OI_WALK_LONG ? 5 : 1;
         est = grown(k);
         if (k + 1 < d->n_levels && est << (2u * d->step_e[k + 1]) <= OI_WALK_TESTS) {
-            d->step_walk[k++] = 2;
+            d->step_walk[k++]++;
             est = grown(k);
         }
     }
@@ -303,7 +306,7 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
         rd ^= 1u;
         if (d->step_walk[k]) {
             // this step, or this and the next one, over a short front
-            const bool two = d->step_walk[k] == 2;
+            const bool two = (d->step_walk[k] & 3u) == 2;
             const uint32_t o = two ? k + 1 : k;
             oi_walk_args w{};
             w.front_in = in;
@@ -317,6 +320,7 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
             w.count_mid = two ? d->counts + k + 1 : nullptr;
             w.count_out = d->counts + o + 1;
             w.cap_out = d->front_cap;
+            w.wgs_long = (d->step_walk[k] & 4u) && !d->stream ? 4u * (uint32_t)std::max(1, c->cus) : 0u;
             w.done = (!narrow && !tail && o + 1 == T) ? done : nullptr;
             HIPCHK(c, oi_launch_bvtt_walk(st, (uint32_t)std::max(1, c->cus) * 2u, &d->tab, &w, d->cands,
                                           &d->ctl->cands, d->cand_cap, d->hits, d->hits_cap, d->ctl, d->implicit_end,

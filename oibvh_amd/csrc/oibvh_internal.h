@@ -290,7 +290,7 @@ struct oi_detector {
     uint32_t depth = 0, expand = 1, flags = 0, implicit_end = 0;
     uint32_t schedule = 0;      // levels per step of the first steps (2 bits each), then `expand`
     uint8_t step_e[256] = {};   // levels descended by each step of the current query
-    uint8_t step_walk[256] = {};  // 1 or 2: step k (and k + 1) as one k_bvtt_walk launch
+    uint8_t step_walk[256] = {};  // 1 or 2: step k (and k + 1) as one k_bvtt_walk launch; + 4: long
     uint32_t local_chunk = 0;   // this query: initial pairs per workgroup of the local walk (0: steps)
     uint32_t local_levels = 0;  // this query: steps done by the local walk
     uint64_t local_off = 0;     // 1 + the tuning generation in which the head walk overflowed (0: none)

@@ -788,6 +788,25 @@ def test_detect_walk_dense_and_sparse(api, ctx, orc, expand, mode):
 
 
 @pytest.mark.parametrize("mode", ["fp32", "separate", "fp64"])
+def test_detect_walk_long_front(api, ctx, orc, mode):
+    """A walk over a front of more than 16,384 pairs (all of a launch's workgroups),
+    one and two steps a launch, and one guessed that long with far fewer pairs (a
+    share of them): the oracle's pairs."""
+    say(f"detect walk long {mode}")
+    fp64 = mode == "fp64"
+    a = M.icosphere(5, 1.0, 0.0, 0)
+    far = (M.icosphere(5, 1.0, 0.0, 1)[0] + np.float32(1.9), a[1])
+    ctx.set_tuning(narrow_separate=1 if mode == "separate" else 0)
+    try:
+        for meshes, entry in (([a, a], 5), ([a, a], 7), ([a, far], 5)):
+            p, st, trees = gpu_pairs(api, ctx, meshes, entry, 3, fp64=fp64)
+            want = orc.detect([orc.Tree(x, f, order=t.perm()) for (x, f), t in zip(meshes, trees)], fp64=fp64)
+            assert np.array_equal(p, want), entry
+    finally:
+        ctx.set_tuning(narrow_separate=0)
+
+
+@pytest.mark.parametrize("mode", ["fp32", "separate", "fp64"])
 @pytest.mark.parametrize("expand", [1, 2, 3])
 def test_detect_steps_dense_and_sparse(api, ctx, orc, expand, mode):
     """Long fronts (k_bvtt_step from an entry level of 2^8 nodes a tree and
