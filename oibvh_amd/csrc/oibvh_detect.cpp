@@ -109,6 +109,8 @@ void oi_det_free(oi_detector* d)
     dfree(d->d_stage);
     dfree(d->ctl_base);
     d->ctl = nullptr;
+    if (d->h_pairs) (void)hipHostFree(d->h_pairs);
+    d->h_pairs = nullptr;
     if (d->h_pub) (void)hipHostFree(d->h_pub);
     d->h_pub = nullptr;
 }
@@ -530,7 +532,9 @@ static uint32_t bits_for(uint32_t max_value)
 // into a 64-bit key, or the list is short, oibvh_pairs.hip sorts it, else LSD
 // radix passes over the bytes that can be non-zero sort hit indices with keys
 // looked up by index, then one gather.
-static oibvh_status sort_hits(oi_detector* d)
+// host (null, or room for OI_PAIRS_RANK_MAX pairs in pinned memory) receives a list
+// of at most that length too, once the stream has run.
+static oibvh_status sort_hits(oi_detector* d, uint4* host = nullptr)
 {
     oibvh_ctx* c = d->ctx;
     const uint32_t n = d->n_pairs;
@@ -546,7 +550,7 @@ static oibvh_status sort_hits(oi_detector* d)
         const oi_pair_bits bits{mbits, tbits};
         if ((r = grow(c, d->d_sorted, d->d_sorted_cap, n, gen)) != OIBVH_OK) return r;
         if (n <= OI_PAIRS_RANK_MAX) {
-            HIPCHK(c, oi_launch_pairs_rank(c->stream, d->hits, n, bits, wide, d->d_sorted));
+            HIPCHK(c, oi_launch_pairs_rank(c->stream, d->hits, n, bits, wide, d->d_sorted, host));
         } else {
             if (d->sort_mem_cap < oi_pairs_sort_bytes(n)) {
                 // sized with headroom, so that the next queries rarely grow it
@@ -618,6 +622,18 @@ oibvh_status oi_det_get_pairs(oi_detector* d, uint32_t* out, uint64_t cap, uint3
     if (n) *n = d->n_pairs;
     if (d->n_pairs == 0) return OIBVH_OK;
     if (!out || cap < d->n_pairs) return oi_set_err(c, OIBVH_ERR_CAPACITY, "need %u pairs", d->n_pairs);
+    if (!d->sorted_ok && d->n_pairs <= OI_PAIRS_RANK_MAX) {
+        // a short list is written to pinned memory by the launch that ranks it; a copy
+        // and the wait for it took 10 us more with 107 pairs, 40 with 1,500 (16 KB and
+        // more are staged)
+        if (!d->h_pairs)
+            HIPCHK(c, hipHostMalloc((void**)&d->h_pairs, OI_PAIRS_RANK_MAX * sizeof(uint4),
+                                    hipHostMallocCoherent | hipHostMallocMapped));
+        if ((r = sort_hits(d, d->h_pairs)) != OIBVH_OK) return r;
+        if ((r = finish(d)) != OIBVH_OK) return r;
+        std::memcpy(out, d->h_pairs, d->n_pairs * sizeof(uint4));
+        return OIBVH_OK;
+    }
     if ((r = sort_hits(d)) != OIBVH_OK) return r;
     HIPCHK(c, hipMemcpyAsync(out, d->d_sorted, d->n_pairs * sizeof(uint4), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -84,7 +84,7 @@ hipError_t oi_launch_pair_vertices(hipStream_t, const oi_build_desc*, const uint
 hipError_t oi_launch_zero_u32(hipStream_t, uint32_t*, uint32_t);
 hipError_t oi_launch_hits_digits(hipStream_t, const uint4*, uint32_t, uint32_t*, uint32_t*, const oi_hit_digits*);
 hipError_t oi_launch_hits_gather(hipStream_t, const uint4*, const uint32_t*, uint32_t, uint4*);
-hipError_t oi_launch_pairs_rank(hipStream_t, const uint4*, uint32_t, oi_pair_bits, int, uint4*);
+hipError_t oi_launch_pairs_rank(hipStream_t, const uint4*, uint32_t, oi_pair_bits, int, uint4*, uint4*);
 uint64_t oi_pairs_sort_bytes(uint32_t);
 hipError_t oi_launch_pairs_sort(hipStream_t, const uint4*, uint32_t, oi_pair_bits, void*, uint4*);
 }
@@ -282,6 +282,7 @@ struct oi_detector {
     // overflows, so that a set does not overflow where another already did)
     uint32_t want_front = 0, want_cands = 0, want_hits = 0;
     oi_detect_ctl* ctl = nullptr;    // counters of the current set
+    uint4* h_pairs = nullptr;        // pinned, at the first use: a short pair list on its way to host memory
     oi_published* h_pub = nullptr;   // pinned: what the last check read (h_pub->seq == pub_seq once it has landed)
     uint32_t pub_seq = 0;
     std::vector<uint32_t> h_counts;

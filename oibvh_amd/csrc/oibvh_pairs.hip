@@ -117,7 +117,8 @@ __device__ __forceinline__ void count_below(const Load& load, uint32_t n, const 
 // CU, a barrier chain per pass).
 template <class K>
 __global__ void __launch_bounds__(PR_THREADS)
-k_pairs_rank(const uint4* __restrict__ hits, uint32_t n, oi_pair_bits bits, uint32_t lgh, uint4* __restrict__ out)
+k_pairs_rank(const uint4* __restrict__ hits, uint32_t n, oi_pair_bits bits, uint32_t lgh, uint4* __restrict__ out,
+             uint4* __restrict__ host)
 {
     __shared__ K s_key[PR_TILE];
     __shared__ uint32_t s_rank[64];
@@ -126,8 +127,13 @@ k_pairs_rank(const uint4* __restrict__ hits, uint32_t n, oi_pair_bits bits, uint
     count_below<K>([&](uint32_t i) { return K::of(load_hit(hits, i), bits); }, n, K::of(h0, bits), K::of(h1, bits), lgh,
                    s_key, s_rank);
     if (threadIdx.x < H) {
-        if (i0 < n) out[s_rank[threadIdx.x]] = h0;
-        if (i0 + H < n) out[s_rank[H + threadIdx.x]] = h1;
+        const uint32_t r0 = s_rank[threadIdx.x], r1 = s_rank[H + threadIdx.x];
+        if (i0 < n) out[r0] = h0;
+        if (i0 + H < n) out[r1] = h1;
+        if (host) {
+            if (i0 < n) host[r0] = h0;
+            if (i0 + H < n) host[r1] = h1;
+        }
     }
 }
 
@@ -329,14 +335,18 @@ static uint32_t rank_lgh(uint32_t n)
 extern "C" {
 
 // wide: the keys' bits do not fit into 64
-hipError_t oi_launch_pairs_rank(hipStream_t st, const uint4* hits, uint32_t n, oi_pair_bits bits, int wide, uint4* out)
+// host: pinned memory that receives the list too, or null
+hipError_t oi_launch_pairs_rank(hipStream_t st, const uint4* hits, uint32_t n, oi_pair_bits bits, int wide, uint4* out,
+                                uint4* host)
 {
     if (n == 0) return hipSuccess;
     const uint32_t lgh = rank_lgh(n), grid = (n + (2u << lgh) - 1u) >> (lgh + 1u);
     if (wide)
-        hipLaunchKernelGGL(k_pairs_rank<Key128>, dim3(grid), dim3(PR_THREADS), 0, st, hits, n, bits, lgh, out);
+        hipLaunchKernelGGL(k_pairs_rank<Key128>, dim3(grid), dim3(PR_THREADS), 0, st, hits, n, bits, lgh, out,
+                           host);
     else
-        hipLaunchKernelGGL(k_pairs_rank<Key64>, dim3(grid), dim3(PR_THREADS), 0, st, hits, n, bits, lgh, out);
+        hipLaunchKernelGGL(k_pairs_rank<Key64>, dim3(grid), dim3(PR_THREADS), 0, st, hits, n, bits, lgh, out,
+                           host);
     return hipGetLastError();
 }
 

@@ -1284,6 +1284,29 @@ def test_pairs_sorted_lengths(api, ctx, orc, subdiv):
     assert np.array_equal(sc.getIntTriPairs(), want)
 
 
+@pytest.mark.parametrize("subdiv", [0, 2, 3])
+def test_pairs_read_in_any_order(api, ctx, orc, subdiv):
+    """Short and longer pair lists read to the host first, after the device list,
+    twice, and again for another pose: always the query's own pairs."""
+    say(f"pair list read order, subdiv {subdiv}")
+    x, f = M.icosphere(subdiv, 1.0, 0.0, 0)
+    t = [gpu_tree(api, ctx, x, f), gpu_tree(api, ctx, x, f)]
+    sc = api.Scene(ctx)
+    for v in t:
+        sc.addOibvhTree(v)
+    for shift, device_first in ((0.0, False), (0.3, True), (0.0, True), (0.6, False)):
+        y = x + np.float32(shift)
+        t[1].refit(y)
+        sc.detectCollision(0, 2)
+        want = orc.detect([orc.Tree(x, f, order=t[0].perm()), orc.Tree(y, f, order=t[1].perm())])
+        assert len(want) > 0
+        if device_first:
+            assert sc.pairs_device()[1] == len(want)
+        for _ in range(2):
+            assert np.array_equal(sc.getIntTriPairs(), want), (shift, device_first)
+        assert sc.pairs_device()[1] == len(want)
+
+
 def test_pairs_sorted_wide_keys(api, ctx, orc):
     """Ids that do not fit into a 64-bit key (301 trees: 9 bits, one of them
     of more than 2^23 faces: 24 bits) are compared as 128 bits."""
