@@ -69,6 +69,22 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s_wsum
 // Meshes come from a device table with a work list, or (d = null) travel in
 // the kernel arguments: up to OI_INLINE_MESHES meshes, mesh m owning the
 // workgroups [boff[m], boff[m + 1]).
+// The mesh is read by its index with scalar loads, from the table or from the
+// argument segment (the table is the kernel's first argument): indexing the argument
+// itself would put a copy of it into scratch memory, and picked from copies in
+// registers the descriptor took 28 VGPRs of k_reduce_w (109 -> 81, so that six waves
+// a SIMD fit instead of four: 128 instanced scenes, 4 frames, 5,136 -> 4,923 us).
+typedef const __attribute__((address_space(4))) uint32_t* args_t;
+__device__ __forceinline__ oi_build_desc uniform_desc(args_t a)
+{
+    uint32_t w[sizeof(oi_build_desc) / 4u];
+#pragma unroll
+    for (uint32_t k = 0; k < sizeof(oi_build_desc) / 4u; k++) w[k] = a[k];
+    oi_build_desc d;
+    __builtin_memcpy(&d, w, sizeof d);
+    return d;
+}
+
 #define OI_INLINE_MESHES 4
 struct BuildTab {
     const oi_build_desc* d;  // device table, or null
@@ -92,14 +108,39 @@ struct BuildTab {
     }
     __device__ __forceinline__ oi_build_desc mesh(uint32_t m) const
     {
-        if (d) return d[m];
-        // constant indices keep the argument block out of scratch memory
-        switch (m) {
-        case 0: return inl[0];
-        case 1: return inl[1];
-        case 2: return inl[2];
-        default: return inl[3];
-        }
+        m = (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
+        return uniform_desc(d ? (args_t)(d + m) : (args_t)__builtin_amdgcn_kernarg_segment_ptr() +
+                                                      (offsetof(BuildTab, inl) + m * sizeof(oi_build_desc)) / 4u);
+    }
+};
+
+// Up to OI_WIDE_MESHES meshes in the kernel arguments, for a refit's launches: one
+// pair for 16 trees instead of four (16 moving bodies 253 -> 216 us a frame, five 127
+// -> 117). A table of its own, so that four trees and fewer pass a quarter of the
+// bytes.
+#define OI_WIDE_MESHES 16
+struct WideTab {
+    uint32_t n;
+    uint32_t boff[OI_WIDE_MESHES + 1];
+    oi_build_desc inl[OI_WIDE_MESHES];
+    __device__ __forceinline__ uint2 item() const { return item_at(blockIdx.x, gridDim.x); }
+    __device__ __forceinline__ uint2 item_at(uint32_t v, uint32_t total) const
+    {
+        const uint32_t w = oi_xcd_remap(v, total);
+        uint32_t m = 0, first = 0;
+#pragma unroll
+        for (uint32_t k = 1; k < OI_WIDE_MESHES; k++)
+            if (k < n && w >= boff[k]) {
+                m = k;
+                first = boff[k];
+            }
+        return make_uint2(m, w - first);
+    }
+    __device__ __forceinline__ oi_build_desc mesh(uint32_t m) const
+    {
+        m = (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
+        return uniform_desc((args_t)__builtin_amdgcn_kernarg_segment_ptr() +
+                            (offsetof(WideTab, inl) + m * sizeof(oi_build_desc)) / 4u);
     }
 };
 
@@ -719,8 +760,9 @@ __device__ __forceinline__ Box6 load_node(const float* nodes, uint32_t r)
     return o;
 }
 
+template <class Tab>
 struct ReduceArgs {
-    BuildTab T;
+    Tab T;  // first (WideTab)
     const uint32_t* vals;  // build: Morton-sorted face ids (fbase + face); null: refit over sfaces
     uint32_t write_perm;   // build: also write perm (faces local to the mesh)
     uint32_t nwork;        // k_reduce_w: work items (0: one per workgroup)
@@ -884,8 +926,8 @@ __device__ void reduce_subtree(const Load& load, float* nodes, uint32_t L, uint3
     __syncthreads();
 }
 
-template <int M>
-__global__ void __launch_bounds__(OI_BLOCK) k_reduce(ReduceArgs a)
+template <int M, class Tab>
+__global__ void __launch_bounds__(OI_BLOCK) k_reduce(ReduceArgs<Tab> a)
 {
     __shared__ float stage[StageSize<M>::floats];
     constexpr uint32_t LGM = (M == 1) ? 0 : (M == 2) ? 1 : (M == 4) ? 2 : 3;
@@ -1029,8 +1071,8 @@ __device__ __forceinline__ void wave_boxes(const oi_build_desc& D, uint32_t f0, 
 // issued before any box is formed. BUILD reads the sorted face ids and writes
 // sfaces and perm; XF applies the model matrix. Both are compile-time, so the
 // loads form one straight run.
-template <bool BUILD, bool XF>
-__device__ __forceinline__ void wave_leaves(const ReduceArgs& A, const oi_build_desc& D, uint32_t f0, uint32_t hw,
+template <bool BUILD, bool XF, class Tab>
+__device__ __forceinline__ void wave_leaves(const ReduceArgs<Tab>& A, const oi_build_desc& D, uint32_t f0, uint32_t hw,
                                             uint32_t nleaf, uint32_t lane, float* stage)
 {
     constexpr int K = RW_W / 64;
@@ -1149,7 +1191,8 @@ struct WaveItem {
     uint32_t hw, hb, f0, nleaf;
     bool on;  // this wave owns leaves of the item
 };
-__device__ __forceinline__ WaveItem wave_item(const ReduceArgs& A, uint2 it, uint32_t wave)
+template <class Tab>
+__device__ __forceinline__ WaveItem wave_item(const ReduceArgs<Tab>& A, uint2 it, uint32_t wave)
 {
     WaveItem w;
     w.D = A.T.mesh(it.x);
@@ -1163,7 +1206,8 @@ __device__ __forceinline__ WaveItem wave_item(const ReduceArgs& A, uint2 it, uin
 }
 
 // one work item; S is the workgroup's staging, free again on return
-__device__ __forceinline__ void reduce_w_item(const ReduceArgs& A, uint2 it, float (*S)[6 * RW_W])
+template <class Tab>
+__device__ __forceinline__ void reduce_w_item(const ReduceArgs<Tab>& A, uint2 it, float (*S)[6 * RW_W])
 {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const WaveItem w = wave_item(A, it, wave);
@@ -1188,7 +1232,8 @@ __device__ __forceinline__ void reduce_w_item(const ReduceArgs& A, uint2 it, flo
     item_top(D, it, w.hw, w.hb, S);
 }
 
-__global__ void __launch_bounds__(OI_BLOCK) k_reduce_w(ReduceArgs A)
+template <class Tab>
+__global__ void __launch_bounds__(OI_BLOCK) k_reduce_w(ReduceArgs<Tab> A)
 {
     __shared__ float S[OI_BLOCK / 64][6 * RW_W];
     reduce_w_item(A, A.T.item(), S);
@@ -1201,7 +1246,8 @@ __global__ void __launch_bounds__(OI_BLOCK) k_reduce_w(ReduceArgs A)
 // registers. (Loading the next item's faces before the current item's
 // vertices was measured: the refit was no faster beside a detect, and the
 // detect slower.)
-__global__ void __launch_bounds__(OI_BLOCK) k_reduce_wl(ReduceArgs A)
+template <class Tab>
+__global__ void __launch_bounds__(OI_BLOCK) k_reduce_wl(ReduceArgs<Tab> A)
 {
     __shared__ float S[OI_BLOCK / 64][6 * RW_W];
     for (uint32_t v = blockIdx.x; v < A.nwork; v += gridDim.x) {
@@ -1237,7 +1283,8 @@ __device__ __forceinline__ void seed_counters(const oi_seed_args& s)
 // are numbered through the XCD remap (BuildTab::item), so the extra workgroup
 // is the one whose remapped index is the last: the others then cover exactly
 // the items 0 .. n - 1 of the work list.
-__global__ void __launch_bounds__(OI_BLOCK) k_reduce_apex(ReduceArgs a, uint32_t lgm, oi_seed_args seed)
+template <class Tab>
+__global__ void __launch_bounds__(OI_BLOCK) k_reduce_apex(ReduceArgs<Tab> a, uint32_t lgm, oi_seed_args seed)
 {
     __shared__ float stage[StageSize<8>::floats];
     if (seed.counts && oi_xcd_remap(blockIdx.x, gridDim.x) == gridDim.x - 1) {
@@ -1311,6 +1358,19 @@ static BuildTab make_btab_inline(const oi_build_desc* meshes, uint32_t n, const 
         t.boff[m] = boff[m];
     }
     t.boff[n < OI_INLINE_MESHES ? n : OI_INLINE_MESHES] = boff[n];
+    return t;
+}
+
+// n (<= OI_WIDE_MESHES) meshes, as make_btab_inline
+static WideTab make_wide(const oi_build_desc* meshes, uint32_t n, const uint32_t* boff)
+{
+    WideTab t{};
+    t.n = n;
+    for (uint32_t m = 0; m < n && m < OI_WIDE_MESHES; m++) {
+        t.inl[m] = meshes[m];
+        t.boff[m] = boff[m];
+    }
+    t.boff[n < OI_WIDE_MESHES ? n : OI_WIDE_MESHES] = boff[n];
     return t;
 }
 
@@ -1521,6 +1581,55 @@ uint32_t oi_reduce_height(int M, uint32_t L)
     return (L < 8 + lgm) ? L : 8 + lgm;
 }
 
+}  // extern "C"
+
+template <class Tab>
+static hipError_t launch_reduce(hipStream_t st, int M, ReduceArgs<Tab> a, uint32_t nblocks, hipEvent_t t0,
+                                hipEvent_t t1, uint32_t max_blocks)
+{
+    if (!t0 != !t1) return hipErrorInvalidValue;
+    dim3 g(nblocks);
+    const dim3 b(OI_BLOCK);
+    if (M == 16 && !a.vals && max_blocks && max_blocks < nblocks) {
+        const uint32_t cap = (max_blocks + 7u) & ~7u;
+        if (cap < nblocks) {
+            a.nwork = nblocks;
+            g = dim3(cap);
+        }
+    }
+    switch (M) {
+    case 1: launch_timed((k_reduce<1, Tab>), g, b, st, t0, t1, a); break;
+    case 2: launch_timed((k_reduce<2, Tab>), g, b, st, t0, t1, a); break;
+    case 4: launch_timed((k_reduce<4, Tab>), g, b, st, t0, t1, a); break;
+    case 16:
+        if (a.nwork)
+            launch_timed((k_reduce_wl<Tab>), g, b, st, t0, t1, a);
+        else
+            launch_timed((k_reduce_w<Tab>), g, b, st, t0, t1, a);
+        break;
+    default: launch_timed((k_reduce<8, Tab>), g, b, st, t0, t1, a); break;
+    }
+    return hipGetLastError();
+}
+
+template <class Tab>
+static hipError_t launch_apex(hipStream_t st, int M, const Tab& t, uint32_t n, const oi_seed_args* seed,
+                              hipEvent_t done)
+{
+    if (seed && seed->n_counts > OI_BLOCK) return hipErrorInvalidValue;
+    const ReduceArgs<Tab> a{t, nullptr, 0, 0};
+    const oi_seed_args sd = seed ? *seed : oi_seed_args{};
+    const dim3 g(n + (seed ? 1u : 0u)), b(OI_BLOCK);
+    // with done the launch records it on completion (no separate event call)
+    if (done)
+        hipExtLaunchKernelGGL((k_reduce_apex<Tab>), g, b, 0, st, nullptr, done, 0, a, lgm_of(M), sd);
+    else
+        hipLaunchKernelGGL((k_reduce_apex<Tab>), g, b, 0, st, a, lgm_of(M), sd);
+    return hipGetLastError();
+}
+
+extern "C" {
+
 // stage 1 (M = leaves per thread: 1, 2, 4 or 8; 16: wave subtrees); vals:
 // build, null: refit. With t0 and t1 (both or neither) the launch records
 // them as it starts and completes. max_blocks > 0 (refits with M = 16 only):
@@ -1530,35 +1639,14 @@ hipError_t oi_launch_reduce(hipStream_t st, int M, const oi_build_desc* d, const
                             const oi_build_desc* one, uint32_t nblocks, const uint32_t* vals, uint32_t write_perm,
                             hipEvent_t t0, hipEvent_t t1, uint32_t max_blocks)
 {
-    if (!t0 != !t1) return hipErrorInvalidValue;
-    ReduceArgs a{make_btab(d, work, one), vals, write_perm};
-    dim3 g(nblocks);
-    const dim3 b(OI_BLOCK);
-    if (M == 16 && !vals && max_blocks && max_blocks < nblocks) {
-        const uint32_t cap = (max_blocks + 7u) & ~7u;
-        if (cap < nblocks) {
-            a.nwork = nblocks;
-            g = dim3(cap);
-        }
-    }
-    switch (M) {
-    case 1: launch_timed(k_reduce<1>, g, b, st, t0, t1, a); break;
-    case 2: launch_timed(k_reduce<2>, g, b, st, t0, t1, a); break;
-    case 4: launch_timed(k_reduce<4>, g, b, st, t0, t1, a); break;
-    case 16:
-        if (a.nwork)
-            launch_timed(k_reduce_wl, g, b, st, t0, t1, a);
-        else
-            launch_timed(k_reduce_w, g, b, st, t0, t1, a);
-        break;
-    default: launch_timed(k_reduce<8>, g, b, st, t0, t1, a); break;
-    }
-    return hipGetLastError();
+    return launch_reduce(st, M, ReduceArgs<BuildTab>{make_btab(d, work, one), vals, write_perm, 0}, nblocks, t0, t1,
+                         max_blocks);
 }
 
 uint32_t oi_inline_meshes() { return OI_INLINE_MESHES; }
+uint32_t oi_wide_meshes() { return OI_WIDE_MESHES; }
 
-// stage 1 over up to OI_INLINE_MESHES meshes passed by value; boff[n + 1]
+// stage 1 over up to OI_WIDE_MESHES meshes passed by value; boff[n + 1]
 // gives each mesh's first workgroup
 // with t0 and t1 (both or neither) the launch itself records them as it
 // starts and completes: their elapsed time is the kernel's own duration.
@@ -1569,31 +1657,12 @@ hipError_t oi_launch_reduce_inline(hipStream_t st, int M, const oi_build_desc* m
                                    const uint32_t* boff, const uint32_t* vals, uint32_t write_perm, hipEvent_t t0,
                                    hipEvent_t t1, uint32_t max_blocks)
 {
-    if (n == 0 || n > OI_INLINE_MESHES) return hipErrorInvalidValue;
-    if (!t0 != !t1) return hipErrorInvalidValue;
-    ReduceArgs a{make_btab_inline(meshes, n, boff), vals, write_perm};
-    dim3 g(boff[n]);
-    const dim3 b(OI_BLOCK);
-    if (M == 16 && !vals && max_blocks && max_blocks < boff[n]) {
-        const uint32_t cap = (max_blocks + 7u) & ~7u;
-        if (cap < boff[n]) {
-            a.nwork = boff[n];
-            g = dim3(cap);
-        }
-    }
-    switch (M) {
-    case 1: launch_timed(k_reduce<1>, g, b, st, t0, t1, a); break;
-    case 2: launch_timed(k_reduce<2>, g, b, st, t0, t1, a); break;
-    case 4: launch_timed(k_reduce<4>, g, b, st, t0, t1, a); break;
-    case 16:
-        if (a.nwork)
-            launch_timed(k_reduce_wl, g, b, st, t0, t1, a);
-        else
-            launch_timed(k_reduce_w, g, b, st, t0, t1, a);
-        break;
-    default: launch_timed(k_reduce<8>, g, b, st, t0, t1, a); break;
-    }
-    return hipGetLastError();
+    if (n == 0 || n > OI_WIDE_MESHES) return hipErrorInvalidValue;
+    if (n <= OI_INLINE_MESHES)
+        return launch_reduce(st, M, ReduceArgs<BuildTab>{make_btab_inline(meshes, n, boff), vals, write_perm, 0},
+                             boff[n], t0, t1, max_blocks);
+    return launch_reduce(st, M, ReduceArgs<WideTab>{make_wide(meshes, n, boff), vals, write_perm, 0}, boff[n], t0, t1,
+                         max_blocks);
 }
 
 // stage 2 for n inline meshes, one workgroup each; with seed (may be null)
@@ -1601,32 +1670,18 @@ hipError_t oi_launch_reduce_inline(hipStream_t st, int M, const oi_build_desc* m
 hipError_t oi_launch_reduce_apex_inline(hipStream_t st, int M, const oi_build_desc* meshes, uint32_t n,
                                         const oi_seed_args* seed, hipEvent_t done)
 {
-    if (n == 0 || n > OI_INLINE_MESHES) return hipErrorInvalidValue;
-    if (seed && seed->n_counts > OI_BLOCK) return hipErrorInvalidValue;
-    uint32_t boff[OI_INLINE_MESHES + 1];
+    if (n == 0 || n > OI_WIDE_MESHES) return hipErrorInvalidValue;
+    uint32_t boff[OI_WIDE_MESHES + 1];
     for (uint32_t m = 0; m <= n; m++) boff[m] = m;
-    ReduceArgs a{make_btab_inline(meshes, n, boff), nullptr, 0};
-    const uint32_t lgm = lgm_of(M);
-    const oi_seed_args sd = seed ? *seed : oi_seed_args{};
-    // with done the launch records it on completion (no separate event call)
-    if (done)
-        hipExtLaunchKernelGGL(k_reduce_apex, dim3(n + (seed ? 1u : 0u)), dim3(OI_BLOCK), 0, st, nullptr, done, 0, a,
-                              lgm, sd);
-    else
-        hipLaunchKernelGGL(k_reduce_apex, dim3(n + (seed ? 1u : 0u)), dim3(OI_BLOCK), 0, st, a, lgm, sd);
-    return hipGetLastError();
+    if (n <= OI_INLINE_MESHES) return launch_apex(st, M, make_btab_inline(meshes, n, boff), n, seed, done);
+    return launch_apex(st, M, make_wide(meshes, n, boff), n, seed, done);
 }
 
 // stage 2, one workgroup per work item (mesh, 0) whose L exceeds the stage-1 height
 hipError_t oi_launch_reduce_apex(hipStream_t st, int M, const oi_build_desc* d, const uint2* work,
                                  const oi_build_desc* one, uint32_t nblocks, const oi_seed_args* seed)
 {
-    if (seed && seed->n_counts > OI_BLOCK) return hipErrorInvalidValue;
-    ReduceArgs a{make_btab(d, work, one), nullptr, 0};
-    const uint32_t lgm = lgm_of(M);
-    const oi_seed_args sd = seed ? *seed : oi_seed_args{};
-    hipLaunchKernelGGL(k_reduce_apex, dim3(nblocks + (seed ? 1u : 0u)), dim3(OI_BLOCK), 0, st, a, lgm, sd);
-    return hipGetLastError();
+    return launch_apex(st, M, make_btab(d, work, one), nblocks, seed, nullptr);
 }
 
 }  // extern "C"

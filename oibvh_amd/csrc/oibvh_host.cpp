@@ -971,11 +971,12 @@ extern "C" oibvh_status oibvh_scene_set_transforms(oibvh_scene* s, const float* 
     return OIBVH_OK;
 }
 
-// Every tree of the scene refit at once: up to four trees per launch pair
+// Every tree of the scene refit at once: up to 16 trees per launch pair
 // (their descriptors travel in the kernel arguments), so the reduce fills the
 // GPU once instead of once per tree. Same results as oibvh_tree_refit on each.
 // the scene refit; with seed, the last apex launch (if there is one) also
 // resets the counters of the detect that follows, and *seeded says so
+#define OI_REFIT_GROUP 16
 static oibvh_status scene_refit(oibvh_scene* s, const oi_seed_args* seed, bool* seeded, hipEvent_t done = nullptr)
 {
     oibvh_ctx* c = s->ctx;
@@ -983,15 +984,15 @@ static oibvh_status scene_refit(oibvh_scene* s, const oi_seed_args* seed, bool* 
     HIPCHK(c, hipSetDevice(c->device));
     for (oibvh_tree* t : s->trees)
         if (!t->built) return oi_set_err(c, OIBVH_ERR_NOT_BUILT, "scene refit: tree not built");
-    const uint32_t per = oi_inline_meshes();
+    const uint32_t per = std::min<uint32_t>(OI_REFIT_GROUP, oi_wide_meshes());
     for (size_t i0 = 0; i0 < s->trees.size(); i0 += per) {
         const uint32_t n = (uint32_t)std::min<size_t>(per, s->trees.size() - i0);
         uint64_t F = 0;
         for (uint32_t k = 0; k < n; k++) F += s->trees[i0 + k]->F;
         int M = (int)c->leaves_per_thread;
         if (!M) M = oi_default_lpt(F, c->cus);
-        oi_build_desc d[8], apex[8];
-        uint32_t boff[9], na = 0;
+        oi_build_desc d[OI_REFIT_GROUP], apex[OI_REFIT_GROUP];
+        uint32_t boff[OI_REFIT_GROUP + 1], na = 0;
         boff[0] = 0;
         for (uint32_t k = 0; k < n; k++) {
             const oibvh_tree* t = s->trees[i0 + k];

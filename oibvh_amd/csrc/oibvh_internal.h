@@ -63,6 +63,7 @@ hipError_t oi_launch_reduce_apex(hipStream_t, int, const oi_build_desc*, const u
                                  uint32_t, const oi_seed_args*);
 hipError_t oi_launch_set_xf(hipStream_t, float*, const float*);
 uint32_t oi_inline_meshes();
+uint32_t oi_wide_meshes();  // of the refit's launches (oi_launch_reduce_inline, oi_launch_reduce_apex_inline)
 hipError_t oi_launch_reduce_inline(hipStream_t, int, const oi_build_desc*, uint32_t, const uint32_t*, const uint32_t*,
                                    uint32_t, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr,
                                    uint32_t max_blocks = 0);

@@ -1326,6 +1326,40 @@ def test_pairs_sorted_wide_keys(api, ctx, orc):
     assert np.array_equal(sc.getIntTriPairs(), want)
 
 
+@pytest.mark.parametrize("lpt", [0, 1, 8, 16])
+@pytest.mark.parametrize("n", [4, 5, 16, 17, 33])
+def test_scene_refit_groups(api, ctx, orc, n, lpt):
+    """A scene's refit in launches of up to 16 trees (descriptors in the kernel
+    arguments, four and fewer in the small table): trees of one face to 40,001,
+    some with a model matrix, end with the nodes their own refit gives them."""
+    say(f"scene refit groups n={n} lpt={lpt}")
+    sizes = [(1, 40001, 3, 257, 2049, 9000, 2)[i % 7] + i // 7 for i in range(n)]
+    meshes = [soup(F, 700 + i) for i, F in enumerate(sizes)]
+    ctx.set_tuning(reduce_leaves_per_thread=lpt)
+    try:
+        trees = []
+        for i, (x, f) in enumerate(meshes):
+            t = api.OibvhTree(ctx, x, f)
+            if i % 3 == 1:
+                t.set_transform(_motion(2 + i, i))
+            t.build()
+            trees.append(t)
+        sc = api.Scene(ctx)
+        for t in trees:
+            sc.addOibvhTree(t)
+        for t, (x, _) in zip(trees, meshes):
+            t.refit(np.ascontiguousarray(-x[::-1]).astype(np.float32))
+        want = [bits(t.nodes()).copy() for t in trees]
+        for t, (x, _) in zip(trees, meshes):
+            t.refit(x)  # other nodes again
+            t.set_positions(np.ascontiguousarray(-x[::-1]).astype(np.float32))
+        sc.refit()
+        for i, (t, w) in enumerate(zip(trees, want)):
+            assert np.array_equal(bits(t.nodes()), w), (i, sizes[i])
+    finally:
+        ctx.set_tuning(reduce_leaves_per_thread=0)
+
+
 def test_scene_build_equals_tree_builds(api, ctx, orc):
     """oibvh_scene_build (the trees sharing each launch of the build chain)
     gives every tree what oibvh_tree_build gives it: leaf order, sorted faces
