@@ -1415,6 +1415,12 @@ extern "C" oibvh_status oibvh_scene_get_pair_vertices(oibvh_scene* s, float* out
     HIPCHK(c, hipSetDevice(c->device));
     HIPCHK(c, oi_ctx_join(c));
     const uint32_t nt = (uint32_t)s->trees.size();
+    // an asynchronous detect not yet checked has no pair count: without it the
+    // geometry table below would be missing or an earlier query's
+    if (ptr_kind == OIBVH_PTR_HOST || ptr_kind == OIBVH_PTR_DEVICE) {
+        const oibvh_status r = oi_det_check(&s->det);
+        if (r != OIBVH_OK) return r;
+    }
     if (s->det.have_result && s->det.n_pairs && nt) {
         std::vector<oi_build_desc> g(nt);
         for (uint32_t m = 0; m < nt; m++) g[m] = tree_desc(s->trees[m]);

@@ -269,6 +269,31 @@ def test_pair_vertices_export(api, ctx, orc):
     assert np.array_equal(bits(sc2.pair_vertices()), bits(expected_pair_vertices(p2, [(x0, f0)])))
 
 
+def test_pair_vertices_of_an_unchecked_detect(api, ctx, orc):
+    """The export as the first call after an asynchronous detect, on a new scene
+    and after a query without pairs."""
+    say("pair vertex export, unchecked detect")
+    (x0, f0), (x1, f1) = M.interpenetrating_icospheres(subdiv=3, offset=0.0)
+    for apart in (False, True):
+        t0, t1 = gpu_tree(api, ctx, x0, f0), gpu_tree(api, ctx, x1, f1)
+        sc = api.Scene(ctx)
+        sc.addOibvhTree(t0)
+        sc.addOibvhTree(t1)
+        if apart:
+            t1.refit(x1 + np.float32(50.0))
+            sc.detectCollision(0, 2)
+            assert sc.getIntTriPairCount() == 0
+            t1.refit(x1)
+        want = orc.detect([orc.Tree(x0, f0), orc.Tree(x1, f1, order=t1.perm())])
+        assert len(want) > 0
+        verts = expected_pair_vertices(want, [(x0, f0), (x1, f1)])
+        buf = api.DeviceBuffer(verts.nbytes)
+        sc.detectCollision(0, 2, asynchronous=True)
+        assert sc.pair_vertices_device(buf.at(0), verts.size) == len(want)
+        assert np.array_equal(bits(buf.download(np.float32, verts.size)), bits(verts.reshape(-1)))
+        buf.free()
+
+
 # --------------------------------------------------------------------- refit
 def test_refit_after_deformation(api, ctx, orc):
     say("refit deforming uv sphere")
