@@ -1269,6 +1269,22 @@ __device__ __forceinline__ void apex_chunks(const oi_build_desc& D, uint32_t lc,
     for (uint32_t c = 0; c < nchunk; c++) reduce_subtree<M>(nl, D.nodes, D.L, D.vl, lc, h2, c, stage);
 }
 
+// Stage 1 leaves more than 2^11 roots of a tree above 2M faces (APEX_MID): one
+// workgroup would climb them a chunk after the other, 9 us each. k_reduce_mid climbs
+// 8 levels in a workgroup per 256 roots first, and k_reduce_apex starts above them:
+// a frame of the folded cloth of 8.4M faces 1,695 -> 1,675 us.
+#define APEX_MID 11u
+template <class Tab>
+__global__ void __launch_bounds__(OI_BLOCK) k_reduce_mid(ReduceArgs<Tab> a, uint32_t lgm)
+{
+    __shared__ float stage[StageSize<1>::floats];
+    const uint2 it = a.T.item();
+    const oi_build_desc D = a.T.mesh(it.x);
+    const uint32_t lc = D.L - (8u + lgm);  // (launched for meshes with lc > APEX_MID)
+    NodeLoad nl{D.nodes, oi_lvl_start(lc, D.L, D.vl)};
+    reduce_subtree<1>(nl, D.nodes, D.L, D.vl, lc, 8u, it.y, stage);
+}
+
 // zeroed level counts and result counters for the detect that follows
 // (the work of the collide side's k_seed, one workgroup)
 __device__ __forceinline__ void seed_counters(const oi_seed_args& s)
@@ -1284,7 +1300,7 @@ __device__ __forceinline__ void seed_counters(const oi_seed_args& s)
 // is the one whose remapped index is the last: the others then cover exactly
 // the items 0 .. n - 1 of the work list.
 template <class Tab>
-__global__ void __launch_bounds__(OI_BLOCK) k_reduce_apex(ReduceArgs<Tab> a, uint32_t lgm, oi_seed_args seed)
+__global__ void __launch_bounds__(OI_BLOCK) k_reduce_apex(ReduceArgs<Tab> a, uint32_t lgm, uint32_t mid, oi_seed_args seed)
 {
     __shared__ float stage[StageSize<8>::floats];
     if (seed.counts && oi_xcd_remap(blockIdx.x, gridDim.x) == gridDim.x - 1) {
@@ -1296,6 +1312,7 @@ __global__ void __launch_bounds__(OI_BLOCK) k_reduce_apex(ReduceArgs<Tab> a, uin
     const uint32_t L = D.L;
     const uint32_t h = (L < 8 + lgm) ? L : 8 + lgm;
     uint32_t lc = L - h;
+    if (mid && lc > APEX_MID) lc -= 8u;  // k_reduce_mid has climbed them
     while (lc > 0) {
         const uint32_t h2 = (lc < 11u) ? lc : 11u;
         if (h2 <= 8)
@@ -1612,8 +1629,9 @@ static hipError_t launch_reduce(hipStream_t st, int M, ReduceArgs<Tab> a, uint32
     return hipGetLastError();
 }
 
+// mid: k_reduce_mid has run for the meshes that need it
 template <class Tab>
-static hipError_t launch_apex(hipStream_t st, int M, const Tab& t, uint32_t n, const oi_seed_args* seed,
+static hipError_t launch_apex(hipStream_t st, int M, const Tab& t, uint32_t n, uint32_t mid, const oi_seed_args* seed,
                               hipEvent_t done)
 {
     if (seed && seed->n_counts > OI_BLOCK) return hipErrorInvalidValue;
@@ -1622,9 +1640,32 @@ static hipError_t launch_apex(hipStream_t st, int M, const Tab& t, uint32_t n, c
     const dim3 g(n + (seed ? 1u : 0u)), b(OI_BLOCK);
     // with done the launch records it on completion (no separate event call)
     if (done)
-        hipExtLaunchKernelGGL((k_reduce_apex<Tab>), g, b, 0, st, nullptr, done, 0, a, lgm_of(M), sd);
+        hipExtLaunchKernelGGL((k_reduce_apex<Tab>), g, b, 0, st, nullptr, done, 0, a, lgm_of(M), mid, sd);
     else
-        hipLaunchKernelGGL((k_reduce_apex<Tab>), g, b, 0, st, a, lgm_of(M), sd);
+        hipLaunchKernelGGL((k_reduce_apex<Tab>), g, b, 0, st, a, lgm_of(M), mid, sd);
+    return hipGetLastError();
+}
+
+// k_reduce_mid over those of n (<= OI_WIDE_MESHES) meshes that need it
+static hipError_t launch_mid(hipStream_t st, int M, const oi_build_desc* meshes, uint32_t n)
+{
+    const uint32_t lgm = lgm_of(M);
+    oi_build_desc d[OI_WIDE_MESHES];
+    uint32_t boff[OI_WIDE_MESHES + 1] = {0}, k = 0;
+    for (uint32_t m = 0; m < n; m++) {
+        if (meshes[m].L <= 8u + lgm + APEX_MID) continue;
+        d[k] = meshes[m];
+        boff[k + 1] = boff[k] + oi_lvl_cnt(d[k].L - (8u + lgm) - 8u, d[k].L, d[k].vl);
+        k++;
+    }
+    if (k == 0) return hipSuccess;
+    const dim3 g(boff[k]), b(OI_BLOCK);
+    if (k <= OI_INLINE_MESHES)
+        hipLaunchKernelGGL((k_reduce_mid<BuildTab>), g, b, 0, st,
+                           (ReduceArgs<BuildTab>{make_btab_inline(d, k, boff), nullptr, 0, 0}), lgm);
+    else
+        hipLaunchKernelGGL((k_reduce_mid<WideTab>), g, b, 0, st,
+                           (ReduceArgs<WideTab>{make_wide(d, k, boff), nullptr, 0, 0}), lgm);
     return hipGetLastError();
 }
 
@@ -1673,15 +1714,21 @@ hipError_t oi_launch_reduce_apex_inline(hipStream_t st, int M, const oi_build_de
     if (n == 0 || n > OI_WIDE_MESHES) return hipErrorInvalidValue;
     uint32_t boff[OI_WIDE_MESHES + 1];
     for (uint32_t m = 0; m <= n; m++) boff[m] = m;
-    if (n <= OI_INLINE_MESHES) return launch_apex(st, M, make_btab_inline(meshes, n, boff), n, seed, done);
-    return launch_apex(st, M, make_wide(meshes, n, boff), n, seed, done);
+    const hipError_t e = launch_mid(st, M, meshes, n);
+    if (e != hipSuccess) return e;
+    if (n <= OI_INLINE_MESHES) return launch_apex(st, M, make_btab_inline(meshes, n, boff), n, 1, seed, done);
+    return launch_apex(st, M, make_wide(meshes, n, boff), n, 1, seed, done);
 }
 
 // stage 2, one workgroup per work item (mesh, 0) whose L exceeds the stage-1 height
 hipError_t oi_launch_reduce_apex(hipStream_t st, int M, const oi_build_desc* d, const uint2* work,
                                  const oi_build_desc* one, uint32_t nblocks, const oi_seed_args* seed)
 {
-    return launch_apex(st, M, make_btab(d, work, one), nblocks, seed, nullptr);
+    if (one) {
+        const hipError_t e = launch_mid(st, M, one, 1);
+        if (e != hipSuccess) return e;
+    }
+    return launch_apex(st, M, make_btab(d, work, one), nblocks, one ? 1u : 0u, seed, nullptr);
 }
 
 }  // extern "C"

@@ -1385,6 +1385,37 @@ def test_scene_refit_groups(api, ctx, orc, n, lpt):
         ctx.set_tuning(reduce_leaves_per_thread=0)
 
 
+@pytest.mark.parametrize("lpt, sizes", [(1, [(1 << 19) + 1]), (1, [(1 << 20) + 5, 300, 1 << 19, (1 << 19) + 77, 2, 5000]),
+                                        (2, [(1 << 20) + 1, 9]), (0, [(1 << 21) + 3])])
+def test_refit_of_large_trees(api, ctx, orc, lpt, sizes):
+    """Trees with more than 2^11 roots left by the reduce's first stage (from 2^19
+    faces with one leaf per thread, 2^21 as it runs by itself), alone and among
+    smaller ones: build, tree refit and scene refit leave the oracle's nodes."""
+    say(f"refit of large trees lpt={lpt} {sizes}")
+    meshes = [soup(F, 90 + F % 1000) for F in sizes]
+    ctx.set_tuning(reduce_leaves_per_thread=lpt)
+    try:
+        trees = [gpu_tree(api, ctx, x, f) for x, f in meshes]
+        sc = api.Scene(ctx)
+        for t, (x, f) in zip(trees, meshes):
+            sc.addOibvhTree(t)
+            check_tree(orc, t, x, f)
+        moved = [np.ascontiguousarray(x[::-1] * np.float32(0.5)) for x, _ in meshes]
+        want = [bits(orc.Tree(y, f, order=t.perm()).nodes()) for t, y, (_, f) in zip(trees, moved, meshes)]
+        for t, y, w in zip(trees, moved, want):
+            t.refit(y)
+            assert np.array_equal(bits(t.nodes()), w)
+        for t, (x, _) in zip(trees, meshes):
+            t.refit(x)
+        for t, y in zip(trees, moved):
+            t.set_positions(y)
+        sc.refit()
+        for t, w in zip(trees, want):
+            assert np.array_equal(bits(t.nodes()), w)
+    finally:
+        ctx.set_tuning(reduce_leaves_per_thread=0)
+
+
 def test_scene_build_equals_tree_builds(api, ctx, orc):
     """oibvh_scene_build (the trees sharing each launch of the build chain)
     gives every tree what oibvh_tree_build gives it: leaf order, sorted faces
