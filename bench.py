@@ -669,9 +669,12 @@ def run_deforming(args, ctx):
         tuned = tuned_alone = autotune.tune(ctx, scene, tune_frame)
         # then the walk's shape again on overlapped frames, around that pick
         keys = ("traverse_blocks", "reduce_leaves_per_thread")
-        cands = [tuned] + [{"entry_level": tuned["entry_level"], "expand_levels": x,
+        # (and from the other entry levels: the one that is best for steps and walks
+        # over short fronts is not the best one for local and tail walks)
+        cands = [tuned] + [{"entry_level": en, "expand_levels": x,
                             **{k: tuned[k] for k in keys}, "traverse_local": lc, "traverse_local_levels": ll,
                             "traverse_tail": tc, "traverse_tail_steps": 0, "narrow_separate": ns}
+                           for en in dict.fromkeys((tuned["entry_level"], 4, 8))
                            for x in (2, 3) for lc, ll in ((0, 0), (128, 3), (256, 3), (256, 2))
                            for tc in (0, 32, 64) for ns in (0, 1)]
         tuned = autotune.tune_overlapped(ctx, scene, overlapped_at, cands)

@@ -49,10 +49,11 @@ def tune(ctx: api.Context, scene: api.Scene, frame, *, entries=(4, 6, 8), expand
     'traverse_tail', 'traverse_tail_steps', 'narrow_separate', 'ms'} of the
     fastest setting and apply the tuning knobs to ctx. `local` lists the
     (initial pairs per workgroup, steps) settings of the head local walk
-    tried at the best step shape, `tail` the (front pairs per workgroup pass,
-    steps) settings of the tail walk tried after the best head setting, with
-    leaf pairs tested inside the walk or in one k_narrow launch (`narrow`)."""
-    best = None
+    tried at each entry level's best step shape, `tail` the (front pairs per
+    workgroup pass, steps) settings of the tail walk tried after the best head
+    setting, with leaf pairs tested inside the walk or in one k_narrow launch
+    (`narrow`)."""
+    shapes: dict = {}
     # reduce variant first, timed on the refit alone (the detect does not
     # depend on it), then the traversal shape
     base = ctx.get_tuning()
@@ -67,12 +68,30 @@ def tune(ctx: api.Context, scene: api.Scene, frame, *, entries=(4, 6, 8), expand
         ctx.set_tuning(traverse_blocks=nb, traverse_expand=expand, traverse_local=0, traverse_local_levels=0,
                        traverse_tail=0, traverse_tail_steps=0)
         ms = _time(ctx, scene, frame, entry, expand, reps)
-        if best is None or ms < best["ms"]:
-            best = {"entry_level": entry, "expand_levels": expand, "traverse_blocks": nb,
-                    "reduce_leaves_per_thread": lpt_best, "traverse_local": 0, "traverse_local_levels": 0,
-                    "traverse_tail": 0, "traverse_tail_steps": 0, "ms": ms}
-    # then the first steps as one workgroup-local launch, at the best shape
-    ctx.set_tuning(traverse_blocks=best["traverse_blocks"], traverse_expand=best["expand_levels"])
+        if entry not in shapes or ms < shapes[entry]["ms"]:
+            shapes[entry] = {"entry_level": entry, "expand_levels": expand, "traverse_blocks": nb,
+                             "reduce_leaves_per_thread": lpt_best, "traverse_local": 0, "traverse_local_levels": 0,
+                             "traverse_tail": 0, "traverse_tail_steps": 0, "ms": ms}
+    # the entry level that is fastest by steps alone need not be the one with
+    # local and tail walks (1M-triangle pair: 95 against 77 us a frame)
+    best = min((_tune_walks(ctx, scene, frame, shape, local, tail, narrow, reps) for shape in shapes.values()),
+               key=lambda b: b["ms"])
+    ctx.set_tuning(**{**{k: base[k] for k in base},
+                      "reduce_leaves_per_thread": best["reduce_leaves_per_thread"],
+                      "traverse_blocks": best["traverse_blocks"], "traverse_expand": best["expand_levels"],
+                      "traverse_local": best["traverse_local"],
+                      "traverse_local_levels": best["traverse_local_levels"],
+                      "traverse_tail": best["traverse_tail"], "traverse_tail_steps": best["traverse_tail_steps"],
+                      "narrow_separate": best["narrow_separate"]})
+    return best
+
+
+def _tune_walks(ctx, scene, frame, best, local, tail, narrow, reps) -> dict:
+    """tune's local and tail walks from one step shape"""
+    # the first steps as one workgroup-local launch
+    ctx.set_tuning(traverse_blocks=best["traverse_blocks"], traverse_expand=best["expand_levels"],
+                   traverse_local=0, traverse_local_levels=0, traverse_tail=0, traverse_tail_steps=0,
+                   narrow_separate=0)
     for chunk, levels in local:
         ctx.set_tuning(traverse_local=chunk, traverse_local_levels=levels)
         ms = _time(ctx, scene, frame, best["entry_level"], best["expand_levels"], reps)
@@ -89,13 +108,6 @@ def tune(ctx: api.Context, scene: api.Scene, frame, *, entries=(4, 6, 8), expand
         ms = _time(ctx, scene, frame, best["entry_level"], best["expand_levels"], reps)
         if ms < best["ms"]:
             best = {**best, "narrow_separate": ns, "traverse_tail": chunk, "traverse_tail_steps": steps, "ms": ms}
-    ctx.set_tuning(**{**{k: base[k] for k in base},
-                      "reduce_leaves_per_thread": best["reduce_leaves_per_thread"],
-                      "traverse_blocks": best["traverse_blocks"], "traverse_expand": best["expand_levels"],
-                      "traverse_local": best["traverse_local"],
-                      "traverse_local_levels": best["traverse_local_levels"],
-                      "traverse_tail": best["traverse_tail"], "traverse_tail_steps": best["traverse_tail_steps"],
-                      "narrow_separate": best["narrow_separate"]})
     return best
 
 
