@@ -5,18 +5,20 @@
 // runs triangle_intersect_kernel over the candidate list (collide.cu:248-300).
 // Here the steps are launched back to back with no host round trip:
 //   k_seed        zeroes the level counts and detect counters;
-//   k_bvtt_step   one BVTT step, grid-stride over the current front (its
+//   k_bvtt_walk   one or two BVTT steps over a short front, 2^e lanes per pair;
+//   k_bvtt_step   one BVTT step, grid-stride over a long front (its
 //                 length is read from device memory): both sides of an
 //                 overlapping pair descend up to E levels (a leaf stands for
 //                 itself, collide.cu:165-176) and every pair of the two
 //                 descendant runs is tested for AABB overlap (collide.cu:
-//                 12-17); overlapping leaf pairs go to the candidate list,
-//                 other overlapping pairs to the next front. Outputs are
-//                 compacted with a block prefix sum and one device-scope
-//                 fetch_add per block;
+//                 12-17); overlapping leaf pairs are tested with the SAT or go
+//                 to the candidate list, other overlapping pairs to the next
+//                 front. Both gather in LDS and leave in blocks, with one
+//                 device-scope fetch_add each;
 //   k_narrow      17-axis SAT (utils.cpp:71-169 / cuda_intersect_tritri.h:
 //                 350-434) over the candidate list, hits appended as
-//                 (meshA, meshB, origTriA, origTriB) in original face ids.
+//                 (meshA, meshB, origTriA, origTriB) in original face ids;
+//   k_publish     the query's counters to pinned memory.
 // Self mode (no reference counterpart) also walks each mesh against itself:
 // a node paired with itself expands to the unordered pairs of its children;
 // leaf pairs sharing a vertex index are dropped before the SAT.
