@@ -48,22 +48,6 @@ __device__ __forceinline__ void st_relaxed(uint32_t* p, uint32_t v)
 }
 
 // ---------------------------------------------------------------------------
-// block-wide exclusive scan of one uint32 per thread (256 threads, wave64)
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s_wsum, uint32_t& total)
-{
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t x = oi_wave_scan_incl(v);
-    if (lane == 63) s_wsum[wave] = x;
-    __syncthreads();
-    uint32_t w0 = s_wsum[0], w1 = s_wsum[1], w2 = s_wsum[2], w3 = s_wsum[3];
-    uint32_t before = (wave > 0 ? w0 : 0u) + (wave > 1 ? w1 : 0u) + (wave > 2 ? w2 : 0u);
-    total = w0 + w1 + w2 + w3;
-    __syncthreads();
-    return before + x - v;
-}
-
-// ---------------------------------------------------------------------------
 // mesh tables
 // ---------------------------------------------------------------------------
 // Meshes come from a device table with a work list, or (d = null) travel in
