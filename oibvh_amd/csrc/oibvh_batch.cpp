@@ -877,7 +877,8 @@ static void detect_key(const oibvh_batch* b, uint32_t flags, uint64_t* k)
     k[2] = (flags & ~(OIBVH_DETECT_ASYNC | OIBVH_FRAME_OVERLAP)) | ((uint64_t)c->narrow_separate << 32);
     k[3] = (uint64_t)b->reduce_M | ((uint64_t)d.tail_chunk << 16) | ((uint64_t)d.tail_from << 40);
     k[4] = d.generation;
-    k[5] = (uint64_t)b->desc_gen ^ ((uint64_t)oi_grid_for(c) << 32);
+    // (the setting itself: 0 and its four workgroups per CU launch different grids)
+    k[5] = (uint64_t)b->desc_gen | ((uint64_t)c->trav_blocks << 32);
     k[6] = (uint64_t)b->cur | ((uint64_t)d.n_levels << 8) | ((uint64_t)d.n_front << 32);
     k[7] = (uint64_t)c->refit_blocks;
 }
