@@ -226,7 +226,11 @@ typedef struct {
                                           subtree of 256 x this many leaves; 16: one subtree of 256
                                           leaves per wave (4 per lane, interleaved), four per
                                           workgroup (0 = by mesh size) */
-    uint32_t traverse_blocks;          /* workgroups per BVTT-level and narrow-phase launch (0 = 4 per CU) */
+    uint32_t traverse_blocks;          /* workgroups per BVTT-step and narrow-phase launch, and the most that
+                                          a walk over a short front launches; the local walks of
+                                          traverse_local and traverse_tail have grids of their own (0 = by
+                                          launch: 4 per CU, 6 for FP32 steps of up to two levels, 2 for a
+                                          walk and 4 for one over a longer front) */
     uint32_t traverse_expand;          /* levels each side descends per BVTT step, 1..3 (0 = the
                                           detect call's expandLevels, clamped to 1..3) */
     uint32_t front_capacity;           /* initial BVTT front entries per buffer, a power of two (0 = 2^22) */

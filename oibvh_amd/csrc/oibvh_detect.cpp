@@ -276,8 +276,11 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
     // instead of 1,849 us a frame, one of 522K 264 instead of 279. With the FP32
     // filter in the step four are faster (331 against 339 us on coplanar scenes),
     // and beside the next frame's refit they leave it room.
-    const uint32_t grid = oi_grid_for(c);
-    const uint32_t grid2 = c->trav_blocks || fuse != 1 || d->stream ? grid : (uint32_t)std::max(1, c->cus) * 6u;
+    const uint32_t cus = (uint32_t)std::max(1, c->cus), grid = oi_grid_for(c);
+    const uint32_t grid2 = c->trav_blocks || fuse != 1 || d->stream ? grid : 6u * cus;
+    // and per walk, over a short and over a long front; a setting is the most they launch
+    const uint32_t most = c->trav_blocks ? c->trav_blocks : ~0u;
+    const uint32_t walk_wgs = std::min(most, 2u * cus), walk_long = std::min(most, 4u * cus);
     // `done` rides on the last launch: k_narrow, else the tail walk, else
     // the last step, else the head walk
     const bool narrow = !d->fused || fp64, tail = T < d->n_levels, steps = T > J;
@@ -322,11 +325,10 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
             w.count_mid = two ? d->counts + k + 1 : nullptr;
             w.count_out = d->counts + o + 1;
             w.cap_out = d->front_cap;
-            w.wgs_long = (d->step_walk[k] & 4u) && !d->stream ? 4u * (uint32_t)std::max(1, c->cus) : 0u;
+            w.wgs_long = (d->step_walk[k] & 4u) && !d->stream ? walk_long : 0u;
             w.done = (!narrow && !tail && o + 1 == T) ? done : nullptr;
-            HIPCHK(c, oi_launch_bvtt_walk(st, (uint32_t)std::max(1, c->cus) * 2u, &d->tab, &w, d->cands,
-                                          &d->ctl->cands, d->cand_cap, d->hits, d->hits_cap, d->ctl, d->implicit_end,
-                                          fuse));
+            HIPCHK(c, oi_launch_bvtt_walk(st, walk_wgs, &d->tab, &w, d->cands, &d->ctl->cands, d->cand_cap, d->hits,
+                                          d->hits_cap, d->ctl, d->implicit_end, fuse));
             k = o;
             continue;
         }
