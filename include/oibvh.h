@@ -229,8 +229,9 @@ typedef struct {
     uint32_t traverse_blocks;          /* workgroups per BVTT-step and narrow-phase launch, and the most that
                                           a walk over a short front launches; the local walks of
                                           traverse_local and traverse_tail have grids of their own (0 = by
-                                          launch: 4 per CU, 6 for FP32 steps of up to two levels, 2 for a
-                                          walk and 4 for one over a longer front) */
+                                          launch: 4 per CU, 2 for a walk; in frames that do not overlap 6
+                                          for FP32 steps of up to two levels and 4 for a walk over a
+                                          longer front) */
     uint32_t traverse_expand;          /* levels each side descends per BVTT step, 1..3 (0 = the
                                           detect call's expandLevels, clamped to 1..3) */
     uint32_t front_capacity;           /* initial BVTT front entries per buffer, a power of two (0 = 2^22) */

@@ -932,7 +932,10 @@ static oibvh_status overlapped_frame(oibvh_batch* b, uint32_t entry, uint32_t ex
     // detect half, captured on the context's stream, run on this detect's side stream
     oibvh_batch::Graph& gd = b->g_detect[b->cur];
     key[7] |= seeded ? (1ull << 40) : 0ull;
-    if ((r = captured(b, gd, key, [&]() { return oi_det_enqueue(&d, false, seeded); })) != OIBVH_OK) return r;
+    d.beside_refit = true;
+    r = captured(b, gd, key, [&]() { return oi_det_enqueue(&d, false, seeded); });
+    d.beside_refit = false;
+    if (r != OIBVH_OK) return r;
     const uint64_t q = c->side_seq;
     hipStream_t side = oi_side_stream(c, q);
     HIPCHK(c, hipStreamWaitEvent(side, c->ev_main, 0));

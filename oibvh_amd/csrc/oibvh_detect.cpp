@@ -275,9 +275,13 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
     // with six instead of four the folded cloth of 8.4M triangles takes 1,743
     // instead of 1,849 us a frame, one of 522K 264 instead of 279. With the FP32
     // filter in the step four are faster (331 against 339 us on coplanar scenes),
-    // and beside the next frame's refit they leave it room.
+    // and beside the next frame's refit they leave it room (overlapped batches, with
+    // six a CU, and four in long walks, against four and two: 32 cloths of 32K
+    // triangles 361 against 323 us a frame, one of 522K 170 against 160, 16 scenes of
+    // rigid bodies 281 against 262; two cloths of 2.1M, one of 8.4M and 128 scenes the
+    // same within 2 %).
     const uint32_t cus = (uint32_t)std::max(1, c->cus), grid = oi_grid_for(c);
-    const uint32_t grid2 = c->trav_blocks || fuse != 1 || d->stream ? grid : 6u * cus;
+    const uint32_t grid2 = c->trav_blocks || fuse != 1 || d->beside_refit ? grid : 6u * cus;
     // and per walk, over a short and over a long front; a setting is the most they launch
     const uint32_t most = c->trav_blocks ? c->trav_blocks : ~0u;
     const uint32_t walk_wgs = std::min(most, 2u * cus), walk_long = std::min(most, 4u * cus);
@@ -325,7 +329,7 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
             w.count_mid = two ? d->counts + k + 1 : nullptr;
             w.count_out = d->counts + o + 1;
             w.cap_out = d->front_cap;
-            w.wgs_long = (d->step_walk[k] & 4u) && !d->stream ? walk_long : 0u;
+            w.wgs_long = (d->step_walk[k] & 4u) && !d->beside_refit ? walk_long : 0u;
             w.done = (!narrow && !tail && o + 1 == T) ? done : nullptr;
             HIPCHK(c, oi_launch_bvtt_walk(st, walk_wgs, &d->tab, &w, d->cands, &d->ctl->cands, d->cand_cap, d->hits,
                                           d->hits_cap, d->ctl, d->implicit_end, fuse));

@@ -1261,8 +1261,10 @@ static oibvh_status overlapped_frame(oibvh_scene* s, uint32_t entry, uint32_t ex
     }
     // the detect's last launch records this detect's ring event
     d.stream = side;
+    d.beside_refit = true;
     r = oi_det_enqueue(&d, !async, seeded, c->ev_ring[q % OI_SIDE_RING]);
     d.stream = nullptr;
+    d.beside_refit = false;
     if (r != OIBVH_OK) return r;
     c->side_seq++;
     if (e1) HIPCHK(c, hipEventRecord(e1, side));

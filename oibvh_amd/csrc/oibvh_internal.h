@@ -301,6 +301,7 @@ struct oi_detector {
     uint64_t tail_off = 0;      // the same for the tail walk
     bool fused = false;  // narrow phase inside the BVTT steps (FP32 queries)
     hipStream_t stream = nullptr;  // stream of the next enqueue (null: the context's)
+    bool beside_refit = false;     // the next enqueue is an overlapped frame's: it runs beside the next refit
     bool unchecked = false;
     bool have_result = false;
     uint32_t n_pairs = 0;

@@ -11,3 +11,9 @@ def test_batch_frame_key_covers_workgroup_setting(tmp_path):
 def test_workgroup_setting_holds_for_every_launch(tmp_path):
     """traverse_blocks is the grid of a step and the most that a walk launches."""
     host_cpp.run("detect_grids", tmp_path)
+
+
+def test_overlapped_batch_query_leaves_room(tmp_path):
+    """An overlapped batch frame's query launches as an overlapped scene's does: four
+    workgroups a CU for a step, two for a walk."""
+    host_cpp.run("overlap_grids", tmp_path)
