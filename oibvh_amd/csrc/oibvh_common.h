@@ -241,6 +241,19 @@ struct oi_hit_digits {
     uint8_t shift[OI_HIT_DIGITS];
 };
 
+// The place in a list of n hits of its sample's i-th of S <= n keys: anywhere in the
+// i-th of S even strides, by a multiplicative hash of i. (Evenly spaced, a list whose
+// order repeats with the stride gave a sample of one kind of its hits: one bucket then
+// held nearly all the others.)
+OI_HD uint32_t oi_sample_at(uint32_t i, uint32_t n, uint32_t S)
+{
+    const uint32_t lo = (uint32_t)((uint64_t)i * n / S), hi = (uint32_t)((uint64_t)(i + 1u) * n / S);
+    uint32_t h = (i + 1u) * 2654435769u;  // 2^32 over the golden ratio
+    h = (h ^ (h >> 16)) * 2654435769u;
+    h ^= h >> 15;
+    return lo + (uint32_t)((uint64_t)h * (hi - lo) >> 32);
+}
+
 // bits that the mesh ids and the face ids of a hit list can have (a sort key
 // holds two of each)
 struct oi_pair_bits {

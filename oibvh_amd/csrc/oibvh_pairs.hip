@@ -155,7 +155,7 @@ struct PairRec {
     uint32_t bucket, at;
 };
 
-// the keys of S evenly spaced hits side by side (every workgroup of
+// the keys of S hits (oi_sample_at) side by side (every workgroup of
 // k_pairs_split reads them all: 512 of them gathering 8192 lines of hits took
 // 32 us), and zeroed bucket counts
 __global__ void __launch_bounds__(256)
@@ -163,7 +163,7 @@ k_pairs_sample(const uint4* __restrict__ hits, uint32_t n, oi_pair_bits bits, ui
                uint32_t nb, uint32_t* __restrict__ counts)
 {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i < S) sample[i] = Key64::of(load_hit(hits, (uint32_t)((u64)i * n / S)), bits).k;
+    if (i < S) sample[i] = Key64::of(load_hit(hits, oi_sample_at(i, n, S)), bits).k;
     if (i < nb) counts[i] = 0u;
 }
 
@@ -276,23 +276,48 @@ __device__ __forceinline__ void wave_order()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// places a < b of a list of m, ascending (places from m on hold the top key)
+__device__ __forceinline__ void order_pair(u64* g, uint32_t a, uint32_t b, uint32_t m)
+{
+    if (b >= m) return;
+    const u64 x = g[a], y = g[b];
+    if (x > y) {
+        g[a] = y;
+        g[b] = x;
+    }
+}
+
 // One bucket per workgroup, bitonic in LDS; a wave's 64 compare-exchanges of a
 // stage of distance <= 64 cover 128 consecutive keys in every such stage, so
 // only wider ones need a barrier. A bucket that outgrew LDS (the sample missed
-// badly) is ranked from memory: slow, and right.
+// badly) is sorted in place in memory, every merge ascending (its first stage
+// compares mirrored places) so that the places past its end never move: all of
+// 40,000 keys in one bucket 1.4 ms, of 175,000 7.1, where ranking them against each
+// other took the square of their number.
 __global__ void __launch_bounds__(PS_THREADS)
-k_pairs_sort(const u64* __restrict__ keys, const uint32_t* __restrict__ starts, oi_pair_bits bits,
-             uint4* __restrict__ out)
+k_pairs_sort(u64* keys, const uint32_t* __restrict__ starts, oi_pair_bits bits, uint4* __restrict__ out)
 {
     __shared__ u64 s[PS_CAP];
     const uint32_t tid = threadIdx.x, p0 = starts[blockIdx.x], m = starts[blockIdx.x + 1u] - p0;
     if (m > PS_CAP) {
-        for (uint32_t i = tid; i < m; i += PS_THREADS) {
-            const u64 k = keys[p0 + i];
-            uint32_t r = 0;
-            for (uint32_t j = 0; j < m; j++) r += keys[p0 + j] < k ? 1u : 0u;
-            out[p0 + r] = hit_of(k, bits);
+        u64* g = keys + p0;
+        uint32_t P = PS_CAP;
+        while (P < m) P <<= 1;  // m <= 2^30
+        for (uint32_t k = 2; k <= P; k <<= 1) {
+            for (uint32_t i = tid; i < (P >> 1); i += PS_THREADS) {
+                const uint32_t a = 2u * i - (i & ((k >> 1) - 1u));
+                order_pair(g, a, a ^ (k - 1u), m);
+            }
+            __syncthreads();
+            for (uint32_t j = k >> 2; j; j >>= 1) {
+                for (uint32_t i = tid; i < (P >> 1); i += PS_THREADS) {
+                    const uint32_t a = 2u * i - (i & (j - 1u));
+                    order_pair(g, a, a + j, m);
+                }
+                __syncthreads();
+            }
         }
+        for (uint32_t i = tid; i < m; i += PS_THREADS) out[p0 + i] = hit_of(g[i], bits);
         return;
     }
     uint32_t P = 128;
@@ -361,7 +386,7 @@ uint64_t oi_pairs_sort_bytes(uint32_t n)
 hipError_t oi_launch_pairs_sort(hipStream_t st, const uint4* hits, uint32_t n, oi_pair_bits bits, void* scratch,
                                 uint4* out)
 {
-    if (n < PS_BUCKETS * PS_OVER / 2u || 2u * (bits.mesh + bits.tri) > 64u) return hipErrorInvalidValue;
+    if (n < PS_BUCKETS * PS_OVER / 2u || n > 1u << 30 || 2u * (bits.mesh + bits.tri) > 64u) return hipErrorInvalidValue;
     PairRec* rec = (PairRec*)scratch;
     u64* keys = (u64*)(rec + n);
     u64* splitters = keys + n;

@@ -17,3 +17,9 @@ def test_overlapped_batch_query_leaves_room(tmp_path):
     """An overlapped batch frame's query launches as an overlapped scene's does: four
     workgroups a CU for a step, two for a walk."""
     host_cpp.run("overlap_grids", tmp_path)
+
+
+def test_pair_sample_of_lists_that_follow_its_stride(tmp_path):
+    """No bucket of the pair lists' sample sort outgrows LDS on lists whose order
+    repeats at any distance."""
+    host_cpp.run("pair_sample", tmp_path)
