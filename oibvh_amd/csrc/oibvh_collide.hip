@@ -879,6 +879,28 @@ __device__ __forceinline__ void ring_leaves(const Args& A, Ring& S, const oi_mes
 // 80 VGPRs (6 waves) unspilled.
 #define STEP_FULL 1024  // kept pairs that leave for the front at a time, at least
 
+// The leaf pairs of a tile by their number: thread t keeps the set bits of mask[t]
+// (bit (x << 3) + y: pair (x, y) from p0[t] on), numbered from off[t] (one that keeps
+// none has the next one's off).
+struct StepFind {
+    u64 mask[TB];
+    uint2 p0[TB];
+    uint32_t off[TB];
+    __device__ __forceinline__ uint2 pair(uint32_t c) const
+    {
+        uint32_t lo = 0, hi = TB - 1;  // last thread whose first is at or before c
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1u) >> 1;
+            if (off[mid] <= c)
+                lo = mid;
+            else
+                hi = mid - 1u;
+        }
+        const uint32_t k = select_bit(mask[lo], c - off[lo]);
+        return make_uint2(p0[lo].x + (k >> 3), p0[lo].y + (k & 7u));
+    }
+};
+
 template <int E, bool FIRST, int FUSE, class Tab>
 __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(E == 3 ? 4 : E == 2 ? 6 : 1, 8)))
 k_bvtt_step(StepArgs<Tab> A)
@@ -890,6 +912,7 @@ k_bvtt_step(StepArgs<Tab> A)
     __shared__ uint32_t s_ibase[MESH_LDS];
     __shared__ uint32_t s_wsum[4];
     __shared__ Ring S;
+    __shared__ std::conditional_t<E == 3, StepFind, char> s_find;
     // after an overflow the count keeps growing past the buffer (writes were
     // dropped and the detect will be re-run): read only what exists
     uint32_t n_in = A.count_in ? *A.count_in : A.n_in;
@@ -926,9 +949,36 @@ k_bvtt_step(StepArgs<Tab> A)
         uint32_t at = leafout ? n_cand + (oc & 0xffffu) : n_out + (oc >> 16);
         n_out += TC >> 16;
         n_cand += TC & 0xffffu;
+        // More leaf pairs than their ring has room for (three levels: up to 64 a thread).
+        // Written by the threads that keep them they would wait for the ring in turn, a
+        // few lanes at a time; every thread takes the next one by its number instead (two
+        // rough shells of 360K triangles, by steps: with 4.9M leaf pairs 701 -> 473 us a
+        // query, with 164M 6,135 -> 3,860). Kept pairs, whose ring mostly holds a tile's,
+        // are written faster by their threads.
+        const uint32_t cand0 = n_cand - (TC & 0xffffu);
+        uint32_t put = cand0;
+        bool by_number = false;
+        if constexpr (E == 3) {
+            by_number = n_cand - cand_done > Ring::CAND;
+            if (by_number) {
+                s_find.mask[tid] = m;
+                s_find.p0[tid] = p0;
+                s_find.off[tid] = oc & 0xffffu;
+                __syncthreads();
+                if (leafout) m = 0;
+            }
+        }
         for (;;) {
             // what fits into the rings; while one is full enough it is emptied
             // and the rest follows
+            if constexpr (E == 3) {
+                if (by_number) {
+                    const uint32_t to = cand_done + min(n_cand - cand_done, Ring::CAND);
+                    for (uint32_t q = put + tid; (int32_t)(to - q) > 0; q += TB)
+                        S.cand[q & (Ring::CAND - 1u)] = s_find.pair(q - cand0);
+                    put = to;
+                }
+            }
             uint2* ring = leafout ? S.cand : S.out;
             const uint32_t wrap = leafout ? Ring::CAND - 1u : Ring::OUT - 1u;
             const uint32_t lim = leafout ? cand_done + Ring::CAND : out_done + Ring::OUT;

@@ -46,3 +46,37 @@ def test_walks_by_few_workgroups(api, ctx, orc, blocks, entry, expand):
         assert np.array_equal(scene.level_counts(), levels)
     finally:
         ctx.set_tuning(**base)
+
+
+def cloud(n, size, seed, spread=1.0):
+    r = np.random.default_rng(seed)
+    xyz = r.uniform(-spread, spread, (n, 1, 3)) + r.uniform(-size, size, (n, 3, 3))
+    return xyz.reshape(-1, 3).astype(np.float32), np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+
+
+@pytest.mark.parametrize("mode", ["fp32", "separate", "fp64"])
+def test_steps_that_keep_every_pair(api, ctx, orc, mode):
+    """Three-level steps (after a head walk of one step, so that none is a walk) over
+    clouds in which every box meets every other: 64 pairs kept per front pair, many
+    times what the rings in LDS hold, all of one kind, both kinds in one tile (trees of
+    unequal depth), and against itself: the oracle's pairs."""
+    print(f"steps that keep every pair, {mode}", flush=True)
+    fp64 = mode == "fp64"
+    a, b, small = cloud(700, 2.0, 1, 0.1), cloud(650, 2.0, 2, 0.1), cloud(40, 2.0, 3, 0.1)
+    base = ctx.get_tuning()
+    ctx.set_tuning(traverse_local=1, traverse_local_levels=1, narrow_separate=1 if mode == "separate" else 0)
+    try:
+        for meshes, entry, self_collide in (([a, b], 1, False), ([a, small], 1, False), ([a, b, small], 3, False),
+                                            ([b], 3, True)):
+            scene, trees = scene_of(api, ctx, meshes)
+            scene.detectCollision(entry, 3, self_collide=self_collide, fp64_fallback=fp64)
+            want = orc.detect([orc.Tree(x, f, order=t.perm()) for (x, f), t in zip(meshes, trees)],
+                              self_collide=self_collide, fp64=fp64)
+            assert len(want) > 5000
+            assert np.array_equal(scene.getIntTriPairs(), want), (len(meshes), entry)
+            if len(meshes) == 2 and meshes[1] is b:
+                # nodes of the levels 1, 4 and 7 over 700 and 650 leaves
+                levels = scene.level_counts()
+                assert list(levels[:2]) == [2 * 2, 11 * 11] and levels[2] > 0.9 * 88 * 82
+    finally:
+        ctx.set_tuning(**base)
