@@ -133,7 +133,8 @@ oibvh_status oi_det_set_front(oi_detector* d, const std::vector<uint2>& front)
 // second's tests are few as well. The host does not know the fronts' lengths: it
 // takes them to grow by e + 1 per step of e levels (measured: 2.0-2.9 for two
 // levels and 2.8-4.2 for three, two bodies), in self mode by 2^e + 3 (4-8 and
-// 9-15, folded cloth). A wrong guess costs speed only.
+// 9-15, folded cloth), or, after a query that met far longer ones, as that query met
+// them (judge_walk). A wrong guess costs speed only.
 // Where the lines lie: one k_bvtt_step of three levels takes 15 us on any front up
 // to 10,000 pairs and 18-25 us at 50,000, a walk of two such steps 11 us at 100
 // pairs, 19 us at 2,800 and of one step 14 us at 10,000; a step of two levels
@@ -141,23 +142,87 @@ oibvh_status oi_det_set_front(oi_detector* d, const std::vector<uint2>& front)
 #define OI_WALK_MAX3 65536u
 #define OI_WALK_MAX 2048u
 #define OI_WALK_TESTS (1u << 21)
-// guessed lengths from here on get workgroups for a long front (beside the next
-// frame's refit they would take its room)
+// lengths from here on get workgroups for a long front (beside the next frame's
+// refit they would take its room)
 #define OI_WALK_LONG 16384u
+static uint64_t walk_max(uint32_t e) { return e == 3 ? OI_WALK_MAX3 : OI_WALK_MAX; }
+
+// walk[k] for n steps of e[k] levels over fronts of len[k] pairs
+static void walk_steps(uint32_t n, const uint8_t* e, const uint32_t* len, uint8_t* walk)
+{
+    std::memset(walk, 0, n);
+    for (uint32_t k = 0; k < n && len[k] <= walk_max(e[k]); k++) {
+        walk[k] = len[k] >= OI_WALK_LONG ? 5 : 1;
+        if (k + 1 < n && (uint64_t)len[k + 1] << (2u * e[k + 1]) <= OI_WALK_TESTS) walk[k++]++;
+    }
+}
+
+// whether a walk of that plan meets a front too long for it, with `far` much too long.
+// (The lines of `far`. First steps: a walk of two levels over 60K pairs of one dense
+// spot takes 98 us where the step takes 124, one of three over 948K, leaf pairs mostly,
+// no more than the step, and 140K pairs with their 500K children 64 against 74; but
+// over 741K others 105 against 69. Second steps: 12K pairs with their 108K children of
+// three levels 62-82 us against 45 by a walk and a step, 39K with 260K 165 against 52.)
+static bool walk_too_long(uint32_t n, const uint8_t* e, const uint8_t* walk, const uint32_t* len, bool far)
+{
+    for (uint32_t k = 0; k < n && walk[k]; k++) {
+        if (len[k] > (far ? 4u : 2u) * OI_WALK_MAX3) return true;
+        if ((walk[k] & 3u) != 2u) continue;
+        k++;
+        if ((uint64_t)len[k] << (2u * e[k]) > (far ? OI_WALK_TESTS * 3u / 2u : OI_WALK_TESTS)) return true;
+    }
+    return false;
+}
+
+static void guess_lengths(const oi_detector* d, uint32_t* len)
+{
+    const bool self = (d->flags & OIBVH_DETECT_SELF) != 0;
+    uint64_t est = d->n_front;
+    for (uint32_t k = 0; k < d->n_levels; k++) {
+        len[k] = (uint32_t)std::min<uint64_t>(est, 1u << 31);
+        est = len[k] * (uint64_t)(self ? (1u << d->step_e[k]) + 3u : d->step_e[k] + 1u);
+    }
+}
+
 static void plan_walk(oi_detector* d)
 {
     std::memset(d->step_walk, 0, sizeof d->step_walk);
+    // lengths that another query met
+    if (d->n_seen && (d->n_seen != d->n_levels || d->seen[0] != d->n_front ||
+                      d->seen_self != ((d->flags & OIBVH_DETECT_SELF) != 0) ||
+                      std::memcmp(d->seen_e, d->step_e, d->n_levels) != 0)) {
+        d->n_seen = 0;
+        d->generation++;
+    }
     if (d->local_chunk || d->tail_chunk || d->n_front == 0) return;
-    const bool self = (d->flags & OIBVH_DETECT_SELF) != 0;
-    uint64_t est = d->n_front;
-    auto grown = [&](uint32_t k) { return est * (self ? (1u << d->step_e[k]) + 3u : d->step_e[k] + 1u); };
-    for (uint32_t k = 0; k < d->n_levels && est <= (d->step_e[k] == 3 ? OI_WALK_MAX3 : OI_WALK_MAX); k++) {
-        d->step_walk[k] = est >= OI_WALK_LONG ? 5 : 1;
-        est = grown(k);
-        if (k + 1 < d->n_levels && est << (2u * d->step_e[k + 1]) <= OI_WALK_TESTS) {
-            d->step_walk[k++]++;
-            est = grown(k);
-        }
+    uint32_t guess[256];
+    if (!d->n_seen) guess_lengths(d, guess);
+    walk_steps(d->n_levels, d->step_e, d->n_seen ? d->seen : guess, d->step_walk);
+}
+
+// After a query whose front lengths have been read: where a walk met a front far past
+// its limit, the next queries are planned by these lengths, until one fits the guess's
+// plan. (Overlapping triangle clouds grow by 9 to 19 a step of three levels. Two of
+// 400,000 triangles: 305 and, denser, 535 us a query as guessed, 158 and 274 from the
+// second query on; 218 and 340 by the steps alone that were there before the walks.)
+static void judge_walk(oi_detector* d)
+{
+    if (d->local_chunk || d->tail_chunk || d->n_front == 0) return;
+    const uint32_t n = d->n_levels, *len = d->h_counts.data();
+    if (walk_too_long(n, d->step_e, d->step_walk, len, true)) {
+        d->n_seen = n;
+        std::copy(len, len + n, d->seen);
+        std::copy(d->step_e, d->step_e + n, d->seen_e);
+        d->seen_self = (d->flags & OIBVH_DETECT_SELF) != 0;
+        d->generation++;
+    } else if (d->n_seen) {
+        uint32_t guess[256];
+        uint8_t walk[256];
+        guess_lengths(d, guess);
+        walk_steps(n, d->step_e, guess, walk);
+        if (walk_too_long(n, d->step_e, walk, len, false)) return;
+        d->n_seen = 0;
+        d->generation++;
     }
 }
 
@@ -510,6 +575,7 @@ oibvh_status oi_det_check(oi_detector* d)
             d->stats.async_errors = earlier;
             d->unchecked = false;
             d->sorted_ok = false;  // a new result: sorted again on demand
+            judge_walk(d);
             return OIBVH_OK;
         }
         retries++;

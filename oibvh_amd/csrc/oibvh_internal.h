@@ -293,6 +293,12 @@ struct oi_detector {
     uint32_t schedule = 0;      // levels per step of the first steps (2 bits each), then `expand`
     uint8_t step_e[256] = {};   // levels descended by each step of the current query
     uint8_t step_walk[256] = {};  // 1 or 2: step k (and k + 1) as one k_bvtt_walk launch; + 4: long
+    // front lengths that a query of n_seen steps of seen_e levels met, where the walks
+    // guessed for it were far too long (n_seen = 0: the guess holds)
+    uint32_t n_seen = 0;
+    uint32_t seen[256] = {};
+    uint8_t seen_e[256] = {};
+    bool seen_self = false;
     uint32_t local_chunk = 0;   // this query: initial pairs per workgroup of the local walk (0: steps)
     uint32_t local_levels = 0;  // this query: steps done by the local walk
     uint64_t local_off = 0;     // 1 + the tuning generation in which the head walk overflowed (0: none)
@@ -317,7 +323,7 @@ struct oi_detector {
     float* d_stage = nullptr;     // vertex export staging for host output
     uint64_t stage_cap = 0;
     oibvh_detect_stats stats{};
-    uint64_t generation = 0;  // bumped whenever a device buffer is replaced
+    uint64_t generation = 0;  // bumped whenever a device buffer is replaced or the walks are planned by other lengths
 };
 
 oibvh_status oi_det_init(oi_detector* d, oibvh_ctx* c);

@@ -80,3 +80,43 @@ def test_steps_that_keep_every_pair(api, ctx, orc, mode):
                 assert list(levels[:2]) == [2 * 2, 11 * 11] and levels[2] > 0.9 * 88 * 82
     finally:
         ctx.set_tuning(**base)
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_walks_over_clouds_that_meet_and_part(api, ctx, orc, batched):
+    """Two clouds whose fronts grow far faster than guessed: the steps are planned
+    again after the first query, and back after the clouds have parted. Always the
+    oracle's pairs, front lengths and statistics of the first query."""
+    print(f"walks over clouds, batched={batched}", flush=True)
+    a, b = cloud(20000, 0.1, 1), cloud(20000, 0.1, 2)
+    far = (b[0] + np.float32(1.9), b[1])
+    on = {"near": b, "far": far}
+    device = {k: api.DeviceBuffer.from_array(v[0]) for k, v in on.items()}
+    if batched:
+        obj = api.Batch(ctx)
+        for m in (a, b):
+            obj.add_mesh(0, *m)
+        obj.build()
+    else:
+        obj, trees = scene_of(api, ctx, [a, b])
+        order = trees[1].perm()
+    want, seen = {}, {}
+    for k, (xyz, f) in on.items():
+        order = obj.perm(1) if batched else order
+        want[k] = orc.detect([orc.Tree(*a), orc.Tree(xyz, f, order=order)])
+    assert len(want["near"]) > 20000 > len(want["far"])
+    for k in ("near", "near", "near", "far", "far", "near", "near"):
+        if batched:
+            obj.set_positions_device(1, device[k].ptr.value)
+            obj.frame(4, 3)
+            got = obj.pairs()
+        else:
+            trees[1].set_positions_device(device[k].ptr.value)
+            obj.frame(None, 4, 3)
+            got = obj.getIntTriPairs()
+        assert np.array_equal(got, want[k]), k
+        levels, stats = obj.level_counts(), obj.stats()
+        if k not in seen:
+            seen[k] = levels, stats["bvtt_tests"], stats["candidates"]
+        assert np.array_equal(levels, seen[k][0]) and (stats["bvtt_tests"], stats["candidates"]) == seen[k][1:], k
+    assert seen["near"][0].max() > 1 << 17 > seen["far"][0].max()

@@ -23,3 +23,9 @@ def test_pair_sample_of_lists_that_follow_its_stride(tmp_path):
     """No bucket of the pair lists' sample sort outgrows LDS on lists whose order
     repeats at any distance."""
     host_cpp.run("pair_sample", tmp_path)
+
+
+def test_walks_follow_the_fronts_that_a_check_has_read(tmp_path):
+    """Steps guessed short that meet fronts far past the walks' limits are
+    planned by those lengths from the next query on, until they fit the guess."""
+    host_cpp.run("walk_plan", tmp_path)
