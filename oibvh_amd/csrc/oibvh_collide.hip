@@ -907,12 +907,16 @@ k_bvtt_step(StepArgs<Tab> A)
 {
     constexpr uint32_t K = 1u << E;
     using M = PairMask<E>;
-    using Ring = RingLds<2 * STEP_FULL, 2 * TB>;
+    // leaf pairs are tested a thread each, or leave for the candidate list like kept
+    // pairs (256 at a time their additions to its count took most of a launch: 11M
+    // candidates of two rough shells 972 -> 534 us a query)
+    constexpr uint32_t LEAF_FULL = FUSE ? TB : STEP_FULL;
+    using Ring = RingLds<2 * STEP_FULL, 2 * LEAF_FULL>;
     __shared__ oi_mesh_desc s_desc[MESH_LDS];
     __shared__ uint32_t s_ibase[MESH_LDS];
     __shared__ uint32_t s_wsum[4];
     __shared__ Ring S;
-    __shared__ std::conditional_t<E == 3, StepFind, char> s_find;
+    __shared__ std::conditional_t<E == 3 && FUSE != 0, StepFind, char> s_find;
     // after an overflow the count keeps growing past the buffer (writes were
     // dropped and the detect will be re-run): read only what exists
     uint32_t n_in = A.count_in ? *A.count_in : A.n_in;
@@ -954,11 +958,11 @@ k_bvtt_step(StepArgs<Tab> A)
         // few lanes at a time; every thread takes the next one by its number instead (two
         // rough shells of 360K triangles, by steps: with 4.9M leaf pairs 701 -> 473 us a
         // query, with 164M 6,135 -> 3,860). Kept pairs, whose ring mostly holds a tile's,
-        // are written faster by their threads.
+        // are written faster by their threads, as are leaf pairs for the candidate list.
         const uint32_t cand0 = n_cand - (TC & 0xffffu);
         uint32_t put = cand0;
         bool by_number = false;
-        if constexpr (E == 3) {
+        if constexpr (E == 3 && FUSE != 0) {
             by_number = n_cand - cand_done > Ring::CAND;
             if (by_number) {
                 s_find.mask[tid] = m;
@@ -971,7 +975,7 @@ k_bvtt_step(StepArgs<Tab> A)
         for (;;) {
             // what fits into the rings; while one is full enough it is emptied
             // and the rest follows
-            if constexpr (E == 3) {
+            if constexpr (E == 3 && FUSE != 0) {
                 if (by_number) {
                     const uint32_t to = cand_done + min(n_cand - cand_done, Ring::CAND);
                     for (uint32_t q = put + tid; (int32_t)(to - q) > 0; q += TB)
@@ -988,15 +992,16 @@ k_bvtt_step(StepArgs<Tab> A)
             }
             __syncthreads();
             const uint32_t no = n_out - out_done, nc = n_cand - cand_done;
-            if (no < STEP_FULL && nc < TB) break;
+            if (no < STEP_FULL && nc < LEAF_FULL) break;
             if (no >= STEP_FULL) {
                 const uint32_t take = min(no, Ring::OUT);
                 ring_flush(A, S, out_done, take);
                 out_done += take;
             }
-            if (nc >= TB) {
-                ring_leaves<FUSE>(A, S, s_desc, s_ibase, cand_done, TB, n_adj);
-                cand_done += TB;
+            if (nc >= LEAF_FULL) {
+                const uint32_t take = FUSE ? LEAF_FULL : min(nc, Ring::CAND);
+                ring_leaves<FUSE>(A, S, s_desc, s_ibase, cand_done, take, n_adj);
+                cand_done += take;
                 __syncthreads();
             }
         }
