@@ -456,9 +456,13 @@ oibvh_status oi_det_enqueue(oi_detector* d, bool reset_sticky, bool seeded, hipE
 // Wait for the sequence number that the last launch on the context's stream
 // writes: a short wait on the memory itself (a stream wait costs about 10 us
 // more than the launch it waits for), then the stream's, which also reports a
-// failed launch.
+// failed launch. A program that chose to block or yield in its waits wants its core
+// back: there the stream's wait only.
 static hipError_t wait_published(oi_detector* d)
 {
+    unsigned flags = 0;
+    if (hipGetDeviceFlags(&flags) == hipSuccess && (flags & (hipDeviceScheduleYield | hipDeviceScheduleBlockingSync)))
+        return hipStreamSynchronize(d->ctx->stream);
     const auto t0 = std::chrono::steady_clock::now();
     while (__atomic_load_n(&d->h_pub->seq, __ATOMIC_ACQUIRE) != d->pub_seq)
         if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20))

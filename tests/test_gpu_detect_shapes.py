@@ -120,3 +120,23 @@ def test_walks_over_clouds_that_meet_and_part(api, ctx, orc, batched):
             seen[k] = levels, stats["bvtt_tests"], stats["candidates"]
         assert np.array_equal(levels, seen[k][0]) and (stats["bvtt_tests"], stats["candidates"]) == seen[k][1:], k
     assert seen["near"][0].max() > 1 << 17 > seen["far"][0].max()
+
+
+def test_checks_with_blocking_waits(api, ctx, orc):
+    """The same results in a program whose waits block (hipDeviceScheduleBlockingSync)."""
+    from oibvh_amd import _lib
+
+    print("checks with blocking waits", flush=True)
+    a, b = M.icosphere(4, 1.0, 0.02, 5), M.icosphere(4, 1.0, 0.02, 6, center=(0.2, 0.1, 0.0))
+    scene, _ = scene_of(api, ctx, [a, b])
+    want = orc.detect([orc.Tree(*a), orc.Tree(*b)])
+    hip = _lib.hip()
+    hip.hipSetDeviceFlags.argtypes = [_lib.C.c_uint]
+    assert hip.hipSetDeviceFlags(4) == 0
+    try:
+        for _ in range(3):
+            scene.detectCollision(4, 3)
+            assert np.array_equal(scene.getIntTriPairs(), want)
+            assert scene.pairs_device()[1] == len(want)
+    finally:
+        assert hip.hipSetDeviceFlags(0) == 0

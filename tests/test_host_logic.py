@@ -29,3 +29,9 @@ def test_walks_follow_the_fronts_that_a_check_has_read(tmp_path):
     """Steps guessed short that meet fronts far past the walks' limits are
     planned by those lengths from the next query on, until they fit the guess."""
     host_cpp.run("walk_plan", tmp_path)
+
+
+def test_checks_do_not_spin_where_waits_block(tmp_path):
+    """A program that chose blocking or yielding waits keeps its core while a check
+    waits for the GPU."""
+    host_cpp.run("check_wait", tmp_path)
