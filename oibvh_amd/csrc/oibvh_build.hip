@@ -943,13 +943,6 @@ __global__ void __launch_bounds__(OI_BLOCK) k_reduce(ReduceArgs<Tab> a)
 #define RW_LG 8
 #define RW_W (1u << RW_LG)
 
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Write `count` staged nodes (at most CMAX) to real index `first` onwards as
 // one contiguous run of float2 per lane; all LDS reads are issued before the
 // first store.
@@ -995,13 +988,13 @@ __device__ __forceinline__ void wave_level(float* stage, uint32_t width, uint32_
         if (has[it]) x[it] = get_box(stage, 2u * t);
         if (two[it]) y[it] = get_box(stage, 2u * t + 1u);
     }
-    wave_sync();
+    oi_wave_fence();
 #pragma unroll
     for (uint32_t it = 0; it < IT; it++) {
         if (two[it]) box_merge_into(x[it], y[it]);
         if (has[it]) put_box(stage, lane + 64u * it, x[it]);
     }
-    wave_sync();
+    oi_wave_fence();
 }
 
 // the refit's sorted faces of the leaves a wave owns
@@ -1117,7 +1110,7 @@ __device__ __forceinline__ void wave_climb_all(const oi_build_desc& D, uint32_t 
                                                uint32_t lane, float* W)
 {
     const uint32_t L = D.L, vl = D.vl;
-    wave_sync();
+    oi_wave_fence();
     wave_copy_out<RW_W>(D.nodes, oi_lvl_start(L, L, vl) + f0, min(1u << hw, nleaf - f0), W, lane);
     if (hw == RW_LG) {
         wave_climb8<1>(W, D.nodes, L, vl, f0, nleaf, lane);

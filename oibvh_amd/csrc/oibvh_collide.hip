@@ -512,12 +512,6 @@ __device__ __forceinline__ bool narrow_gather(const Tab& T, const uint32_t* s_ib
                                               uint2 c, bool count_adj, uint32_t& n_adj, v3f* P, v3f* Q, uint4& id);
 template <class Tab>
 __device__ __forceinline__ uint4 hit_ids(const Tab& T, const oi_mesh_desc* s_desc, uint4 id);
-template <bool FP64, class Tab>
-__device__ __forceinline__ void narrow_one(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
-                                           uint2 c, bool& hit, uint4& out, uint32_t& n_fp64, uint32_t& n_adj);
-template <class Tab>
-__device__ __forceinline__ void narrow_one_filter(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
-                                                  uint2 c, bool& hit, bool& defer, uint4& out, uint32_t& n_adj);
 
 // position of the k-th set bit of m (k < popcount(m))
 __device__ __forceinline__ uint32_t select_bit(u64 m, uint32_t k)
@@ -637,71 +631,54 @@ __device__ __forceinline__ void entry_expand(const Tab& T, const oi_mesh_desc* s
     }
 }
 
-// LDS the workgroup needs to test its leaf pairs cooperatively
-struct FusedLds {
-    u64 cmask[TB];
-    uint32_t coff[TB], ga[TB], gb[TB];
-    uint32_t hbase, dbase;
+// The leaf pairs of a workgroup by their number: thread t keeps the set bits of
+// mask[t] (bit (x << E) + y: pair (x, y) from p0[t] on), numbered from off[t] (one that
+// keeps none has the next one's off).
+template <int E>
+struct LeafFind {
+    u64 mask[TB];
+    uint2 p0[TB];
+    uint32_t off[TB];
+    __device__ __forceinline__ uint2 pair(uint32_t c) const
+    {
+        uint32_t lo = 0, hi = TB - 1;  // last thread whose first is at or before c
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1u) >> 1;
+            if (off[mid] <= c)
+                lo = mid;
+            else
+                hi = mid - 1u;
+        }
+        const uint32_t k = select_bit(mask[lo], c - off[lo]);
+        return make_uint2(p0[lo].x + (k >> E), p0[lo].y + (k & ((1u << E) - 1u)));
+    }
 };
 
-// The workgroup's C leaf pairs (thread t owns the set bits of cmask[t],
-// numbered from coff[t]) through the FP32 SAT (FILTER: the FP32 filter,
-// undecided pairs to the defer list for the FP64 pass): pair c is found by a
-// binary search over the offsets and a select in the owner's mask; hits (and
-// deferred pairs) are appended with one fetch_add each per round.
-template <int E, bool FILTER, class Tab>
-__device__ __forceinline__ void fused_narrow(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
-                                             FusedLds& F, uint32_t C, uint32_t* s_wsum, uint4* hits,
-                                             uint32_t* n_hits, uint32_t hits_cap, uint2* defer,
-                                             uint32_t* defer_count, uint32_t defer_cap, uint32_t* error,
-                                             uint32_t& n_fp64, uint32_t& n_adj)
+// The C leaf pairs of a local walk's workgroup through the FP32 SAT; hits are appended
+// with one fetch_add per round.
+template <int E, class Args>
+__device__ __forceinline__ void fused_narrow(const Args& A, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
+                                             const LeafFind<E>& F, uint32_t C, uint32_t* s_wsum, uint32_t& s_hbase,
+                                             uint32_t& n_adj)
 {
-    constexpr int K = 1 << E;
     const uint32_t tid = threadIdx.x;
     for (uint32_t c0 = 0; c0 < C; c0 += TB) {
-        const uint32_t c = c0 + tid;
-        bool hit = false, dfr = false;
-        uint2 pr = make_uint2(0, 0);
+        bool hit = false;
         uint4 h = make_uint4(0, 0, 0, 0);
-        if (c < C) {
-            uint32_t lo = 0, hi = TB - 1;  // last thread whose offset is <= c
-            while (lo < hi) {
-                const uint32_t mid = (lo + hi + 1u) >> 1;
-                if (F.coff[mid] <= c)
-                    lo = mid;
-                else
-                    hi = mid - 1u;
-            }
-            const uint32_t bit = select_bit(F.cmask[lo], c - F.coff[lo]);
-            pr = make_uint2(F.ga[lo] + (bit >> E), F.gb[lo] + (bit & (K - 1)));
-            if (FILTER)
-                narrow_one_filter<Tab>(T, s_ibase, s_desc, pr, hit, dfr, h, n_adj);
-            else
-                narrow_one<false, Tab>(T, s_ibase, s_desc, pr, hit, h, n_fp64, n_adj);
+        if (c0 + tid < C) {
+            v3f P[3], Q[3];
+            if (narrow_gather(A.tab, s_ibase, s_desc, F.pair(c0 + tid), true, n_adj, P, Q, h)) hit = sat_f32(P, Q);
+            if (hit) h = hit_ids(A.tab, s_desc, h);
         }
-        // one scan for both counts: hits in the high half, deferred pairs in
-        // the low half (at most 256 each)
-        uint32_t HD;
-        const uint32_t o = block_scan((hit ? 65536u : 0u) + (dfr ? 1u : 0u), s_wsum, HD);
-        const uint32_t H = HD >> 16, D = HD & 0xffffu;
-        if (tid == 0) {
-            F.hbase = H ? add_u32(n_hits, H) : 0u;
-            if (FILTER) F.dbase = D ? add_u32(defer_count, D) : 0u;
-        }
+        uint32_t H;
+        const uint32_t o = block_scan(hit ? 1u : 0u, s_wsum, H);
+        if (tid == 0) s_hbase = H ? add_u32(A.n_hits, H) : 0u;
         __syncthreads();
         if (hit) {
-            const uint32_t pos = F.hbase + (o >> 16);
-            if (pos < hits_cap)
-                hits[pos] = h;
+            if (s_hbase + o < A.hits_cap)
+                A.hits[s_hbase + o] = h;
             else
-                or_u32(error, OI_ERR_HITS_OVERFLOW);
-        }
-        if (FILTER && dfr) {
-            const uint32_t pos = F.dbase + (o & 0xffffu);
-            if (pos < defer_cap)
-                defer[pos] = pr;
-            else
-                or_u32(error, OI_ERR_CAND_OVERFLOW);
+                or_u32(A.error, OI_ERR_HITS_OVERFLOW);
         }
     }
 }
@@ -879,28 +856,6 @@ __device__ __forceinline__ void ring_leaves(const Args& A, Ring& S, const oi_mes
 // 80 VGPRs (6 waves) unspilled.
 #define STEP_FULL 1024  // kept pairs that leave for the front at a time, at least
 
-// The leaf pairs of a tile by their number: thread t keeps the set bits of mask[t]
-// (bit (x << 3) + y: pair (x, y) from p0[t] on), numbered from off[t] (one that keeps
-// none has the next one's off).
-struct StepFind {
-    u64 mask[TB];
-    uint2 p0[TB];
-    uint32_t off[TB];
-    __device__ __forceinline__ uint2 pair(uint32_t c) const
-    {
-        uint32_t lo = 0, hi = TB - 1;  // last thread whose first is at or before c
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi + 1u) >> 1;
-            if (off[mid] <= c)
-                lo = mid;
-            else
-                hi = mid - 1u;
-        }
-        const uint32_t k = select_bit(mask[lo], c - off[lo]);
-        return make_uint2(p0[lo].x + (k >> 3), p0[lo].y + (k & 7u));
-    }
-};
-
 template <int E, bool FIRST, int FUSE, class Tab>
 __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(E == 3 ? 4 : E == 2 ? 6 : 1, 8)))
 k_bvtt_step(StepArgs<Tab> A)
@@ -916,7 +871,7 @@ k_bvtt_step(StepArgs<Tab> A)
     __shared__ uint32_t s_ibase[MESH_LDS];
     __shared__ uint32_t s_wsum[4];
     __shared__ Ring S;
-    __shared__ std::conditional_t<E == 3 && FUSE != 0, StepFind, char> s_find;
+    __shared__ std::conditional_t<E == 3 && FUSE != 0, LeafFind<E>, char> s_find;
     // after an overflow the count keeps growing past the buffer (writes were
     // dropped and the detect will be re-run): read only what exists
     uint32_t n_in = A.count_in ? *A.count_in : A.n_in;
@@ -1086,14 +1041,6 @@ struct WalkLds : RingLds<WALK_RING, WALK_RING> {
     uint32_t n_out, n_cand;          // pairs ever put into the rings
 };
 
-// orders a wave's LDS accesses (its lanes exchange boxes)
-__device__ __forceinline__ void wave_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // One pass of the workgroup over the n pairs of src from the i0-th on, e levels
 // down: lane x of a pair's 2^e lanes tests child x of the first side against every
 // child of the second (whose boxes its lanes share through LDS W). Returns the
@@ -1136,7 +1083,7 @@ __device__ __forceinline__ uint32_t walk_pass(const WalkArgs<Tab>& A, float* W, 
         w[1] = make_float2(bb[2], bb[3]);
         w[2] = make_float2(bb[4], bb[5]);
     }
-    wave_fence();
+    oi_wave_fence();
     if (!mine) return 0u;
     uint32_t hit = 0;
     const float2* w = reinterpret_cast<const float2*>(W + 6u * (lane & ~(K - 1u)));
@@ -1386,7 +1333,8 @@ __global__ void __launch_bounds__(TB) k_bvtt_local(LocalArgs<Tab> A)
     __shared__ uint32_t s_wsum[4];
     __shared__ uint32_t s_qn, s_obase, s_cbase;
     __shared__ uint2 s_q[2][LQ];
-    __shared__ std::conditional_t<FUSED, FusedLds, char> s_f[1];
+    __shared__ std::conditional_t<FUSED, LeafFind<E>, char> s_f;
+    __shared__ uint32_t s_hbase;
     // after an overflow the count keeps growing past the buffer (writes were
     // dropped and the detect will be re-run): read only what exists
     uint32_t n_in = A.count_in ? *A.count_in : A.n_in;
@@ -1394,7 +1342,7 @@ __global__ void __launch_bounds__(TB) k_bvtt_local(LocalArgs<Tab> A)
     if (blockIdx.x * A.chunk >= n_in) return;
     tab_init(A.tab, s_desc, s_ibase);
     const uint32_t tid = threadIdx.x;
-    uint32_t n_tests = 0, n_adj = 0, n_cands = 0, n_fp64 = 0;
+    uint32_t n_tests = 0, n_adj = 0, n_cands = 0;
     bool overflow = false;
     for (uint32_t c0 = blockIdx.x * A.chunk; c0 < n_in; c0 += gridDim.x * A.chunk) {
         uint32_t n_cur = min(A.chunk, n_in - c0);
@@ -1442,10 +1390,9 @@ __global__ void __launch_bounds__(TB) k_bvtt_local(LocalArgs<Tab> A)
                     if (!FUSED) s_cbase = C ? add_u32(A.cand_count, C) : 0u;
                 }
                 if constexpr (FUSED) {
-                    s_f[0].cmask[tid] = leafout ? mask : 0ull;
-                    s_f[0].coff[tid] = coff;
-                    s_f[0].ga[tid] = baseA + sa.start;
-                    s_f[0].gb[tid] = baseB + sb.start;
+                    s_f.mask[tid] = mask;
+                    s_f.p0[tid] = make_uint2(baseA + sa.start, baseB + sb.start);
+                    s_f.off[tid] = coff;
                 }
                 __syncthreads();
                 if (nout && !leafout) {
@@ -1479,8 +1426,7 @@ __global__ void __launch_bounds__(TB) k_bvtt_local(LocalArgs<Tab> A)
                 if constexpr (FUSED) {
                     if (C) {
                         if (tid == 0) n_cands += C;
-                        fused_narrow<E, false, Tab>(A.tab, s_ibase, s_desc, s_f[0], C, s_wsum, A.hits, A.n_hits,
-                                                    A.hits_cap, nullptr, nullptr, 0, A.error, n_fp64, n_adj);
+                        fused_narrow<E>(A, s_ibase, s_desc, s_f, C, s_wsum, s_hbase, n_adj);
                     }
                 }
                 __syncthreads();
@@ -1617,39 +1563,6 @@ __device__ __forceinline__ uint4 hit_ids(const Tab& T, const oi_mesh_desc* s_des
         id.w = oi_g(mesh_perm(T, s_desc, id.y))[id.w];
     }
     return id;
-}
-
-// FP32 narrow phase of one candidate (the fused BVTT steps use it)
-template <bool FP64, class Tab>
-__device__ __forceinline__ void narrow_one(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
-                                           uint2 c, bool& hit, uint4& out, uint32_t& n_fp64, uint32_t& n_adj)
-{
-    static_assert(!FP64, "the FP64 fallback runs in k_narrow's two passes");
-    hit = false;
-    v3f P[3], Q[3];
-    uint4 id;
-    if (!narrow_gather(T, s_ibase, s_desc, c, true, n_adj, P, Q, id)) return;
-    if (sat_f32(P, Q)) {
-        hit = true;
-        out = hit_ids(T, s_desc, id);
-    }
-}
-
-// the FP32 filter on one candidate (the fused steps of an FP64-fallback
-// query): a hit, a pair left to the FP64 pass (defer), or neither
-template <class Tab>
-__device__ __forceinline__ void narrow_one_filter(const Tab& T, const uint32_t* s_ibase, const oi_mesh_desc* s_desc,
-                                                  uint2 c, bool& hit, bool& defer, uint4& out, uint32_t& n_adj)
-{
-    hit = false;
-    defer = false;
-    v3f P[3], Q[3];
-    uint4 id;
-    if (!narrow_gather(T, s_ibase, s_desc, c, true, n_adj, P, Q, id)) return;
-    const int r = sat_filter(P, Q);
-    hit = r == SAT_HIT;
-    defer = r == SAT_UNDECIDED;
-    if (hit) out = hit_ids(T, s_desc, id);
 }
 
 template <int MODE, class Tab>

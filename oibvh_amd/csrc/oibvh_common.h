@@ -34,6 +34,13 @@ __device__ __forceinline__ void oi_ld3(const uint32_t* base, uint32_t i, uint32_
     o[1] = q[1];
     o[2] = q[2];
 }
+// orders a wave's LDS accesses (its lanes exchange values through LDS)
+__device__ __forceinline__ void oi_wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 // inclusive prefix sum over the 64 lanes of a wave (every lane active) with
 // DPP moves instead of LDS permutes: a Kogge-Stone scan inside each row of
 // 16 lanes (row_shr 1, 2, 4, 8; a lane shifted in from outside its row

@@ -269,13 +269,6 @@ k_pairs_scatter(const PairRec* __restrict__ rec, uint32_t n, uint32_t nb, const 
         if (i0 + j * PS_THREADS < n) keys[s_start[r[j].bucket] + r[j].at] = r[j].key;
 }
 
-__device__ __forceinline__ void wave_order()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // places a < b of a list of m, ascending (places from m on hold the top key)
 __device__ __forceinline__ void order_pair(u64* g, uint32_t a, uint32_t b, uint32_t m)
 {
@@ -339,7 +332,7 @@ k_pairs_sort(u64* keys, const uint32_t* __restrict__ starts, oi_pair_bits bits, 
             if (j > 64u || next > 64u)
                 __syncthreads();
             else
-                wave_order();
+                oi_wave_fence();
         }
     }
     for (uint32_t i = tid; i < m; i += PS_THREADS) out[p0 + i] = hit_of(s[i], bits);
